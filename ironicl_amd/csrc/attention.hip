@@ -7,24 +7,15 @@
 //    backend (src/kernels/cuda/kernels.rs:183-213, 1523-1702), with the
 //    semantics of softmax(q k^T / 8) v in FP32 (src/kernels/reference.rs:792-1024).
 //
-//    A wave owns 64 queries (two blocks of 32). It computes the transposed
-//    products
-//      S^T[key, q] = K Q^T       (v_mfma_f32_32x32x2f32, k = head dim)
-//      O^T[d, q]  += V^T P^T     (k = keys)
-//    so that in the accumulator layout lane (q = lane % 32, half = lane / 32)
-//    holds all of one query's scores for half of each 32-key block, and all of
-//    its 64 output dims across the two 32-row output tiles; each K or V
-//    fragment read from LDS feeds both query blocks. The softmax state is per
-//    lane. Scores live in the exp2 domain (q pre-scaled by log2(e)/8) and are
-//    exponentiated against a lazy reference (see the kernel): the subtraction
-//    rides in the first MFMA's accumulator and the maximum is only taken when
-//    the reference must move. The P^T operand of the second product is the
-//    first product's accumulator register as is; each lane fetches the V
-//    elements of the key that register holds. The two output tiles take the
-//    even and the odd dims, so one 8-byte LDS read serves both. Keys stream
-//    through double-buffered 64-key LDS tiles filled by direct global -> LDS
-//    loads; only a range's last tile is clamped and masked. One workgroup of
-//    four waves per CU: each wave may use 512 registers.
+//    Passes of more than 32 queries multiply on the FP16 matrix cores with
+//    every FP32 operand held as a pair of FP16 values (icl_attention_kernel);
+//    smaller ones stream the keys on the FP32 ones (icl_decode_kernel). Both
+//    compute the transposed products
+//      S^T[key, q] = K Q^T
+//      O^T[d, q]  += V^T P^T
+//    so that a lane's accumulators hold scores of one query, which are the
+//    second product's operand where they are. Scores live in the exp2 domain
+//    and are exponentiated against a lazy reference, raised only when it must.
 //
 //    Key ranges are split over workgroups to fill the chip (prediction
 //    passes); the build's many query tiles run whole rounds with every key
@@ -73,16 +64,9 @@ typedef __attribute__((address_space(3))) void lds_void;
 constexpr int kIclWaves = 4;
 constexpr int kIclQueries = kIclWaves * 64;  // queries per workgroup, 64 per wave
 
-// One 64-key tile of K and V in LDS, 16 KB each, written by direct global ->
-// LDS loads (a wave-wide 16-byte load lands as 1 KB, lane after lane). K is
-// kept in 1 KB blocks b = (chunk / 4) * 4 + key / 16, each holding 16 keys x
-// 4 chunks of 4 dims at position (chunk % 4) * 16 + key % 16, so that the 16
-// lanes of a 16-byte LDS read that fetch one chunk of 16 consecutive keys
-// touch every bank once. V is key-major: a half-wave reads one key's 64 dims.
-struct IclTile {
-    float k[kKeyTile * 64];
-    float v[kKeyTile * 64];
-};
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ half8 as_half8(u32x4 v) { return __builtin_bit_cast(half8, v); }
 
 __device__ __forceinline__ void wait_loads() {
     // vmcnt(0); expcnt and lgkmcnt left at their maxima (no wait).
@@ -100,34 +84,201 @@ __device__ __forceinline__ float halves_sum(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Long key ranges (FLUSH) accumulate in two levels: every kFlushTiles tiles
-// the register accumulators (O^T and the row sums) are added into totals the
-// lane keeps in LDS and restart from zero. A single FP32 accumulator over
-// tens of thousands of keys loses the contributions that arrive after a
-// dominant one (each addend below half an ulp of the sum is rounded away);
-// with peaked attention over 50,000 keys that cost 3e-4 of the output.
-constexpr int kFlushTiles = 64;
-constexpr int kFlushFloats = kIclWaves * 2 * 2 * 16 * 64;  // [j][b][r / 4][thread][r % 4]
+// Maximum over a wave of magnitudes (x >= 0), in every lane: rotations within
+// rows of 16 lanes, then the rows.
+__device__ __forceinline__ float wave_magnitude(float x) {
+#define IRX_ROTATE(n) \
+    x = fmaxf(x, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + n, 0xf, 0xf, true)))
+    IRX_ROTATE(8);
+    IRX_ROTATE(4);
+    IRX_ROTATE(2);
+    IRX_ROTATE(1);
+#undef IRX_ROTATE
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return halves_max(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
 
-// SPLIT: the keys are split over workgroups and each writes a partial output
-// and its log2-sum-exp, merged afterwards; otherwise the output is final.
+// Long key ranges (FLUSH) accumulate in two levels: every kFlushTiles tiles
+// the register accumulators (O^T and the row sums) are added into totals in
+// LDS and restart from zero. A single FP32 accumulator over tens of thousands
+// of keys loses the contributions that arrive after a dominant one (each
+// addend below half an ulp of the sum is rounded away); with peaked attention
+// over 50,000 keys that cost 3e-4 of the output.
+constexpr int kFlushTiles = 64;
+
+// ---- FP32 attention of wide passes: FP32 operands as pairs of FP16 values ----
+//
+// Every operand x of the two products (queries, keys, probabilities, values)
+// is scaled by a power of two and split into hi = fp16(x), lo = fp16(x - hi),
+// both rounded to nearest: hi + lo holds x to 2^-23. A product is
+//   lo.hi + hi.lo + hi.hi
+// into one FP32 accumulator on the 32x32x16 FP16 MFMA (lo.lo, below 2^-24 of
+// the product, is left out). Random operands against float64 (K = 64 / 512 /
+// 4,096 / 16,384): 1.1e-7 / 2.6e-7 / 7.2e-7 / 1.5e-6 of the result, where the
+// FP32 MFMA gives 1.4e-7 / 4.0e-7 / 1.1e-6 / 2.3e-6 (it rounds its
+// accumulator every two terms, this one every sixteen); truncated parts would
+// give 3.6e-7 at K = 64. Three FP16 products cost 3/16 of an FP32 one, and
+// unlike FP32 MFMAs they run beside the other wave's VALU work.
+//
+// A workgroup is eight waves: wave w takes queries 64 (w % 4) .. + 63 of the
+// tile against key half w / 4 of each 64-key tile, so the two waves of a SIMD
+// read each half of a tile for 64 queries per LDS byte. Per tile a wave has a
+// VALU phase (softmax, and its share of the staging; about 310 instructions)
+// and an MFMA phase (the output products of this tile, the scores of the next;
+// 48 MFMAs, 1,536 cycles); the key halves run them in opposite order, a
+// barrier after each phase, so a SIMD's matrix cores and its VALU are both in
+// use throughout. The halves' results are merged through LDS at the end (and,
+// FLUSH, every kFlushTiles tiles).
+//
+// Bound by the FP16 matrix cores' power-limited rate: 512 queries x 50,000
+// keys x 8 pairs takes 162 us, 970 TFLOP/s of FP16 products (a large FP16
+// matrix product reaches 1,100 here), at 2.0 GHz; orders of the same work that
+// take fewer cycles (fragments read across the barrier, wave priorities, the
+// conversions stage by stage) take the same time. The FP32 MFMA kernel before
+// it took 388 us, 135 of 157 TFLOP/s; 10,007 queries x 10,007 keys went from
+// 1,556 to 595 us.
+//   S^T (key x query), A = K[key 32 (w / 4) + lane % 32][dims 16 m +
+//     8 (lane / 32) .. +7], B = the lane's query, same dims; register r is
+//     key 8 (r / 4) + 4 (lane / 32) + r % 4 of the half;
+//   O^T (dim x query), step g: B = the probabilities in registers 8 g .. +7
+//     as they are, A = V^T[dim][those keys], which the tile's key order makes
+//     one 16-byte read (each 16 keys in the order 0..3, 8..11, 4..7, 12..15).
+// K and V come as FP32 rows: wave w loads keys 8 w .. + 7 of a tile of K and
+// the eight keys of V's stored chunk w of the next tile into registers a phase
+// ahead, then writes their pairs to LDS in its next VALU phase. Counting half
+// 0's VALU phase of tile t as phase 2 t (its MFMA phase, and half 1's VALU
+// phase, as 2 t + 1): K tile u is written in phases 2 u - 3 (half 1) and 2 u -
+// 2, read in 2 u - 1 and 2 u, so two buffers do; V tile u is written in 2 u -
+// 2 and 2 u - 1 and read in 2 u + 1 and 2 u + 2, which takes three. The scales
+// of K tile u are read in phases 2 u and 2 u + 1, of V too (four slots).
+//
+// Scales, all powers of two. Queries: per row, in registers. Keys and values:
+// per wave's share of a tile (8 keys x 64 dims), kept while the share's
+// largest scaled magnitude stays in [2^11, 2^15] and else set to bring it into
+// [2^13, 2^14): an operand is held to 2^-23 of itself or 2^-36 of the largest
+// of its eight keys. The key scale joins the softmax's multiply (four keys of
+// it to a register group); the value scale joins the exponent, so that the
+// probability carries its inverse, and is taken out of the row sum. The
+// reference the exponent is taken against is raised, to 8 (base 2) below the
+// running maximum, when a scaled probability would pass 2^15.
+//
+// Infinite keys or values, values all below 2^-47, and keys so large that
+// scores could pass 2^20 (where one scale would serve neither those keys nor
+// their neighbours) are left to a plain FP32 loop over the workgroup's
+// queries (icl_row_fp32).
+struct IclPairTile {
+    u32x4 h[kKeyTile * 8], l[kKeyTile * 8];  // K: [key][8 chunks of 8 dims]; V: [dim][8 chunks of 8 keys]
+};
+struct IclPairTiles {
+    IclPairTile k[2], v[3];
+};
+// Chunk c of row r is stored at chunk c ^ pair_swizzle(r): the 16 rows that 16
+// lanes read or write at one chunk cover all 64 LDS banks.
+__device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
+constexpr int kPairWaves = 8;
+constexpr float kPairHigh = 32768.0f, kPairLow = 2048.0f;
+
+// Eight FP32 values as FP16 pairs, both parts rounded to nearest.
+__device__ __forceinline__ void pair8(const float *x, half8 &hi, half8 &lo) {
+    typedef _Float16 half2 __attribute__((ext_vector_type(2)));
+    // An opaque -1 makes each remainder one v_fma_mix_f32 (as a subtraction it
+    // is a conversion and a subtraction).
+    float minus = -1.0f;
+    asm("" : "+s"(minus));
+    u32x4 h, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const half2 hp = __builtin_convertvector((f32x2{x[2 * i], x[2 * i + 1]}), half2);
+        const f32x2 r = {__builtin_fmaf((float)hp[0], minus, x[2 * i]), __builtin_fmaf((float)hp[1], minus, x[2 * i + 1])};
+        const half2 lp = __builtin_convertvector(r, half2);
+        h[i] = __builtin_bit_cast(unsigned, hp);
+        l[i] = __builtin_bit_cast(unsigned, lp);
+    }
+    hi = __builtin_bit_cast(half8, h);
+    lo = __builtin_bit_cast(half8, l);
+}
+
+// 2^e for -126 <= e <= 127.
+__device__ __forceinline__ float pow2(int e) { return __uint_as_float((unsigned)(e + 127) << 23); }
+// The exponent of the scale that brings a finite magnitude `m` into [2^13,
+// 2^14) (as far as 2^e and 2^-e are normal).
+__device__ __forceinline__ int pair_exponent(float m) {
+    return min(126, 13 - ((int)(__float_as_uint(m) >> 23) - 127));
+}
+
+// One query against `keys` keys in plain FP32 by a pair of threads (32 dims
+// each) with a running maximum: the unnormalized output, its sum and reference.
+__device__ __forceinline__ void icl_row_fp32(const float *q, const float *k, const float *v, int keys, int part,
+                                           float *o, float &m, float &l) {
+    float qr[32];
+#pragma unroll
+    for (int d = 0; d < 32; ++d) qr[d] = q[32 * part + d] * (0.125f * kLog2e), o[d] = 0.f;
+    m = -INFINITY, l = 0.f;
+    for (int key = 0; key < keys; ++key) {
+        const float *kr = k + (long long)key * 64 + 32 * part, *vr = v + (long long)key * 64 + 32 * part;
+        float s = 0.f;
+#pragma unroll
+        for (int d = 0; d < 32; ++d) s = __builtin_fmaf(qr[d], kr[d], s);
+        s += __shfl_xor(s, 1, 64);
+        const float mn = fmaxf(m, s);
+        const float a = key ? __builtin_amdgcn_exp2f(m - mn) : 0.f, w = __builtin_amdgcn_exp2f(s - mn);
+        l = l * a + w;
+#pragma unroll
+        for (int d = 0; d < 32; ++d) o[d] = o[d] * a + w * vr[d];
+        m = mn;
+    }
+}
+
+// x *= f in x's own registers: in a rarely taken branch the compiler otherwise
+// gives the products of all accumulators registers of their own, and spills.
+// The caller has read a later MFMA's result since x's last one was issued
+// (MFMAs finish in order; the compiler adds no wait states before asm), and
+// the s_nop covers f coming straight from a transcendental.
+__device__ __forceinline__ void scale_in_place(f32x16 &x, float f) {
+    asm("s_nop 1" : "+v"(f));
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        float v = x[r];
+        asm("v_mul_f32 %0, %0, %1" : "+v"(v) : "v"(f));
+        x[r] = v;
+    }
+}
+
+// A barrier between phases: LDS accesses are complete, global loads stay in
+// flight, and nothing is scheduled across it.
+__device__ __forceinline__ void phase_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 template <bool SPLIT, bool FLUSH>
-__global__ __launch_bounds__(kIclWaves * 64, 1) void icl_attention_kernel(IclAttention p, IclLaunch g) {
-    // One LDS object: the K/V tiles, then (FLUSH) each thread's O^T totals
-    // and its row-sum totals [j][thread]. (As a second LDS object the totals
-    // made the compiler wait for the in-flight tile loads before every read
-    // of the current tile.)
+__global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAttention p, IclLaunch g) {
+    struct Totals {
+        float o[2][2][4][4 * 64][4];  // [query block][dim block][r / 4][thread of the query groups][r % 4]
+        float m[2][4 * 64], l[2][4 * 64];
+    };
     struct LdsPlain {
-        IclTile tiles[2];
+        union {
+            IclPairTiles tiles;
+            Totals totals;
+        };
     };
     struct LdsFlush {
-        IclTile tiles[2];
-        float totals[kFlushFloats + kIclWaves * 2 * 64];
+        IclPairTiles tiles;
+        Totals totals;
     };
-    __shared__ __attribute__((aligned(16))) std::conditional_t<FLUSH, LdsFlush, LdsPlain> lds;
-    IclTile *tiles = lds.tiles;
-    float *totals = nullptr;
-    if constexpr (FLUSH) totals = lds.totals;
+    struct Shared {
+        std::conditional_t<FLUSH, LdsFlush, LdsPlain> data;
+        float k_inv[4][kPairWaves];     // per tile and staging wave: inverse key scale;
+        f32x2 v_exp[4][kPairWaves];     // the value scale's exponent and the scale
+        float largest[kPairWaves];      // largest query magnitude of each wave
+        unsigned special[kPairWaves];
+    };
+    __shared__ __attribute__((aligned(16))) Shared lds;
 
     const int bid = bid_x();
     const int t_id = (bid % 8) * g.per_xcd + bid / 8;
@@ -145,320 +296,360 @@ __global__ __launch_bounds__(kIclWaves * 64, 1) void icl_attention_kernel(IclAtt
         const int rest = t_id / g.qtiles;
         split = rest % g.splits, pair = rest / g.splits;
     }
-    // Workgroup-uniform; read into scalars so the key loop runs on scalar registers.
     const int k_begin = __builtin_amdgcn_readfirstlane(split * g.keys_per_split);
     const int k_end = __builtin_amdgcn_readfirstlane(min(p.kv_rows, k_begin + g.keys_per_split));
 
-    const int tid = tid_x(), lane = tid & 63, wave = tid >> 6;
+    const int tid = tid_x(), lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qgroup = wave & 3, khalf = wave >> 2;
     const int half = lane >> 5, r32 = lane & 31;
-    // Query block j of this wave holds rows qrow0 + 32 j.
-    const int qrow0 = qt * kIclQueries + wave * 64 + r32;
+    const int qrow0 = qt * kIclQueries + qgroup * 64 + r32;
 
-    // The lane's queries: dims 32*half .. 32*half + 31, scaled into the exp2 domain.
-    float qreg[2][32];
-    {
-        const float scale = 0.125f * kLog2e;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int qrow = qrow0 + 32 * j;
-            if (qrow < p.q_rows) {
-                const float *src = p.q + pair * p.q_pair_stride + (long long)qrow * 64 + 32 * half;
-#pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    f32x4 v = *reinterpret_cast<const f32x4 *>(src + 4 * c);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) qreg[j][4 * c + e] = v[e] * scale;
-                }
-            } else {
-#pragma unroll
-                for (int t = 0; t < 32; ++t) qreg[j][t] = 0.f;
-            }
-        }
-    }
-
-    // Staging: wave w moves K blocks 4w .. 4w + 3 (chunks 4w .. 4w + 3 of key
-    // blocks 0..3) and V blocks 4w .. 4w + 3 (keys 16w .. 16w + 15).
-    const float *kbase = p.k + pair * p.kv_pair_stride;
-    const float *vbase = p.v + pair * p.kv_pair_stride;
-    // Lane offsets (floats) within a full tile: K key 16 i + lane % 16, chunk
-    // 4w + lane / 16; V key 16w + 4i + lane / 16, chunk lane % 16. The wave
-    // index is read into a scalar so that tile bases and LDS destinations are
-    // scalar arithmetic.
-    const int wv = __builtin_amdgcn_readfirstlane(wave);
-    const int k_lane = (lane & 15) * 64 + 4 * (4 * wv + (lane >> 4));
-    const int v_lane = (lane >> 4) * 64 + 4 * (lane & 15);
-    auto issue_tile = [&](int k0, int buf) {
-        const float *kt = kbase + (long long)k0 * 64, *vt = vbase + (long long)(k0 + 16 * wv) * 64;
-        if (k0 + kKeyTile <= k_end) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                __builtin_amdgcn_global_load_lds(kt + i * 1024 + k_lane, (lds_void *)&tiles[buf].k[(4 * wv + i) * 256],
-                                                 16, 0, 0);
-                __builtin_amdgcn_global_load_lds(vt + i * 256 + v_lane, (lds_void *)&tiles[buf].v[(4 * wv + i) * 256],
-                                                 16, 0, 0);
-            }
-        } else {
-            // A range's last tile: keys past it repeat its last key (masked later).
-            const int last = k_end - 1 - k0;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int kk = min(16 * i + (lane & 15), last);
-                const int vk = min(16 * wv + 4 * i + (lane >> 4), last);
-                __builtin_amdgcn_global_load_lds(kbase + (long long)(k0 + kk) * 64 + 4 * (4 * wv + (lane >> 4)),
-                                                 (lds_void *)&tiles[buf].k[(4 * wv + i) * 256], 16, 0, 0);
-                __builtin_amdgcn_global_load_lds(vbase + (long long)(k0 + vk) * 64 + 4 * (lane & 15),
-                                                 (lds_void *)&tiles[buf].v[(4 * wv + i) * 256], 16, 0, 0);
-            }
-        }
-    };
-
-    // O^T accumulators of query block j: o[j][0] even dims d = 2i, o[j][1] odd
-    // dims d = 2i + 1, where i = half*4 + (r&3) + 8*(r>>2) for register r.
-    f32x16 o[2][2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o[j][0][r] = 0.f, o[j][1][r] = 0.f;
-    // Softmax reference m_ref[j] per query (shared by the lane pair l, l ^ 32):
-    // probabilities are exp2(s - m_ref). The range's first tile sets it to
-    // that tile's maxima (its products start from zero); after that it is
-    // raised, and the tile redone, only when a tile's probabilities could
-    // exceed 2^64, so most tiles skip the maximum reduction; -m_ref is the
-    // products' initial accumulator, which folds the subtraction into the
-    // MFMA. Relative to the true running maximum a probability is at most
-    // 2^64 and anything below 2^-126 of the maximum is lost, as in the exact
-    // online softmax.
-    float m_ref[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
-    f32x16 neg_ref[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) neg_ref[j][r] = 0.f;
-    bool fresh = true;  // workgroup-uniform: no tile of the range done yet
-    constexpr float kLazyLimit = 18446744073709551616.0f;  // 2^64
-    // K fragment of chunk 8*half + cc for key r32 of block 0 is at kfrag + (cc >> 2) * 1024 + (cc & 3) * 64;
-    // block 1 (keys 32..63) is 512 floats further.
-    const int kfrag = (8 * half + (r32 >> 4)) * 256 + (r32 & 15) * 4;
-
-    // FLUSH: the keys run in chunks of kFlushTiles tiles, each chunk's
-    // accumulators added into the lane's LDS totals after it (flushed: some
-    // chunk was; workgroup-uniform). The totals' addresses are formed where
-    // they are used, so nothing extra stays live through the tile loop.
-    bool flushed = false;
-    // Rescales owed to the totals since the last flush (the reference moved):
-    // applied when the totals are next read, so the tile loop touches no LDS
-    // besides its tiles.
-    float tot_scale[2] = {1.f, 1.f};
-    // O^T totals as [j][b][r / 4][thread] groups of four: one 16-byte LDS
-    // access per group of a lane's four consecutive registers.
-    auto o_tot = [&](int j, int b, int q) -> f32x4 & {
-        return *reinterpret_cast<f32x4 *>(&totals[(((j * 2 + b) * 4 + q) * 64 * kIclWaves + tid_x()) * 4]);
-    };
-    auto l_tot = [&](int j) -> float & { return totals[kFlushFloats + tid_x() + j * 64 * kIclWaves]; };
-    const int chunk = FLUSH ? kFlushTiles * kKeyTile : k_end - k_begin;
-
-    issue_tile(k_begin, 0);
-    int buf = 0;
-    for (int c0 = k_begin; c0 < k_end; c0 = __builtin_amdgcn_readfirstlane(c0 + chunk)) {
-    const int c1 = __builtin_amdgcn_readfirstlane(min(k_end, c0 + chunk));
-    for (int k0 = c0; k0 < c1; k0 = __builtin_amdgcn_readfirstlane(k0 + kKeyTile)) {
-        wait_loads();
-        __syncthreads();
-        if (k0 + kKeyTile < k_end) issue_tile(k0 + kKeyTile, buf ^ 1);
-        const float *kt = tiles[buf].k;
-        const float *vt = tiles[buf].v;
-
-        // S^T[key, q] - m_ref for key blocks 0 / 1 and query blocks 0 / 1.
-        f32x16 s[2][2];
-        // K fragments are read one chunk ahead of their MFMAs (the scheduling
-        // groups keep the compiler from sinking the reads to their first use).
-        f32x4 ka = *reinterpret_cast<const f32x4 *>(kt + kfrag);
-        f32x4 kb = *reinterpret_cast<const f32x4 *>(kt + kfrag + 512);
-#pragma unroll
-        for (int cc = 0; cc < 8; ++cc) {
-            f32x4 na = ka, nb = kb;
-            if (cc < 7) {
-                const int off = kfrag + ((cc + 1) >> 2) * 1024 + ((cc + 1) & 3) * 64;
-                na = *reinterpret_cast<const f32x4 *>(kt + off);
-                nb = *reinterpret_cast<const f32x4 *>(kt + off + 512);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    const f32x16 &c0 = (cc == 0 && e == 0) ? neg_ref[j] : s[j][0];
-                    const f32x16 &c1 = (cc == 0 && e == 0) ? neg_ref[j] : s[j][1];
-                    s[j][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(ka[e], qreg[j][4 * cc + e], c0, 0, 0, 0);
-                    s[j][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(kb[e], qreg[j][4 * cc + e], c1, 0, 0, 0);
-                }
-            if (cc < 7) {
-                __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // the two DS reads
-                __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);  // then this chunk's MFMAs
-            }
-            ka = na, kb = nb;
-        }
-        // Only the last tile of a range can hold keys past it.
-        if (k0 + kKeyTile > k_end) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int key = k0 + half * 4 + (r & 3) + 8 * (r >> 2);
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    if (key >= k_end) s[j][0][r] = -INFINITY;
-                    if (key + 32 >= k_end) s[j][1][r] = -INFINITY;
-                }
-            }
-        }
-        if (fresh) {
-            // The range's first tile: its scores (from a zero accumulator)
-            // give the reference.
-            fresh = false;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                float mt = -INFINITY;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) mt = fmaxf(mt, fmaxf(s[j][0][r], s[j][1][r]));
-                const float m = halves_max(mt);
-                m_ref[j] = m;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    neg_ref[j][r] = -m;
-                    s[j][0][r] -= m, s[j][1][r] -= m;
-                }
-            }
-        }
-        // Softmax per query block (exp2 domain) against the lazy reference.
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            float lsum = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[j][0][r] = __builtin_amdgcn_exp2f(s[j][0][r]);
-                s[j][1][r] = __builtin_amdgcn_exp2f(s[j][1][r]);
-                lsum += s[j][0][r] + s[j][1][r];
-            }
-            if (__any(!(lsum <= kLazyLimit))) {
-                // The reference is too low for this tile: recompute the
-                // block's scores from zero and raise it to the running maximum.
-                f32x16 t0, t1;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) t0[r] = 0.f, t1[r] = 0.f;
-#pragma unroll
-                for (int cc = 0; cc < 8; ++cc) {
-                    const int off = kfrag + (cc >> 2) * 1024 + (cc & 3) * 64;
-                    const f32x4 a = *reinterpret_cast<const f32x4 *>(kt + off);
-                    const f32x4 b = *reinterpret_cast<const f32x4 *>(kt + off + 512);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        t0 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], qreg[j][4 * cc + e], t0, 0, 0, 0);
-                        t1 = __builtin_amdgcn_mfma_f32_32x32x2f32(b[e], qreg[j][4 * cc + e], t1, 0, 0, 0);
-                    }
-                }
-                if (k0 + kKeyTile > k_end) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int key = k0 + half * 4 + (r & 3) + 8 * (r >> 2);
-                        if (key >= k_end) t0[r] = -INFINITY;
-                        if (key + 32 >= k_end) t1[r] = -INFINITY;
-                    }
-                }
-                float mt = -INFINITY;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) mt = fmaxf(mt, fmaxf(t0[r], t1[r]));
-                const float m_new = fmaxf(m_ref[j], halves_max(mt));
-                const float alpha = __builtin_amdgcn_exp2f(m_ref[j] - m_new);
-                l_run[j] *= alpha;
-                lsum = 0.f;
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    o[j][0][r] *= alpha, o[j][1][r] *= alpha;
-                    neg_ref[j][r] = -m_new;
-                    s[j][0][r] = __builtin_amdgcn_exp2f(t0[r] - m_new);
-                    s[j][1][r] = __builtin_amdgcn_exp2f(t1[r] - m_new);
-                    lsum += s[j][0][r] + s[j][1][r];
-                }
-                if constexpr (FLUSH) tot_scale[j] *= alpha;  // the totals are in the old scale too
-                m_ref[j] = m_new;
-            }
-            l_run[j] += lsum;
-        }
-        // O^T += V^T P^T: register r of s[j][b] is key b*32 + half*4 + (r&3) + 8*(r>>2);
-        // the lane fetches that key's dims 2*r32 and 2*r32 + 1, one key ahead
-        // of its products (scheduling fences keep the reads there: left to
-        // itself the compiler moves each read next to its first use).
-        auto vrow = [&](int r) { return vt + (half * 4 + (r & 3) + 8 * (r >> 2)) * 64 + 2 * r32; };
-        f32x2 v0 = *reinterpret_cast<const f32x2 *>(vrow(0));
-        f32x2 v1 = *reinterpret_cast<const f32x2 *>(vrow(0) + 32 * 64);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            f32x2 n0 = v0, n1 = v1;
-            if (r < 15) {
-                n0 = *reinterpret_cast<const f32x2 *>(vrow(r + 1));
-                n1 = *reinterpret_cast<const f32x2 *>(vrow(r + 1) + 32 * 64);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                o[j][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(v0[0], s[j][0][r], o[j][0], 0, 0, 0);
-                o[j][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(v0[1], s[j][0][r], o[j][1], 0, 0, 0);
-                o[j][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(v1[0], s[j][1][r], o[j][0], 0, 0, 0);
-                o[j][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(v1[1], s[j][1][r], o[j][1], 0, 0, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            v0 = n0, v1 = n1;
-        }
-        buf ^= 1;
-    }
-    if constexpr (FLUSH) {
-        if (c1 < k_end) {
-            // Each lane moves only its own values: no barrier.
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const float ts = tot_scale[j];
-                l_tot(j) = flushed ? l_tot(j) * ts + l_run[j] : l_run[j];
-                l_run[j] = 0.f;
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        f32x4 t = flushed ? o_tot(j, b, q) : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            t[e] = flushed ? t[e] * ts + o[j][b][4 * q + e] : o[j][b][4 * q + e];
-                            o[j][b][4 * q + e] = 0.f;
-                        }
-                        o_tot(j, b, q) = t;
-                    }
-                tot_scale[j] = 1.f;
-            }
-            flushed = true;
-        }
-    }
-    }
-    if constexpr (FLUSH) {
-        if (flushed) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const float ts = tot_scale[j];
-                l_run[j] += l_tot(j) * ts;
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const f32x4 t = o_tot(j, b, q);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) o[j][b][4 * q + e] += t[e] * ts;
-                    }
-            }
-        }
-    }
-
+    // The lane's queries (row qrow0 + 32 j), dims 16 m + 8 half .. +7, as
+    // scaled pairs; coef[j] takes a product of scaled queries and unscaled
+    // keys to the exp2 domain.
+    half8 qh[2][4], ql[2][4];
+    float coef[2];
+    float q_largest = 0.f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int qrow = qrow0 + 32 * j;
-        const float l_tot = halves_sum(l_run[j]);
+        float x[32];
+#pragma unroll
+        for (int i = 0; i < 32; ++i) x[i] = 0.f;
+        if (qrow < p.q_rows) {
+            const float *src = p.q + pair * p.q_pair_stride + (long long)qrow * 64 + 8 * half;
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const f32x4 a = *reinterpret_cast<const f32x4 *>(src + 16 * m + 4 * c);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[8 * m + 4 * c + e] = a[e];
+                }
+        }
+        float mx = 0.f;
+#pragma unroll
+        for (int i = 0; i < 32; ++i) mx = fmaxf(mx, fabsf(x[i]));
+        mx = halves_max(mx);
+        q_largest = fmaxf(q_largest, mx);
+        const int e = pair_exponent(mx);
+        const float s = pow2(e);
+        coef[j] = 0.125f * kLog2e * pow2(-e);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            float y[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) y[i] = x[8 * m + i] * s;
+            pair8(y, qh[j][m], ql[j][m]);
+        }
+    }
+
+    const float *kbase = p.k + pair * p.kv_pair_stride;
+    const float *vbase = p.v + pair * p.kv_pair_stride;
+    // Staging: thread t holds key t / 8's dims 8 (t % 8) .. +7 and dim `lane`
+    // of the eight keys at stored chunk `wave`. The loads go through buffer
+    // descriptors that end with the range: keys past it read as zeros (their
+    // scores are masked), and the addresses take no VALU work.
+    const int s_key = tid >> 3, s_chunk = tid & 7;
+    float kr[8], vr[8];
+    auto rsrc = [&](const float *base, int k0) {
+        const float *tile = base + (long long)k0 * 64;
+        const long long bytes = min((long long)(k_end - k0) * 256, 0x7fffffffLL);
+        return __builtin_amdgcn_make_buffer_rsrc((void *)tile, 0, (int)bytes, 0x00020000);
+    };
+    const int k_off = tid * 32, v_off = (16 * (wave >> 1) + 4 * (wave & 1)) * 256 + lane * 4;
+    auto load_k = [&](int k0) {
+        const auto r = rsrc(kbase, k0);
+        const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, k_off, 0, 0);
+        const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(r, k_off + 16, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kr[e] = __uint_as_float(a[e]), kr[4 + e] = __uint_as_float(b[e]);
+    };
+    auto load_v = [&](int k0) {
+        const auto r = rsrc(vbase, k0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            vr[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, v_off + ((i & 3) + 8 * (i >> 2)) * 256, 0, 0));
+    };
+    bool special = false;
+    q_largest = wave_magnitude(q_largest);
+    if (lane == 0) lds.largest[wave] = q_largest;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kPairWaves; ++w) q_largest = fmaxf(q_largest, lds.largest[w]);
+    q_largest = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(q_largest)));
+    // The wave's scales, 2^ek and 2^ev, brought up to date with the staged
+    // values (rarely anything to do).
+    int ek = 0, ev = 0;
+    auto update_scales = [&]() {
+        float km = 0.f, vm = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) km = fmaxf(km, fabsf(kr[i])), vm = fmaxf(vm, fabsf(vr[i]));
+        const float ks = km * pow2(ek), vs = vm * pow2(ev);
+        const unsigned long long high = __ballot(fmaxf(ks, vs) > kPairHigh);
+        const unsigned long long k_ok = __ballot(ks >= kPairLow), v_ok = __ballot(vs >= kPairLow);
+        if (__builtin_expect(high != 0 || k_ok == 0 || v_ok == 0, 0)) {
+            km = wave_magnitude(km), vm = wave_magnitude(vm);
+            const unsigned kb = __builtin_amdgcn_readfirstlane(__float_as_uint(km));
+            const unsigned vb = __builtin_amdgcn_readfirstlane(__float_as_uint(vm));
+            // 8 |q| |k| bounds a score (64 dims, times 1/8).
+            if (kb >= 0x7f800000u || vb >= 0x7f800000u || __uint_as_float(kb) * 8.0f * q_largest > 1048576.0f ||
+                (vb && __uint_as_float(vb) < 7e-15f))
+                special = true;
+            if (kb && kb < 0x7f800000u) ek = pair_exponent(__uint_as_float(kb));
+            // (A share of zeros takes the scale of the smallest values, so that
+            // its probabilities do not set the reference.)
+            if (vb < 0x7f800000u) ev = vb ? min(60, pair_exponent(__uint_as_float(vb))) : 60;
+        }
+    };
+    // The staged tiles, u of K and w of V (to buffer `vb`), to LDS. Every lane
+    // writes the wave's scales (to one address): a branch would cost more.
+    auto convert_k = [&](int u) {
+        IclPairTile &t = lds.data.tiles.k[u & 1];
+        half8 hi, lo;
+        float x[8];
+        const float sc = pow2(ek);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = kr[i] * sc;
+        pair8(x, hi, lo);
+        const int c = s_key * 8 + (s_chunk ^ pair_swizzle(s_key));
+        t.h[c] = __builtin_bit_cast(u32x4, hi), t.l[c] = __builtin_bit_cast(u32x4, lo);
+        lds.k_inv[u & 3][wave] = pow2(-ek);
+    };
+    auto convert_v = [&](int w, int vb) {
+        IclPairTile &t = lds.data.tiles.v[vb];
+        half8 hi, lo;
+        float x[8];
+        const float sc = pow2(ev);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = vr[i] * sc;
+        pair8(x, hi, lo);
+        const int c = lane * 8 + (wave ^ pair_swizzle(lane));
+        t.h[c] = __builtin_bit_cast(u32x4, hi), t.l[c] = __builtin_bit_cast(u32x4, lo);
+        lds.v_exp[w & 3][wave] = f32x2{(float)ev, sc};
+    };
+
+    f32x16 o[2][2];  // [dim block][query block]
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[d][j][r] = 0.f;
+    constexpr float kLowest = -3.0e38f;  // a finite reference below every score
+    float m_ref[2] = {kLowest, kLowest}, l_run[2] = {0.f, 0.f};
+    f32x16 s[2];    // scores of the tile (raw products)
+    half8 ph[2][2], pl[2][2];  // its probabilities, [query block][step]
+    // Scores of the tile whose keys are in buffer `kb`. Fragments are
+    // read one step ahead of their products; the scheduling fences keep the
+    // compiler from reading them all at once, which spills.
+    auto scores = [&](int kb) {
+        const IclPairTile &t = lds.data.tiles.k[kb];
+        const int krow = 32 * khalf + r32;
+        auto kc = [&](int m) { return krow * 8 + ((2 * m + half) ^ pair_swizzle(krow)); };
+        u32x4 ah = t.h[kc(0)], al = t.l[kc(0)];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[j][r] = 0.f;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            u32x4 nh = ah, nl = al;
+            if (m < 3) nh = t.h[kc(m + 1)], nl = t.l[kc(m + 1)];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) s[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_half8(al), qh[j][m], s[j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) s[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_half8(ah), ql[j][m], s[j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) s[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_half8(ah), qh[j][m], s[j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            ah = nh, al = nl;
+        }
+    };
+    auto output = [&](int vb) {
+        const IclPairTile &t = lds.data.tiles.v[vb];
+        auto vc = [&](int i) {
+            const int row = 32 * (i & 1) + r32;
+            return row * 8 + ((4 * khalf + 2 * (i >> 1) + half) ^ pair_swizzle(row));
+        };
+        u32x4 bh = t.h[vc(0)], bl = t.l[vc(0)];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int d = i & 1, gk = i >> 1;
+            u32x4 nh = bh, nl = bl;
+            if (i < 3) nh = t.h[vc(i + 1)], nl = t.l[vc(i + 1)];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) o[d][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_half8(bl), ph[j][gk], o[d][j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) o[d][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_half8(bh), pl[j][gk], o[d][j], 0, 0, 0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) o[d][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_half8(bh), ph[j][gk], o[d][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            bh = nh, bl = nl;
+        }
+    };
+    // Tile u's scores to probabilities.
+    auto softmax = [&](int u) {
+        const int k0 = k_begin + u * kKeyTile;
+        if (__builtin_expect(k0 + kKeyTile > k_end, 0)) {
+            // A range's last tile: its keys past the range score -inf.
+            const int left = k_end - k0 - 32 * khalf - 4 * half;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (8 * (r >> 2) + (r & 3) >= left) s[0][r] = -INFINITY, s[1][r] = -INFINITY;
+        }
+        const f32x4 kinv = *reinterpret_cast<const f32x4 *>(&lds.k_inv[u & 3][4 * khalf]);
+        const f32x2 v0 = lds.v_exp[u & 3][4 * khalf + half], v1 = lds.v_exp[u & 3][4 * khalf + 2 + half];
+        float c[2][4], mx[2], over = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            float t[4];
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                c[j][a] = fmaxf(coef[j] * kinv[a], 1.2e-38f);  // never 0: masked scores are -inf
+                t[a] = fmaxf(fmaxf(s[j][4 * a], s[j][4 * a + 1]), fmaxf(s[j][4 * a + 2], s[j][4 * a + 3])) * c[j][a];
+            }
+            mx[j] = fmaxf(fmaxf(t[0], t[1]) - v0[0], fmaxf(t[2], t[3]) - v1[0]);
+            over = fmaxf(over, mx[j] - m_ref[j]);
+        }
+        if (__builtin_expect(__any(over > 15.0f), 0)) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const float m_new = fmaxf(m_ref[j], halves_max(mx[j]) - 8.0f);
+                const float alpha = __builtin_amdgcn_exp2f(m_ref[j] - m_new);
+                l_run[j] *= alpha;
+                scale_in_place(o[0][j], alpha), scale_in_place(o[1][j], alpha);
+                m_ref[j] = m_new;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int gk = 0; gk < 2; ++gk) {
+                const float off = -(m_ref[j] + (gk ? v1[0] : v0[0]));
+                float x[8], sum = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    x[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j][8 * gk + e], c[j][2 * gk + (e >> 2)], off));
+                    sum += x[e];
+                }
+                l_run[j] = __builtin_fmaf(sum, gk ? v1[1] : v0[1], l_run[j]);
+                pair8(x, ph[j][gk], pl[j][gk]);
+            }
+    };
+
+    // Adds the accumulators into the query group's totals in LDS (start: sets
+    // them) and clears them. The halves do this in different phases.
+    Totals &tot = lds.data.totals;
+    const int slot = qgroup * 64 + lane;
+    auto flush = [&](bool start) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const float m_old = start ? kLowest : tot.m[j][slot], l_old = start ? 0.f : tot.l[j][slot];
+            const float m_new = fmaxf(m_old, m_ref[j]);
+            const float a = __builtin_amdgcn_exp2f(m_old - m_new), b = __builtin_amdgcn_exp2f(m_ref[j] - m_new);
+            tot.m[j][slot] = m_new, tot.l[j][slot] = l_old * a + l_run[j] * b;
+            l_run[j] = 0.f;
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    f32x4 &dst = *reinterpret_cast<f32x4 *>(tot.o[j][d][i][slot]);
+                    const f32x4 old = start ? f32x4{0.f, 0.f, 0.f, 0.f} : dst;
+                    f32x4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        v[e] = old[e] * a + o[d][j][4 * i + e] * b;
+                        o[d][j][4 * i + e] = 0.f;
+                    }
+                    dst = v;
+                }
+        }
+    };
+
+    const int tiles = (k_end - k_begin + kKeyTile - 1) / kKeyTile;
+    // Tiles past the last repeat it; what is made of them is never used.
+    const int k_last = k_begin + (tiles - 1) * kKeyTile;
+    auto tile_at = [&](int u) { return min(k_begin + u * kKeyTile, k_last); };
+    load_k(k_begin), load_v(k_begin);
+    update_scales();
+    convert_k(0), convert_v(0, 0);
+    load_k(tile_at(1)), load_v(tile_at(1));
+    phase_barrier();
+    scores(0);
+    if (khalf) {
+        // Half 1 runs a phase behind half 0, and writes K a tile ahead of it.
+        update_scales();
+        convert_k(1);
+        load_k(tile_at(2));
+        phase_barrier();
+    }
+    bool flushed = false;
+    int since = 0;
+    for (int t = 0, vb = 0; t < tiles; ++t) {
+        const int vb_next = vb == 2 ? 0 : vb + 1;
+        // VALU phase.
+        if constexpr (FLUSH) {
+            if (since == kFlushTiles) {
+                flush(!flushed && khalf == 0);
+                flushed = true, since = 0;
+            }
+            ++since;
+        }
+        update_scales();
+        convert_k(t + 1 + khalf), convert_v(t + 1, vb_next);
+        load_k(tile_at(t + 2 + khalf)), load_v(tile_at(t + 2));
+        softmax(t);
+        phase_barrier();
+        // MFMA phase.
+        output(vb);
+        scores((t + 1) & 1);
+        phase_barrier();
+        vb = vb_next;
+    }
+    if (khalf == 0) phase_barrier();
+    if (lane == 0) lds.special[wave] = special;
+    __syncthreads();
+    unsigned any_special = 0;
+#pragma unroll
+    for (int w = 0; w < kPairWaves; ++w) any_special |= lds.special[w];
+    if (__builtin_amdgcn_readfirstlane(any_special)) {
+        // Plain FP32 for the whole range: thread pairs (2 i, 2 i + 1) take query i.
+        const int row = tid >> 1, part = tid & 1, qrow = qt * kIclQueries + row;
+        const int safe = min(qrow, p.q_rows - 1);
+        float out[32], m, l;
+        icl_row_fp32(p.q + pair * p.q_pair_stride + (long long)safe * 64, kbase + (long long)k_begin * 64,
+                      vbase + (long long)k_begin * 64, k_end - k_begin, part, out, m, l);
+        if (qrow >= p.q_rows) return;
+        float *dst;
+        if constexpr (!SPLIT) {
+            const int b = pair / kHeads, head = pair - b * kHeads;
+            dst = p.o + ((long long)b * p.q_rows + qrow) * p.ldo + head * 64;
+        } else {
+            const long long prow =
+                g.tail_units ? split * g.part_rows + (long long)tail_unit * kIclQueries + row
+                             : split * g.part_rows + (long long)pair * g.q_padded + qrow;
+            dst = p.partial + prow * 64;
+            if (part == 0) p.partial[(long long)g.splits * g.part_rows * 64 + prow] = m + log2f(l);
+        }
+#pragma unroll
+        for (int d = 0; d < 32; ++d) dst[32 * part + d] = out[d] / l;
+        return;
+    }
+    if (khalf == 0) flush(!flushed);
+    __syncthreads();
+    if (khalf == 1) flush(false);
+    __syncthreads();
+
+    // Wave (qgroup, khalf) writes dim block khalf of its query group.
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int qrow = qrow0 + 32 * j;
+        const float l = halves_sum(tot.l[j][slot]);
         if (qrow >= p.q_rows) continue;
-        const float inv = 1.0f / l_tot;
+        const float inv = 1.0f / l;
         float *dst;
         if constexpr (!SPLIT) {
             const int b = pair / kHeads, head = pair - b * kHeads;
@@ -468,14 +659,14 @@ __global__ __launch_bounds__(kIclWaves * 64, 1) void icl_attention_kernel(IclAtt
                 g.tail_units ? split * g.part_rows + (long long)tail_unit * kIclQueries + (qrow - qt * kIclQueries)
                              : split * g.part_rows + (long long)pair * g.q_padded + qrow;
             dst = p.partial + row * 64;
-            if (half == 0) p.partial[(long long)g.splits * g.part_rows * 64 + row] = m_ref[j] + log2f(l_tot);
+            if (half == 0 && khalf == 0)
+                p.partial[(long long)g.splits * g.part_rows * 64 + row] = tot.m[j][slot] + log2f(l);
         }
+        // Register r of block d: dims 32 d + 8 (r / 4) + 4 half + r % 4.
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int i = half * 4 + (r & 3) + 8 * (r >> 2);
-            f32x2 v;
-            v[0] = o[j][0][r] * inv, v[1] = o[j][1][r] * inv;
-            *reinterpret_cast<f32x2 *>(dst + 2 * i) = v;
+        for (int i = 0; i < 4; ++i) {
+            const f32x4 v = *reinterpret_cast<const f32x4 *>(tot.o[j][khalf][i][slot]);
+            *reinterpret_cast<f32x4 *>(dst + 32 * khalf + 8 * i + 4 * half) = v * inv;
         }
     }
 }
@@ -501,15 +692,10 @@ __global__ __launch_bounds__(kIclWaves * 64, 1) void icl_attention_kernel(IclAtt
 // of row r is stored at chunk c ^ (r % 8) so that the 8 rows a half-wave
 // group reads hit distinct banks. Probabilities stay below 2^15 (the lazy
 // reference's limit here), so their high parts fit FP16.
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-
 struct IclTile16 {
     u32x4 k[kKeyTile * 8];  // 64 rows x 8 chunks of 16 bytes
     u32x4 v[kKeyTile * 8];
 };
-
-__device__ __forceinline__ half8 as_half8(u32x4 v) { return __builtin_bit_cast(half8, v); }
 
 // FP8 tiles (IRX_PRECISION_HALF): K [64 keys x 64 bytes] and V^T [64 dims x
 // 64 keys] bytes, 4 KB each; the 16-byte chunk c of row r is stored at chunk
@@ -2300,7 +2486,7 @@ void icl_attention(const IclAttention &args, hipStream_t stream) {
         } else {
             // Ranges of more than 2 x kFlushTiles tiles accumulate in two levels.
             auto wide = [&](const IclLaunch &l) {
-                const dim3 grid(l.per_xcd * 8), block(kIclWaves * 64);
+                const dim3 grid(l.per_xcd * 8), block(kPairWaves * 64);
                 const bool flush = l.keys_per_split > 2 * kFlushTiles * kKeyTile;
                 if (l.splits > 1 && flush)
                     hipLaunchKernelGGL((icl_attention_kernel<true, true>), grid, block, 0, stream, args, l);

@@ -100,6 +100,77 @@ def attention64(q, k, v, scale):
     return (p / p.sum(-1, keepdims=True)) @ v.astype(np.float64)
 
 
+@pytest.mark.parametrize("query_rows,rows", [(33, 1), (65, 31), (64, 129), (257, 700), (300, 9001)])
+@pytest.mark.parametrize("kind", ["spread", "tiny", "large", "zeros", "outlier"])
+def test_icl_attention_operand_ranges(device, query_rows, rows, kind):
+    """The FP16-pair products scale their operands by the magnitudes they meet:
+    per query row, and per eight keys. Keys and values spread over 2^-12 ..
+    2^12 from row to row (with queries kept small, so that scores stay of
+    order one) and dims over 2^-6 .. 2^6; all of them tiny or large; rows of
+    zeros; one key of 1e4 times the others' size that no query attends to. An
+    error is at most a few FP32 roundings of the row's sum of |p v| (2^-18 of
+    it: scores of at most 16 carry 16 x 2^-23, exponentiated, and the sums'
+    roundings)."""
+    pairs = 8
+    rng = np.random.default_rng(query_rows + rows)
+    q, k, v = (rng.standard_normal((pairs, n, 64)).astype(np.float32) for n in (query_rows, rows, rows))
+    if kind == "spread":
+        v *= np.exp2(rng.integers(-12, 13, (pairs, rows, 1))).astype(np.float32)
+        v *= np.exp2(rng.integers(-6, 7, (1, 1, 64))).astype(np.float32)
+        size = np.exp2(rng.integers(-12, 1, (pairs, rows, 1))).astype(np.float32)
+        k *= size
+    elif kind == "tiny":
+        k *= np.float32(1e-20)
+        q *= np.float32(1e20)
+        v *= np.float32(1e-30)
+    elif kind == "large":
+        k *= np.float32(1e18)
+        q *= np.float32(1e-18)
+        v *= np.float32(1e30)
+    elif kind == "zeros":
+        k[:, rows // 3:] = 0.0
+        v[:, : rows // 2] = 0.0
+        q[:, ::2] = 0.0
+    else:
+        q = np.abs(q)
+        k[:, rows // 2] = -1e4 * np.abs(k[:, rows // 2])
+        v[:, rows // 2] *= np.float32(1e4)
+    out = np.zeros_like(q)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_icl_attention(device.handle, F(q), F(k), F(v), pairs, query_rows, rows, F(out)))
+    for pair in (0, 7):
+        scores = q[pair].astype(np.float64) @ k[pair].astype(np.float64).T / 8.0
+        p = np.exp(scores - scores.max(axis=1, keepdims=True))
+        p /= p.sum(axis=1, keepdims=True)
+        want = p @ v[pair].astype(np.float64)
+        bound = p @ np.abs(v[pair]).astype(np.float64)
+        worst = (np.abs(out[pair] - want) / np.maximum(bound, 1e-300)).max() if rows > 1 or kind != "zeros" else 0.0
+        assert worst < 2.0 ** -18, (pair, worst)
+
+
+@pytest.mark.parametrize("query_rows,rows", [(33, 40), (300, 9001)])
+def test_icl_attention_beyond_the_scaled_products(device, query_rows, rows):
+    """Keys and values that no scaled FP16 pair serves go to the plain FP32
+    loop: infinite values stay infinite in their own dim only, and a key of
+    the type's lowest value scores below every other and is left out."""
+    pairs = 8
+    rng = np.random.default_rng(7)
+    q, k, v = (rng.standard_normal((pairs, n, 64)).astype(np.float32) for n in (query_rows, rows, rows))
+    q[:, :, 0] = 1.0
+    k[:, rows - 1] = 0.0
+    k[:, rows - 1, 0] = np.finfo(np.float32).min
+    v[0, rows // 2, 5] = np.inf
+    out = np.zeros_like(q)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_icl_attention(device.handle, F(q), F(k), F(v), pairs, query_rows, rows, F(out)))
+    for pair in (0, 7):
+        want = attention64(q[pair], k[pair, :-1], np.where(np.isinf(v[pair, :-1]), 0.0, v[pair, :-1]), 0.125)
+        if pair == 0:
+            assert np.all(out[0, :, 5] == np.inf)
+            want[:, 5] = out[0, :, 5] = 0.0
+        assert np.abs(out[pair] - want).max() < 1e-5
+
+
 @pytest.mark.parametrize("rows", [1, 63, 64, 65, 2000, 10007])
 def test_icl_attention_matches_float64(device, rows):
     pairs = 64
