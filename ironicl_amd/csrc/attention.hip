@@ -38,7 +38,6 @@ namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 
 // This file builds with IEEE mode off (-mno-amdgpu-ieee), which the device
 // library's work-item functions were not built with, so they would stay
@@ -63,10 +62,6 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 constexpr int kIclWaves = 4;
 constexpr int kIclQueries = kIclWaves * 64;  // queries per workgroup, 64 per wave
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ half8 as_half8(u32x4 v) { return __builtin_bit_cast(half8, v); }
 
 __device__ __forceinline__ void wait_loads() {
     // vmcnt(0); expcnt and lgkmcnt left at their maxima (no wait).
@@ -108,17 +103,8 @@ constexpr int kFlushTiles = 64;
 
 // ---- FP32 attention of wide passes: FP32 operands as pairs of FP16 values ----
 //
-// Every operand x of the two products (queries, keys, probabilities, values)
-// is scaled by a power of two and split into hi = fp16(x), lo = fp16(x - hi),
-// both rounded to nearest: hi + lo holds x to 2^-23. A product is
-//   lo.hi + hi.lo + hi.hi
-// into one FP32 accumulator on the 32x32x16 FP16 MFMA (lo.lo, below 2^-24 of
-// the product, is left out). Random operands against float64 (K = 64 / 512 /
-// 4,096 / 16,384): 1.1e-7 / 2.6e-7 / 7.2e-7 / 1.5e-6 of the result, where the
-// FP32 MFMA gives 1.4e-7 / 4.0e-7 / 1.1e-6 / 2.3e-6 (it rounds its
-// accumulator every two terms, this one every sixteen); truncated parts would
-// give 3.6e-7 at K = 64. Three FP16 products cost 3/16 of an FP32 one, and
-// unlike FP32 MFMAs they run beside the other wave's VALU work.
+// Queries, keys, probabilities and values are scaled by powers of two and held
+// as FP16 pairs (common.hpp); products on the 32x32x16 FP16 MFMA.
 //
 // A workgroup is eight waves: wave w takes queries 64 (w % 4) .. + 63 of the
 // tile against key half w / 4 of each 64-key tile, so the two waves of a SIMD
@@ -177,34 +163,6 @@ struct IclPairTiles {
 __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 constexpr int kPairWaves = 8;
 constexpr float kPairHigh = 32768.0f, kPairLow = 2048.0f;
-
-// Eight FP32 values as FP16 pairs, both parts rounded to nearest.
-__device__ __forceinline__ void pair8(const float *x, half8 &hi, half8 &lo) {
-    typedef _Float16 half2 __attribute__((ext_vector_type(2)));
-    // An opaque -1 makes each remainder one v_fma_mix_f32 (as a subtraction it
-    // is a conversion and a subtraction).
-    float minus = -1.0f;
-    asm("" : "+s"(minus));
-    u32x4 h, l;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const half2 hp = __builtin_convertvector((f32x2{x[2 * i], x[2 * i + 1]}), half2);
-        const f32x2 r = {__builtin_fmaf((float)hp[0], minus, x[2 * i]), __builtin_fmaf((float)hp[1], minus, x[2 * i + 1])};
-        const half2 lp = __builtin_convertvector(r, half2);
-        h[i] = __builtin_bit_cast(unsigned, hp);
-        l[i] = __builtin_bit_cast(unsigned, lp);
-    }
-    hi = __builtin_bit_cast(half8, h);
-    lo = __builtin_bit_cast(half8, l);
-}
-
-// 2^e for -126 <= e <= 127.
-__device__ __forceinline__ float pow2(int e) { return __uint_as_float((unsigned)(e + 127) << 23); }
-// The exponent of the scale that brings a finite magnitude `m` into [2^13,
-// 2^14) (as far as 2^e and 2^-e are normal).
-__device__ __forceinline__ int pair_exponent(float m) {
-    return min(126, 13 - ((int)(__float_as_uint(m) >> 23) - 127));
-}
 
 // One query against `keys` keys in plain FP32 by a pair of threads (32 dims
 // each) with a running maximum: the unnormalized output, its sum and reference.

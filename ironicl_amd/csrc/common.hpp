@@ -54,6 +54,52 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// ---- FP32 operands as pairs of FP16 values ----
+//
+// Products on the FP16 matrix cores hold an FP32 operand x, scaled by a power
+// of two into FP16's range, as hi = fp16(x) and lo = fp16(x - hi), both rounded
+// to nearest: hi + lo is x to 2^-23 (down to 2^-25 absolute). A product is
+// lo.hi + hi.lo + hi.hi into one FP32 accumulator; lo.lo, below 2^-24 of it, is
+// left out. Random operands against float64 (K = 64 / 512 / 4,096 / 16,384):
+// 1.1e-7 / 2.6e-7 / 7.2e-7 / 1.5e-6 of the result, where the FP32 MFMA gives
+// 1.4e-7 / 4.0e-7 / 1.1e-6 / 2.3e-6 (it rounds its accumulator every two to four
+// terms, the FP16 one every 16 or 32); parts rounded toward zero would give
+// 3.6e-7 at K = 64. Three FP16 products take 3/16 of an FP32 one's cycles, and
+// unlike FP32 MFMAs they run beside VALU work.
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ half8 as_half8(u32x4 v) { return __builtin_bit_cast(half8, v); }
+
+// Eight FP32 values as FP16 pairs, both parts rounded to nearest.
+__device__ __forceinline__ void pair8(const float *x, half8 &hi, half8 &lo) {
+    typedef _Float16 half2 __attribute__((ext_vector_type(2)));
+    // An opaque -1 makes each remainder one v_fma_mix_f32 (as a subtraction it
+    // is a conversion and a subtraction).
+    float minus = -1.0f;
+    asm("" : "+s"(minus));
+    u32x4 h, l;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const half2 hp = __builtin_convertvector((f32x2{x[2 * i], x[2 * i + 1]}), half2);
+        const f32x2 r = {__builtin_fmaf((float)hp[0], minus, x[2 * i]), __builtin_fmaf((float)hp[1], minus, x[2 * i + 1])};
+        const half2 lp = __builtin_convertvector(r, half2);
+        h[i] = __builtin_bit_cast(unsigned, hp);
+        l[i] = __builtin_bit_cast(unsigned, lp);
+    }
+    hi = __builtin_bit_cast(half8, h);
+    lo = __builtin_bit_cast(half8, l);
+}
+
+// 2^e for -126 <= e <= 127.
+__device__ __forceinline__ float pow2(int e) { return __uint_as_float((unsigned)(e + 127) << 23); }
+// The exponent of the scale that brings a finite magnitude `m` into [2^13,
+// 2^14) (as far as 2^e and 2^-e are normal).
+__device__ __forceinline__ int pair_exponent(float m) {
+    return min(126, 13 - ((int)(__float_as_uint(m) >> 23) - 127));
+}
+
 // GELU, 0.5 x (1 + erf(x / sqrt 2)) (src/kernels/reference.rs:52-54), with
 // 1 + erf(x / sqrt 2) = 2 - erfc(t) for x >= 0 and erfc(t) for x < 0, t =
 // |x| / sqrt 2, and erfc(t) = 2^P(t) from one polynomial P(t) = t Q(t) of
@@ -156,8 +202,10 @@ bool gemm_fuses_ln(long long m, int n);
 // Post-attention half of a 128-wide block in one kernel (cpu.rs:1555-1601):
 // s1 = state + (att Wo^T + bo); state = s1 + (gelu(LN2(s1) W1^T + b1) W2^T + b2).
 // `pack` holds Wo [128,128], W1 [256,128] and W2 [128,256] as packed by
-// tail128_pack (host code, kTail128PackFloats floats).
-constexpr size_t kTail128PackFloats = 10 * 8192;
+// tail128_pack (host code, kTail128PackFloats floats): FP16 pairs, then
+// kPackScales words of scales.
+constexpr size_t kPackScales = 64;
+constexpr size_t kTail128PackFloats = 10 * 8192 + kPackScales;
 struct Tail128 {
     const float *att;  // [m, 128], row stride lda
     long long lda;
@@ -167,7 +215,8 @@ struct Tail128 {
     const float *bo, *n2w, *n2b, *b1, *b2;  // all [128] or [256]; bias-free LayerNorms pass zeros
     long long m;
 };
-void tail128_pack(const float *wo, const float *w1, const float *w2, float *out);
+void tail128_pack(const float *wo, const float *n2w, const float *n2b, const float *w1, const float *b1,
+                  const float *w2, float *out);
 // rows16: the small-pass form (16 rows per workgroup, bitwise the same results).
 void tail128(const Tail128 &t, hipStream_t stream, bool rows16 = false);
 
@@ -185,8 +234,10 @@ struct Head128 {
     long long m;
     int nb;
 };
-size_t head128_pack_floats(int outputs);
-void head128_pack(const float *w, int outputs, float *out);
+constexpr __host__ __device__ size_t head128_pack_floats(int outputs) {
+    return (size_t)(8 * (outputs / 16) + 31) / 32 * 8192 + kPackScales;
+}
+void head128_pack(const float *lnw, const float *lnb, const float *w, int outputs, float *out);
 void head128(const Head128 &h, hipStream_t stream);
 
 // A cached column block in one kernel (multihead_attn2 of a column ISAB block

@@ -732,18 +732,21 @@ struct Loader {
     // Out-projection and FFN weights of a 128-wide block in tail128's fragment order.
     void pack_tail(BlockW &b) {
         const size_t wo = offset_of(&b.out.w), w1 = offset_of(&b.l1.w), w2 = offset_of(&b.l2.w);
+        const size_t b1 = offset_of(&b.l1.b), nw = offset_of(&b.n2w), nb = offset_of(&b.n2b);
         const size_t offset = (host.size() + 63) / 64 * 64;
         host.resize(offset + kTail128PackFloats, 0.f);
-        tail128_pack(host.data() + wo, host.data() + w1, host.data() + w2, host.data() + offset);
+        const float *f = host.data();
+        tail128_pack(f + wo, f + nw, f + nb, f + w1, f + b1, f + w2, host.data() + offset);
         pending.push_back({&b.tail_pack, offset});
     }
 
     // The in_proj rows [row0, row0 + outputs) of a 128-wide block in head128's fragment order.
     void pack_head(BlockW &b, int row0, int outputs) {
-        const size_t w = offset_of(&b.in_w);
+        const size_t w = offset_of(&b.in_w), nw = offset_of(&b.n1w), nb = offset_of(&b.n1b);
         const size_t offset = (host.size() + 63) / 64 * 64;
         host.resize(offset + head128_pack_floats(outputs), 0.f);
-        head128_pack(host.data() + w + (size_t)row0 * 128, outputs, host.data() + offset);
+        const float *f = host.data();
+        head128_pack(f + nw, f + nb, f + w + (size_t)row0 * 128, outputs, host.data() + offset);
         pending.push_back({&b.head_pack, offset});
         b.head_nb = outputs / 16, b.head_row0 = row0;
     }
@@ -2169,7 +2172,7 @@ int irx_test_block_head(irx_device *device, int fused, const float *x, size_t ro
             fail(IRX_INVALID_ARGUMENT, "block head arguments do not match");
         set_device(device);
         std::vector<float> pack(head128_pack_floats((int)outputs));
-        head128_pack(w, (int)outputs, pack.data());
+        head128_pack(lnw, lnb, w, (int)outputs, pack.data());
         auto up = [](const float *h, size_t count) {
             DevBuf d(count * 4);
             IRX_HIP(hipMemcpy(d.p, h, count * 4, hipMemcpyHostToDevice));
@@ -2211,7 +2214,7 @@ int irx_test_block_tail(irx_device *device, int fused, const float *att, const f
         for (int i = 0; i < 9; ++i) offs[i] = total, total += (sizes[i] + 63) / 64 * 64;
         host.assign(total, 0.f);
         for (int i = 0; i < 8; ++i) std::memcpy(host.data() + offs[i], srcs[i], sizes[i] * 4);
-        tail128_pack(wo, w1, w2, host.data() + offs[8]);
+        tail128_pack(wo, n2w, n2b, w1, b1, w2, host.data() + offs[8]);
         DevBuf dw(total * 4), datt(n * 4), dstate(n * 4), dnorm(n * 4), dhid(2 * n * 4);
         IRX_HIP(hipMemcpy(dw.p, host.data(), total * 4, hipMemcpyHostToDevice));
         IRX_HIP(hipMemcpy(datt.p, att, n * 4, hipMemcpyHostToDevice));
@@ -2253,8 +2256,8 @@ int irx_test_column_block(irx_device *device, int fused, const float *state, siz
         for (int i = 0; i < kParts; ++i) offs[i] = total, total += (sizes[i] + 63) / 64 * 64;
         host.assign(total, 0.f);
         for (int i = 0; i < 12; ++i) std::memcpy(host.data() + offs[i], srcs[i], sizes[i] * 4);
-        head128_pack(wq, 128, host.data() + offs[12]);
-        tail128_pack(wo, w1, w2, host.data() + offs[13]);
+        head128_pack(lnw, lnb, wq, 128, host.data() + offs[12]);
+        tail128_pack(wo, n2w, n2b, w1, b1, w2, host.data() + offs[13]);
         DevBuf dw(total * 4), dstate(n * 4), dk(cols * kColumnCache * 4), dv(cols * kColumnCache * 4);
         DevBuf dnorm(n * 4), dq(n * 4), datt(n * 4), dhid(2 * n * 4);
         IRX_HIP(hipMemcpy(dw.p, host.data(), total * 4, hipMemcpyHostToDevice));

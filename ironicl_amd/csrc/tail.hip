@@ -8,24 +8,35 @@
 // registers.
 //
 // Each wave owns 16 rows for the whole chain. Products are computed
-// transposed, D = W X^T, on v_mfma_f32_16x16x4f32: the weights are the A
-// operand and the rows the B operand. In D, lane (m, g) = (lane % 16,
-// lane / 16) holds row m's features 16 b + 4 g + r in register r of block b,
-// which is exactly what the next product's B operand needs at step r of
-// k-block b, so the chain runs without moving data between lanes. The same
-// per-lane layout is used to load att and state and to store the result.
+// transposed, D = W X^T, on v_mfma_f32_16x16x32_f16 with both operands as FP16
+// pairs (common.hpp): the weights are the A operand and the rows the B
+// operand. In D, lane (m, g) = (lane % 16, lane / 16) holds row m's features
+// 16 b + 4 g + r in register r of block b. The next product's B operand, for
+// the 32 features of blocks 2 kb and 2 kb + 1, is the lane's eight of them:
+// slot e is feature 32 kb + 16 (e / 4) + 4 g + e % 4, and the A operand's slots
+// are packed the same way, so the chain runs without moving data between
+// lanes. The same per-lane layout is used to load att and state and to store
+// the result.
+//
+// Scales. Weights are packed times a power of two that brings the matrix's
+// largest into [2^13, 2^14). LayerNormed rows are bounded by sqrt(128) times
+// the weights' largest plus the biases', the hidden layer by its weights' row
+// norms, so their scales are fixed when the weights are packed; attention
+// outputs, which can come from an imported cache, are scaled by row.
 //
 // The weights are packed once (tail128_pack) into A-operand fragments, 1 KB
-// per 16 x 16 block, lane after lane, in the order the kernel consumes them:
-// ten 32 KB chunks (Wo in two, then per 32-unit slice of the hidden layer the
-// W1 rows and W2 columns it touches). A workgroup streams each chunk as two
-// 16 KB halves (out-projection k-blocks, or a slice's W1 rows then its W2
-// columns) through two 16 KB LDS buffers with direct global -> LDS loads, so
+// per 16 x 32 block of hi or lo parts, lane after lane, in the order the kernel
+// consumes them: ten 32 KB chunks (Wo in two, then per 32-unit slice of the
+// hidden layer the W1 rows and W2 columns it touches). A workgroup streams
+// each chunk as two 16 KB halves (an out-projection k-block, or a slice's W1
+// rows then its W2 columns) through two 16 KB LDS buffers with direct global ->
+// LDS loads, so
 // three workgroups share a CU; every LDS read is one 16-byte read per lane
 // of consecutive addresses (no bank conflicts).
 #include "common.hpp"
 
 #include <algorithm>
+#include <cmath>
 
 namespace irx {
 namespace {
@@ -51,6 +62,74 @@ __device__ __forceinline__ f32x4 mfma(float a, float b, const f32x4 &acc) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
 }
 
+// An operand of 32 k-slots as an FP16 pair.
+struct Pair {
+    half8 h, l;
+};
+
+// acc += W X over 32 k-slots for N output blocks, each accumulator's products
+// in the same order in every kernel (the small-pass forms repeat the bits).
+template <int N>
+__device__ __forceinline__ void pair_mfma(const Pair (&w)[N], const Pair &x, f32x4 (&acc)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[i].l, x.h, acc[i], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[i].h, x.l, acc[i], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < N; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w[i].h, x.h, acc[i], 0, 0, 0);
+}
+
+// The fragments (hi, then lo 1 KB further) at `f`, the lane's base.
+__device__ __forceinline__ Pair pair_at(const float *f) {
+    return {as_half8(*reinterpret_cast<const u32x4 *>(f)), as_half8(*reinterpret_cast<const u32x4 *>(f + 256))};
+}
+
+// acc[0..7] += eight output blocks' fragments at `frag` times x, four at a
+// time (all eight in flight take registers the kernels need).
+__device__ __forceinline__ void pair_blocks(const float *frag, const Pair &x, f32x4 *acc) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        Pair f[4];
+        f32x4 a[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) f[i] = pair_at(frag + (4 * half + i) * 512), a[i] = acc[4 * half + i];
+        pair_mfma<4>(f, x, a);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[4 * half + i] = a[i];
+    }
+}
+
+// The lane's features of blocks 2 kb and 2 kb + 1, times `scale`.
+__device__ __forceinline__ Pair pair_of(const f32x4 &a, const f32x4 &b, float scale) {
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = a[e] * scale, y[4 + e] = b[e] * scale;
+    Pair p;
+    pair8(y, p.h, p.l);
+    return p;
+}
+
+// The exponent that brings the row's largest of x (over the row's four lanes)
+// into [2^13, 2^14).
+__device__ __forceinline__ int row_exponent(const f32x4 (&x)[8]) {
+    float m = 0.f;
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(x[b][e]));
+    m = fmaxf(m, __shfl_xor(m, 16, 64));
+    m = fmaxf(m, __shfl_xor(m, 32, 64));
+    return pair_exponent(m);
+}
+
+// Words of scales after a pack's fragments. Tail: the out-projection's inverse
+// weight scale; LN2's scale and the inverse of its product's; the hidden
+// layer's and the inverse of its product's. Head: LN1's and the inverse of its
+// product's.
+constexpr size_t kTailScales = 10 * 8192;
+enum { kTailOutInv, kTailLn, kTailLnInv, kTailHid, kTailHidInv };
+enum { kHeadLn, kHeadInv };
+
 __device__ __forceinline__ f32x4 lds4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
 
 // The chain after a 128-wide block's attention (cpu.rs:1555-1601): x holds
@@ -61,31 +140,22 @@ __device__ __forceinline__ f32x4 lds4(const float *p) { return *reinterpret_cast
 template <class Next>
 __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &&next, int h0, const Tail128 &t,
                                            float *out, bool live, int g) {
+    const float *sc = t.pack + kTailScales;
     f32x4 acc[8];
 #pragma unroll
     for (int b = 0; b < 8; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // Out-projection: half-chunks 0 .. 3 hold k-blocks 2 hc and 2 hc + 1,
-    // each with the eight output blocks' fragments. The second k-block's
-    // fragments are read while the first one's 32 products (8 independent
-    // accumulators) run.
+    // Out-projection: half-chunk hc holds 32-wide k-block hc's fragments of the
+    // eight output blocks.
+    const int ea = row_exponent(x);
+    const float a_scale = pow2(ea), a_inv = sc[kTailOutInv] * pow2(-ea);
+    Pair xp[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) xp[kb] = pair_of(x[2 * kb], x[2 * kb + 1], a_scale);
 #pragma unroll
     for (int hc = 0; hc < 4; ++hc) {
         const float *frag = next(h0 + hc);
-        f32x4 fa[2][8];
-#pragma unroll
-        for (int ob = 0; ob < 8; ++ob) fa[0][ob] = lds4(frag + ob * 256);
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
-            if (kb == 0) {
-#pragma unroll
-                for (int ob = 0; ob < 8; ++ob) fa[1][ob] = lds4(frag + (8 + ob) * 256);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int ob = 0; ob < 8; ++ob) acc[ob] = mfma(fa[kb][ob][e], x[2 * hc + kb][e], acc[ob]);
-        }
+        pair_blocks(frag, xp[hc], acc);
     }
 
     // s1 = state + (acc + bo), then LN2 over the row's 128 features, held by
@@ -96,7 +166,7 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
         const f32x4 bo = *reinterpret_cast<const f32x4 *>(t.bo + 16 * b + 4 * g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            s1[b][e] = s1[b][e] + (acc[b][e] + bo[e]);
+            s1[b][e] = s1[b][e] + __builtin_fmaf(acc[b][e], a_inv, bo[e]);
             sum += s1[b][e];
         }
     }
@@ -127,44 +197,31 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
     // 16 hb + 4 g + e from half-chunk 4 + 2 c (even and odd k-blocks in
     // separate accumulators, four independent chains), then acc += W2 h from
     // half-chunk 5 + 2 c.
+    const float ln_scale = sc[kTailLn], ln_inv = sc[kTailLnInv], hid_scale = sc[kTailHid], hid_inv = sc[kTailHidInv];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) xp[kb] = pair_of(x[2 * kb], x[2 * kb + 1], ln_scale);
 #pragma unroll 1
     for (int c = 0; c < 8; ++c) {
         const float *frag = next(h0 + 4 + 2 * c);
         f32x4 h[2][2];
 #pragma unroll
         for (int i = 0; i < 4; ++i) h[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
-        f32x4 fw[2][2];
-        fw[0][0] = lds4(frag), fw[0][1] = lds4(frag + 256);
 #pragma unroll
-        for (int kb = 0; kb < 8; ++kb) {
-            if (kb < 7) {
-                fw[(kb + 1) & 1][0] = lds4(frag + ((kb + 1) * 2) * 256);
-                fw[(kb + 1) & 1][1] = lds4(frag + ((kb + 1) * 2 + 1) * 256);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int hb = 0; hb < 2; ++hb) h[hb][kb & 1] = mfma(fw[kb & 1][hb][e], x[kb][e], h[hb][kb & 1]);
+        for (int kb = 0; kb < 4; ++kb) {
+            const Pair f[2] = {pair_at(frag + (kb * 2) * 512), pair_at(frag + (kb * 2 + 1) * 512)};
+            pair_mfma<2>(f, xp[kb], h[kb & 1]);
         }
         f32x4 hg[2];
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
             const f32x4 b1 = *reinterpret_cast<const f32x4 *>(t.b1 + 32 * c + 16 * hb + 4 * g);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) hg[hb][e] = gelu_erf((h[hb][0][e] + h[hb][1][e]) + b1[e]);
-        }
-        const float *frag2 = next(h0 + 5 + 2 * c);
-        f32x4 f2[2][8];
-#pragma unroll
-        for (int ob = 0; ob < 8; ++ob) f2[0][ob] = lds4(frag2 + ob * 256);
-#pragma unroll
-        for (int ob = 0; ob < 8; ++ob) f2[1][ob] = lds4(frag2 + (8 + ob) * 256);
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
             for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int ob = 0; ob < 8; ++ob) acc[ob] = mfma(f2[j][ob][e], hg[j][e], acc[ob]);
+                hg[hb][e] = gelu_erf(__builtin_fmaf(h[0][hb][e] + h[1][hb][e], ln_inv, b1[e]));
+        }
+        const Pair hp = pair_of(hg[0], hg[1], hid_scale);
+        const float *frag2 = next(h0 + 5 + 2 * c);
+        pair_blocks(frag2, hp, acc);
     }
 
     if (!live) return;
@@ -173,7 +230,7 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
         const f32x4 b2 = *reinterpret_cast<const f32x4 *>(t.b2 + 16 * b + 4 * g);
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = (acc[b][e] + b2[e]) + s1[b][e];
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[b][e], hid_inv, b2[e]) + s1[b][e];
         *reinterpret_cast<f32x4 *>(out + 16 * b) = v;
     }
 }
@@ -312,23 +369,24 @@ __global__ __launch_bounds__(256, 3) void column_block_kernel(ColumnBlock p, int
 
     // q: lane (m, g) holds head h's dims 4 g .. 4 g + 3 of row m in q[h],
     // scaled into the exp2 domain (1 / sqrt(16) = 0.25).
+    const float *qsc = p.qpack + head128_pack_floats(128) - kPackScales;
+    const float ln_scale = qsc[kHeadLn], q_inv = qsc[kHeadInv];
     f32x4 q[8];
 #pragma unroll
     for (int ob = 0; ob < 8; ++ob) q[ob] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
+        const Pair xp = pair_of(x[2 * c], x[2 * c + 1], ln_scale);
         const float *frag = next(c) + lane * 4;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int f = 16 * c + i, kb = f / 8, ob = f % 8;
-            const f32x4 a = lds4(frag + i * 256);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) q[ob] = mfma(a[e], x[kb][e], q[ob]);
-        }
+        pair_blocks(frag, xp, q);
     }
     const float scale = 0.25f * kLog2e;
 #pragma unroll
-    for (int ob = 0; ob < 8; ++ob) q[ob] = (q[ob] + *reinterpret_cast<const f32x4 *>(p.qb + 16 * ob + 4 * g)) * scale;
+    for (int ob = 0; ob < 8; ++ob) {
+        const f32x4 qb = *reinterpret_cast<const f32x4 *>(p.qb + 16 * ob + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[ob][e] = __builtin_fmaf(q[ob][e], q_inv, qb[e]) * scale;
+    }
 
     // Per head: S^T = K Q^T (lane (m, g) holds keys 16 kb + 4 g + r of row
     // m), the exact softmax over the 128 keys, O^T = V^T P^T, which leaves
@@ -373,7 +431,7 @@ __global__ __launch_bounds__(256, 3) void column_block_kernel(ColumnBlock p, int
     }
 
     Tail128 t{};
-    t.bo = p.bo, t.n2w = p.n2w, t.n2b = p.n2b, t.b1 = p.b1, t.b2 = p.b2;
+    t.pack = p.pack, t.bo = p.bo, t.n2w = p.n2w, t.n2b = p.n2b, t.b1 = p.b1, t.b2 = p.b2;
     tail_chain(att, s1, [&](int h) { return next(h) + lane * 4; }, 12, t, xrow, live, g);
 }
 
@@ -396,28 +454,25 @@ __global__ __launch_bounds__(256, 3) void column_block_kernel(ColumnBlock p, int
 constexpr int kRows16S1Stride = 132, kRows16HidStride = 260;
 
 __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[8], f32x4 (&s1)[2],
-                                             const f32x4 (&fo)[8][2], const f32x4 (&f1)[2][8][2], float *s1s,
+                                             const Pair (&fo)[4][2], const Pair (&f1)[2][4][2], float *s1s,
                                              float *hs, const float *pk, int w, int m16, int g, float *out,
                                              bool live) {
     constexpr int kS1Stride = kRows16S1Stride, kHidStride = kRows16HidStride;
-    auto w2_frag = [&](int c, int j, int ob) {
-        return *reinterpret_cast<const f32x4 *>(pk + (2 + c) * kChunkFloats + 4096 + (j * 8 + ob) * 256);
-    };
+    const float *sc = t.pack + kTailScales;
+    auto w2_frag = [&](int c, int ob) { return pair_at(pk + (2 + c) * kChunkFloats + 4096 + ob * 512); };
     f32x4 xn[8];
     // Out-projection of output blocks 2 w + j; s1 = state + (acc + bo) to LDS.
     f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    const int ea = row_exponent(x);
+    const float a_scale = pow2(ea), a_inv = sc[kTailOutInv] * pow2(-ea);
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[j] = mfma(fo[kb][j][e], x[kb][e], acc[j]);
+    for (int kb = 0; kb < 4; ++kb) pair_mfma<2>(fo[kb], pair_of(x[2 * kb], x[2 * kb + 1], a_scale), acc);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int c0 = 16 * (2 * w + j) + 4 * g;
         const f32x4 bo = *reinterpret_cast<const f32x4 *>(t.bo + c0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s1[j][e] = s1[j][e] + (acc[j][e] + bo[e]);
+        for (int e = 0; e < 4; ++e) s1[j][e] = s1[j][e] + __builtin_fmaf(acc[j][e], a_inv, bo[e]);
         *reinterpret_cast<f32x4 *>(&s1s[m16 * kS1Stride + c0]) = s1[j];
     }
     __syncthreads();
@@ -454,6 +509,10 @@ __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[
     }
 
     // Hidden slices c = 2 w + sl: gelu(W1 x + b1) to LDS.
+    const float ln_scale = sc[kTailLn], ln_inv = sc[kTailLnInv], hid_scale = sc[kTailHid], hid_inv = sc[kTailHidInv];
+    Pair xp[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) xp[kb] = pair_of(xn[2 * kb], xn[2 * kb + 1], ln_scale);
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl) {
         const int c = 2 * w + sl;
@@ -461,42 +520,31 @@ __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[
 #pragma unroll
         for (int i = 0; i < 4; ++i) h[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kb = 0; kb < 8; ++kb)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int hb = 0; hb < 2; ++hb) h[hb][kb & 1] = mfma(f1[sl][kb][hb][e], xn[kb][e], h[hb][kb & 1]);
+        for (int kb = 0; kb < 4; ++kb) pair_mfma<2>(f1[sl][kb], xp[kb], h[kb & 1]);
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
             const f32x4 b1 = *reinterpret_cast<const f32x4 *>(t.b1 + 32 * c + 16 * hb + 4 * g);
             f32x4 hg;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) hg[e] = gelu_erf((h[hb][0][e] + h[hb][1][e]) + b1[e]);
+            for (int e = 0; e < 4; ++e) hg[e] = gelu_erf(__builtin_fmaf(h[0][hb][e] + h[1][hb][e], ln_inv, b1[e]));
             *reinterpret_cast<f32x4 *>(&hs[m16 * kHidStride + 32 * c + 16 * hb + 4 * g]) = hg;
         }
     }
     // This wave's W2 fragments (output blocks 2 w + j), in flight over the barrier.
-    f32x4 f2[8][2][2];
+    Pair f2[8][2];
 #pragma unroll
     for (int c = 0; c < 8; ++c)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int ob = 0; ob < 2; ++ob) f2[c][j][ob] = w2_frag(c, j, 2 * w + ob);
+        for (int ob = 0; ob < 2; ++ob) f2[c][ob] = w2_frag(c, 2 * w + ob);
     __syncthreads();
 
     // FFN down over the 256 hidden units, slice by slice as tail128 does.
     f32x4 acc2[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-    for (int c = 0; c < 8; ++c)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const f32x4 hv = *reinterpret_cast<const f32x4 *>(&hs[m16 * kHidStride + 32 * c + 16 * j + 4 * g]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int ob = 0; ob < 2; ++ob) acc2[ob] = mfma(f2[c][j][ob][e], hv[e], acc2[ob]);
-        }
+    for (int c = 0; c < 8; ++c) {
+        const float *hv = &hs[m16 * kHidStride + 32 * c + 4 * g];
+        pair_mfma<2>(f2[c], pair_of(lds4(hv), lds4(hv + 16), hid_scale), acc2);
+    }
     if (!live) return;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -504,7 +552,7 @@ __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[
         const f32x4 b2 = *reinterpret_cast<const f32x4 *>(t.b2 + c0 + 4 * g);
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = (acc2[j][e] + b2[e]) + s1[j][e];
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc2[j][e], hid_inv, b2[e]) + s1[j][e];
         *reinterpret_cast<f32x4 *>(out + c0) = v;
     }
 }
@@ -520,31 +568,25 @@ __global__ __launch_bounds__(256) void tail128_rows16_kernel(Tail128 p) {
     const bool live = row < p.m;
     const long long r = live ? row : p.m - 1;
     const float *pk = p.pack + lane * 4;
-    // Fragment (k-block kb, output block ob) of Wo; (kb, hb) of slice c's W1
-    // rows (tail128_pack's order).
-    auto wo_frag = [&](int kb, int ob) { return *reinterpret_cast<const f32x4 *>(pk + kb * 2048 + ob * 256); };
-    auto w1_frag = [&](int c, int kb, int hb) {
-        return *reinterpret_cast<const f32x4 *>(pk + (2 + c) * kChunkFloats + (kb * 2 + hb) * 256);
-    };
-
-    f32x4 fo[8][2], x[8], s1[2];
+    Pair fo[4][2];
+    f32x4 x[8], s1[2];
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
+    for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) fo[kb][j] = wo_frag(kb, 2 * w + j);
+        for (int j = 0; j < 2; ++j) fo[kb][j] = pair_at(pk + (kb * 8 + 2 * w + j) * 512);
     const float *att = p.att + r * p.lda + 4 * g;
 #pragma unroll
     for (int b = 0; b < 8; ++b) x[b] = *reinterpret_cast<const f32x4 *>(att + 16 * b);
     const float *st = p.state + r * p.ldx + 4 * g;
 #pragma unroll
     for (int j = 0; j < 2; ++j) s1[j] = *reinterpret_cast<const f32x4 *>(st + 16 * (2 * w + j));
-    f32x4 f1[2][8][2];
+    Pair f1[2][4][2];
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl)
 #pragma unroll
-        for (int kb = 0; kb < 8; ++kb)
+        for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-            for (int hb = 0; hb < 2; ++hb) f1[sl][kb][hb] = w1_frag(2 * w + sl, kb, hb);
+            for (int hb = 0; hb < 2; ++hb) f1[sl][kb][hb] = pair_at(pk + (2 + 2 * w + sl) * kChunkFloats + (kb * 2 + hb) * 512);
 
     rows16_chain(p, x, s1, fo, f1, s1s, hs, pk, w, m16, g, p.state + r * p.ldx + 4 * g, live);
 }
@@ -577,14 +619,15 @@ __global__ __launch_bounds__(256) void column_block_rows16_kernel(ColumnBlock p,
     const float *vh = p.v + coff + (2 * w) * (kInducing * kColumnHead);
     const float *qk = p.qpack + lane * 4, *pk = p.pack + lane * 4;
 
-    f32x4 x[8], fq[8][2], kf[2][8];
+    f32x4 x[8], kf[2][8];
+    Pair fq[4][2];
     float vv[2][8][4];
 #pragma unroll
     for (int b = 0; b < 8; ++b) x[b] = *reinterpret_cast<const f32x4 *>(xrow + 16 * b);
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
+    for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) fq[kb][j] = *reinterpret_cast<const f32x4 *>(qk + (kb * 8 + 2 * w + j) * 256);
+        for (int j = 0; j < 2; ++j) fq[kb][j] = pair_at(qk + (kb * 8 + 2 * w + j) * 512);
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -622,31 +665,32 @@ __global__ __launch_bounds__(256) void column_block_rows16_kernel(ColumnBlock p,
         }
     }
     f32x4 q[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+    const float *qsc = p.qpack + head128_pack_floats(128) - kPackScales;
+    const float q_scale = qsc[kHeadLn], q_inv = qsc[kHeadInv];
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) q[j] = mfma(fq[kb][j][e], x[kb][e], q[j]);
+    for (int kb = 0; kb < 4; ++kb) pair_mfma<2>(fq[kb], pair_of(x[2 * kb], x[2 * kb + 1], q_scale), q);
     const float scale = 0.25f * kLog2e;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) q[j] = (q[j] + *reinterpret_cast<const f32x4 *>(p.qb + 16 * (2 * w + j) + 4 * g)) * scale;
+    for (int j = 0; j < 2; ++j) {
+        const f32x4 qb = *reinterpret_cast<const f32x4 *>(p.qb + 16 * (2 * w + j) + 4 * g);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q[j][e] = __builtin_fmaf(q[j][e], q_inv, qb[e]) * scale;
+    }
 
     // The tail's fragments for this wave and its state blocks, in flight
     // during the attention.
-    f32x4 fo[8][2], f1[2][8][2], s1[2];
+    Pair fo[4][2], f1[2][4][2];
+    f32x4 s1[2];
 #pragma unroll
-    for (int kb = 0; kb < 8; ++kb)
+    for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) fo[kb][j] = *reinterpret_cast<const f32x4 *>(pk + kb * 2048 + (2 * w + j) * 256);
+        for (int j = 0; j < 2; ++j) fo[kb][j] = pair_at(pk + (kb * 8 + 2 * w + j) * 512);
 #pragma unroll
     for (int sl = 0; sl < 2; ++sl)
 #pragma unroll
-        for (int kb = 0; kb < 8; ++kb)
+        for (int kb = 0; kb < 4; ++kb)
 #pragma unroll
-            for (int hb = 0; hb < 2; ++hb)
-                f1[sl][kb][hb] =
-                    *reinterpret_cast<const f32x4 *>(pk + (2 + 2 * w + sl) * kChunkFloats + (kb * 2 + hb) * 256);
+            for (int hb = 0; hb < 2; ++hb) f1[sl][kb][hb] = pair_at(pk + (2 + 2 * w + sl) * kChunkFloats + (kb * 2 + hb) * 512);
 #pragma unroll
     for (int j = 0; j < 2; ++j) s1[j] = *reinterpret_cast<const f32x4 *>(xrow + 16 * (2 * w + j));
 
@@ -688,7 +732,7 @@ __global__ __launch_bounds__(256) void column_block_rows16_kernel(ColumnBlock p,
 #pragma unroll
     for (int b = 0; b < 8; ++b) x[b] = *reinterpret_cast<const f32x4 *>(&as[m16 * kS1Stride + 16 * b + 4 * g]);
     Tail128 t{};
-    t.bo = p.bo, t.n2w = p.n2w, t.n2b = p.n2b, t.b1 = p.b1, t.b2 = p.b2;
+    t.pack = p.pack, t.bo = p.bo, t.n2w = p.n2w, t.n2b = p.n2b, t.b1 = p.b1, t.b2 = p.b2;
     rows16_chain(t, x, s1, fo, f1, s1s, hs, pk, w, m16, g, xrow, live);
 }
 
@@ -701,7 +745,6 @@ __global__ __launch_bounds__(256, 3) void head128_kernel(Head128 p) {
     // per workgroup, so three (four at 8 and 16 output blocks, whose
     // registers allow it) share a CU.
     __shared__ __attribute__((aligned(16))) float buf[2][kHalfFloats];
-    constexpr int kFrags = 8 * NB, kHeadHalves = (kFrags + 15) / 16;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int m16 = lane & 15, g = lane >> 4;
@@ -747,46 +790,78 @@ __global__ __launch_bounds__(256, 3) void head128_kernel(Head128 p) {
         for (int e = 0; e < 4; ++e) x[b][e] = (x[b][e] - mean) * rstd * w[e] + bb[e];
     }
 
+    const float *sc = p.pack + head128_pack_floats(16 * NB) - kPackScales;
+    const float ln_scale = sc[kHeadLn], inv = sc[kHeadInv];
+    Pair xp[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) xp[kb] = pair_of(x[2 * kb], x[2 * kb + 1], ln_scale);
     f32x4 acc[NB];
 #pragma unroll
     for (int ob = 0; ob < NB; ++ob) acc[ob] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // Half c holds the pairs of eight (k-block, output block) fragments.
 #pragma unroll
-    for (int c = 0; c < kHeadHalves; ++c) {
+    for (int c = 0; c < NB / 2; ++c) {
         wait_vm();
         __syncthreads();
-        if (c + 1 < kHeadHalves) issue(c + 1);
+        if (c + 1 < NB / 2) issue(c + 1);
         const float *frag = &buf[c & 1][lane * 4];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int f = 16 * c + i;
-            if (f < kFrags) {
-                const int kb = f / NB, ob = f % NB;
-                const f32x4 a = lds4(frag + i * 256);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[ob] = mfma(a[e], x[kb][e], acc[ob]);
-            }
-        }
+        const int kb = 8 * c / NB, ob0 = 8 * c % NB;
+        pair_blocks(frag, xp[kb], &acc[ob0]);
     }
     if (!live) return;
     float *out = p.out + row * p.ldo + 4 * g;
 #pragma unroll
-    for (int ob = 0; ob < NB; ++ob)
-        *reinterpret_cast<f32x4 *>(out + 16 * ob) = acc[ob] + *reinterpret_cast<const f32x4 *>(p.b + 16 * ob + 4 * g);
+    for (int ob = 0; ob < NB; ++ob) {
+        const f32x4 b = *reinterpret_cast<const f32x4 *>(p.b + 16 * ob + 4 * g);
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[ob][e], inv, b[e]);
+        *reinterpret_cast<f32x4 *>(out + 16 * ob) = v;
+    }
+}
+
+// Fragment pair (rows r0.., columns c0 .. c0 + 31) of a row-major [.., ld]
+// matrix times `scale`: lane (n, g) = (l % 16, l / 16) slot e holds row r0 + n,
+// column c0 + 16 (e / 4) + 4 g + e % 4; 1 KB of hi parts, then of lo parts.
+void pack_pair(const float *w, int ld, int r0, int c0, float scale, float *dst) {
+    _Float16 *hi = reinterpret_cast<_Float16 *>(dst), *lo = reinterpret_cast<_Float16 *>(dst + 256);
+    for (int l = 0; l < 64; ++l)
+        for (int e = 0; e < 8; ++e) {
+            const float x = w[(long long)(r0 + (l & 15)) * ld + c0 + 16 * (e >> 2) + 4 * (l >> 4) + (e & 3)] * scale;
+            const _Float16 h = (_Float16)x;
+            hi[l * 8 + e] = h;
+            lo[l * 8 + e] = (_Float16)(x - (float)h);
+        }
+}
+
+// The exponent that brings magnitudes up to `largest` to at most 2^`top`.
+int scale_exponent(double largest, int top) {
+    if (!(largest > 0.0)) return 0;
+    return std::max(-60, std::min(60, top - 1 - std::ilogb(largest)));
+}
+int weight_exponent(const float *w, size_t count) {
+    float largest = 0.f;
+    for (size_t i = 0; i < count; ++i) largest = std::max(largest, std::fabs(w[i]));
+    return scale_exponent(largest, 14);
+}
+// The bound of a LayerNormed row's values: at most sqrt(128) of deviation.
+int ln_exponent(const float *w, const float *b) {
+    float lw = 0.f, lb = 0.f;
+    for (int i = 0; i < 128; ++i) lw = std::max(lw, std::fabs(w[i])), lb = std::max(lb, std::fabs(b[i]));
+    return scale_exponent(11.5 * lw + lb, 15);
 }
 
 }  // namespace
 
-size_t head128_pack_floats(int outputs) { return (size_t)(8 * (outputs / 16) + 31) / 32 * kChunkFloats; }
-
-void head128_pack(const float *w, int outputs, float *out) {
+void head128_pack(const float *lnw, const float *lnb, const float *w, int outputs, float *out) {
     const int nb = outputs / 16;
     std::fill(out, out + head128_pack_floats(outputs), 0.f);
-    for (int kb = 0; kb < 8; ++kb)
-        for (int ob = 0; ob < nb; ++ob) {
-            float *dst = out + (size_t)(kb * nb + ob) * 256;
-            for (int l = 0; l < 64; ++l)
-                for (int e = 0; e < 4; ++e) dst[l * 4 + e] = w[(long long)(16 * ob + (l & 15)) * 128 + 16 * kb + 4 * (l >> 4) + e];
-        }
+    const int ew = weight_exponent(w, (size_t)outputs * 128), el = ln_exponent(lnw, lnb);
+    for (int kb = 0; kb < 4; ++kb)
+        for (int ob = 0; ob < nb; ++ob)
+            pack_pair(w, 128, 16 * ob, 32 * kb, std::ldexp(1.f, ew), out + (size_t)(kb * nb + ob) * 512);
+    float *sc = out + head128_pack_floats(outputs) - kPackScales;
+    sc[kHeadLn] = std::ldexp(1.f, el), sc[kHeadInv] = std::ldexp(1.f, -el - ew);
 }
 
 void head128(const Head128 &h, hipStream_t stream) {
@@ -808,24 +883,35 @@ void head128(const Head128 &h, hipStream_t stream) {
     IRX_HIP(hipGetLastError());
 }
 
-void tail128_pack(const float *wo, const float *w1, const float *w2, float *out) {
-    // Fragment (rows r0.., columns c0..) of a row-major [.., ld] matrix:
-    // lane (n, g) = (l % 16, l / 16) holds W[r0 + n][c0 + 4 g .. c0 + 4 g + 3].
-    auto fragment = [](const float *w, int ld, int r0, int c0, float *dst) {
-        for (int l = 0; l < 64; ++l)
-            for (int e = 0; e < 4; ++e) dst[l * 4 + e] = w[(long long)(r0 + (l & 15)) * ld + c0 + 4 * (l >> 4) + e];
-    };
-    for (int c = 0; c < 2; ++c)
-        for (int kb = 0; kb < 4; ++kb)
-            for (int ob = 0; ob < 8; ++ob)
-                fragment(wo, 128, 16 * ob, 16 * (4 * c + kb), out + c * kChunkFloats + (kb * 8 + ob) * 256);
+void tail128_pack(const float *wo, const float *n2w, const float *n2b, const float *w1, const float *b1,
+                  const float *w2, float *out) {
+    std::fill(out, out + kTail128PackFloats, 0.f);
+    // A hidden unit: at most sqrt(128) times the norm of its weights times
+    // LN2's, plus what the biases give it; its GELU is no larger.
+    double hidden = 0.0;
+    for (int u = 0; u < 256; ++u) {
+        double norm = 0.0, bias = b1[u];
+        for (int i = 0; i < 128; ++i) {
+            const double a = (double)w1[u * 128 + i] * n2w[i];
+            norm += a * a, bias += (double)w1[u * 128 + i] * n2b[i];
+        }
+        hidden = std::max(hidden, 11.5 * std::sqrt(norm) + std::fabs(bias));
+    }
+    const int eo = weight_exponent(wo, 128 * 128), e1 = weight_exponent(w1, 256 * 128);
+    const int e2 = weight_exponent(w2, 128 * 256), el = ln_exponent(n2w, n2b), eh = scale_exponent(hidden, 15);
+    const float so = std::ldexp(1.f, eo), s1 = std::ldexp(1.f, e1), s2 = std::ldexp(1.f, e2);
+    for (int kb = 0; kb < 4; ++kb)
+        for (int ob = 0; ob < 8; ++ob) pack_pair(wo, 128, 16 * ob, 32 * kb, so, out + (kb * 8 + ob) * 512);
     for (int c = 0; c < 8; ++c) {
         float *chunk = out + (2 + c) * kChunkFloats;
-        for (int kb = 0; kb < 8; ++kb)
-            for (int hb = 0; hb < 2; ++hb) fragment(w1, 128, 32 * c + 16 * hb, 16 * kb, chunk + (kb * 2 + hb) * 256);
-        for (int j = 0; j < 2; ++j)
-            for (int ob = 0; ob < 8; ++ob) fragment(w2, 256, 16 * ob, 32 * c + 16 * j, chunk + 4096 + (j * 8 + ob) * 256);
+        for (int kb = 0; kb < 4; ++kb)
+            for (int hb = 0; hb < 2; ++hb) pack_pair(w1, 128, 32 * c + 16 * hb, 32 * kb, s1, chunk + (kb * 2 + hb) * 512);
+        for (int ob = 0; ob < 8; ++ob) pack_pair(w2, 256, 16 * ob, 32 * c, s2, chunk + 4096 + ob * 512);
     }
+    float *sc = out + kTailScales;
+    sc[kTailOutInv] = std::ldexp(1.f, -eo);
+    sc[kTailLn] = std::ldexp(1.f, el), sc[kTailLnInv] = std::ldexp(1.f, -el - e1);
+    sc[kTailHid] = std::ldexp(1.f, eh), sc[kTailHidInv] = std::ldexp(1.f, -eh - e2);
 }
 
 void tail128(const Tail128 &t, hipStream_t stream, bool rows16) {

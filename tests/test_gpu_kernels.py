@@ -427,6 +427,35 @@ def test_block_tail_matches_float64(device, rows, fused):
     assert np.abs(out.reshape(rows, 128) - want).max() < 2e-5
 
 
+@pytest.mark.parametrize("fused", [1, 2])
+@pytest.mark.parametrize("att_size,wo_size,ln_size,ffn_size", [(1e6, 1e-6, 1.0, 1.0), (1e-9, 1e9, 30.0, 1e-4),
+                                                               (1.0, 1.0, 1e-3, 1e3), (3.0, 1.0, 1e4, 1e-3)])
+def test_block_tail_operand_ranges(device, fused, att_size, wo_size, ln_size, ffn_size):
+    """The tail's products scale their operands: attention outputs by row
+    (rows of very different sizes here, one of zeros), weights and LayerNormed
+    and hidden values by bounds taken from the weights. Every product's error
+    stays that of FP32 sums of its own terms: 2^-19 of the sum of magnitudes
+    (256 terms' roundings, the GELU's 1.2e-7 and the operands' 2^-23)."""
+    rows = 70
+    rng = np.random.default_rng(3)
+    att = (fast_values(rows * 128, 1, att_size).reshape(rows, 128) * np.exp2(rng.integers(-8, 9, (rows, 1)))).astype(np.float32)
+    att[7] = 0.0
+    state = fast_values(rows * 128, 2, 3.0)
+    wo, bo = fast_values(128 * 128, 3, 0.09 * wo_size), fast_values(128, 4, 0.1)
+    n2w, n2b = (fast_values(128, 5, 0.2) + 1.0) * np.float32(ln_size), fast_values(128, 6, 0.1)
+    w1, b1 = fast_values(256 * 128, 7, 0.09 / ln_size), fast_values(256, 8, 0.1)
+    w2, b2 = fast_values(128 * 256, 9, 0.06 * ffn_size), fast_values(128, 10, 0.1)
+    out = np.zeros_like(state)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_block_tail(device.handle, fused, F(att), F(state), rows, F(wo), F(bo), F(n2w),
+                                            F(n2b), F(w1), F(b1), F(w2), F(b2), 1, F(out)))
+    want = block_tail64(att, state.reshape(rows, 128), wo.reshape(128, 128), bo, n2w, n2b, w1.reshape(256, 128), b1,
+                        w2.reshape(128, 256), b2)
+    first = np.abs(att.astype(np.float64)) @ np.abs(wo.reshape(128, 128)).T + np.abs(state.reshape(rows, 128)) + 1.0
+    size = first + 256 * 4.0 * 0.06 * ffn_size * np.abs(fast_values(8, 9, 1.0)).max()
+    assert (np.abs(out.reshape(rows, 128) - want) / size).max() < 2.0 ** -19
+
+
 @pytest.mark.parametrize("rows", [1, 16, 33, 1000])
 def test_block_tail_small_pass_form_equals_tail128(device, rows):
     """The 16-rows-per-workgroup tail takes every product in tail128's order:
