@@ -404,6 +404,13 @@ int irx_test_column_block(irx_device *device, int fused, const float *state, siz
                           const float *bq, const float *wo, const float *bo, const float *n2w, const float *n2b,
                           const float *w1, const float *b1, const float *w2, const float *b2, size_t repeats,
                           float *out);
+/* The ICL stage's products on FP16 pairs: out [m, n] = epilogue(x w^T + b), x
+ * [m, k] (k 512 or 1,024) or, with lnw and lnb, LN(x) (k 512), w [n, k], n a
+ * multiple of 64; epilogue 0 none, 1 GELU, 2 plus residual [m, n] (updated in
+ * place on the device). */
+int irx_test_pair_linear(irx_device *device, int epilogue, const float *x, size_t m, size_t k, const float *lnw,
+                         const float *lnb, const float *w, const float *b, size_t n, const float *residual,
+                         float *out);
 /* LayerNorm fused into a 512-wide product, x [m, 512], w [n, 512]:
  * epilogue 1 (GELU): out [m, n] = gelu(LN(x) w^T + b); epilogue 2 (QASS, the
  * ICL query path, n = 512): q = LN(x) w^T + b, then per head

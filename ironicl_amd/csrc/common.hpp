@@ -199,6 +199,37 @@ void gemm(const GemmArgs &args, hipStream_t stream);
 // m x n product with K = 128 and plain row-major output.
 bool gemm_fuses_ln(long long m, int n);
 
+// A weight matrix [n, k] packed as FP16 pairs (pair_pack, pairlinear.hip), the
+// inverse of its scale, and the scale of LayerNormed rows with the inverse of
+// that product's.
+struct PairW {
+    const float *pack = nullptr;
+    float inv = 0.f, ln_scale = 0.f, ln_inv = 0.f;
+};
+// Packs W (host copy for its largest value, device copy to read) into `out`
+// (n k floats on the device); lnw / lnb: host copies of the LayerNorm taken in
+// the product's prologue, or null. n a multiple of 16, k of 512.
+PairW pair_pack(const float *host, const float *device, int n, int k, const float *lnw, const float *lnb, float *out,
+                hipStream_t stream);
+// The exponent that brings magnitudes up to `largest` to at most 2^`top`.
+int pair_scale_exponent(double largest, int top);
+// c = epilogue(A W^T + bias), A [m, k] (k = 512 or 1,024) or LN(A) (lnw / lnb
+// [512]); n a multiple of 64. The residual may be the output.
+struct PairLinear {
+    const float *x;
+    long long ldx;
+    const float *lnw, *lnb;
+    PairW w;
+    const float *bias;
+    const float *residual;
+    long long ldr;
+    float *c;
+    OutMap out;
+    int m, n, k;
+    int epilogue;
+};
+void pair_linear(const PairLinear &a, hipStream_t stream);
+
 // Post-attention half of a 128-wide block in one kernel (cpu.rs:1555-1601):
 // s1 = state + (att Wo^T + bo); state = s1 + (gelu(LN2(s1) W1^T + b1) W2^T + b2).
 // `pack` holds Wo [128,128], W1 [256,128] and W2 [128,256] as packed by

@@ -339,12 +339,14 @@ void return_stream(irx_device *d, hipStream_t s) {
 
 struct Lin {
     const float *w = nullptr, *b = nullptr;
+    PairW pairs = {};  // 512-wide blocks and the decoder: w as FP16 pairs
 };
 
 struct BlockW {
     int dim = 0;
     const float *n1w = nullptr, *n1b = nullptr, *n2w = nullptr, *n2b = nullptr;
     const float *in_w = nullptr, *in_b = nullptr;  // [3 dim, dim], [3 dim]
+    PairW in_pairs = {};                           // 512-wide blocks: in_w as FP16 pairs
     Lin out, l1, l2;
     bool qass = false;
     Lin qm0, qm2;  // QASS query MLP, per head: hd -> 64 -> hd
@@ -359,7 +361,7 @@ struct irx_weights {
     int task = 0;
     int width = 0;
     size_t bytes = 0;
-    DevBuf arena;
+    DevBuf arena, pairs;
     const float *in_w = nullptr, *in_b = nullptr;
     const float *ind[kColumnBlocks] = {};
     BlockW col1[kColumnBlocks], col2[kColumnBlocks], row[kRowBlocks], icl[kIclBlocks];
@@ -439,10 +441,16 @@ void set_device(const irx_device *d) { IRX_HIP(hipSetDevice(d->ordinal)); }
 
 // ---- stages shared by the build and the predictor ----
 
-// Rows up to which 512-wide LayerNorms run fused into the product that reads
-// them (prediction passes); larger products (the build's N rows) keep the
-// tiled GEMMs, whose large tiles reuse the weights across rows.
+// Rows up to which the ICL query path (LN1, projection, QASS) runs as one
+// launch (prediction passes); larger ones (the build's N rows) take the
+// LayerNorm that the K/V projection shares and separate products.
 constexpr long long kLnLinearRows = 8192;
+// Rows above which the other 512-wide products run on FP16 pairs
+// (pair_linear): per 512-row pass the out-projection, FFN and decoder products
+// they replace took 12-21 us each on FP32 MFMAs; 1,024 rows against 10,000 x
+// 100 at auto went from 2.53 to 2.30 ms, the 10,000 x 100 fit from 41.2 to 39.8.
+// Smaller passes are bound by reading each weight once, not by products.
+constexpr long long kPairRows = 64;
 // States (columns x rows) from which a cached column block runs as one
 // kernel of 64-row tiles (column_block) rather than its small-pass form of
 // 16 rows per workgroup. Measured per block at 64 columns (the three
@@ -464,6 +472,16 @@ struct Stages {
         g.out = OutMap::row_major(n, ldc);
         g.m = (int)m, g.n = n, g.k = k, g.epilogue = epi;
         gemm(g, s);
+    }
+
+    // The same product of a packed matrix, for m rows (pair_rows).
+    void linear_pairs(const float *a, long long lda, long long m, int k, const PairW &wt, const float *b, int n,
+                      float *c, const OutMap &map, int epi = kEpiNone, const float *res = nullptr, long long ldr = 0,
+                      const float *lnw = nullptr, const float *lnb = nullptr) const {
+        PairLinear g{};
+        g.x = a, g.ldx = lda, g.lnw = lnw, g.lnb = lnb, g.w = wt, g.bias = b, g.residual = res, g.ldr = ldr, g.c = c;
+        g.out = map, g.m = (int)m, g.n = n, g.k = k, g.epilogue = epi;
+        pair_linear(g, s);
     }
 
     // LayerNorm of 128-wide rows x [m, 128] and the product that reads it:
@@ -519,8 +537,16 @@ struct Stages {
         const bool packed = d == 128 && bw.tail_pack;
         const bool use_fused = fused < 0 ? packed : fused >= 1;
         const bool rows16 = fused < 0 ? m < 16384 : fused == 2;
-        if (d == 512 && m <= kLnLinearRows) {
-            // Prediction-sized 512-wide blocks: LN2 fused into the FFN's first product.
+        if (d == 512 && m > kPairRows) {
+            const OutMap rows = OutMap::row_major(d, d);
+            linear_pairs(att, d, m, d, bw.out.pairs, bw.out.b, d, state, rows, kEpiResidual, state, d);
+            linear_pairs(state, d, m, d, bw.l1.pairs, bw.l1.b, 2 * d, hid, OutMap::row_major(2 * d, 2 * d), kEpiGelu,
+                         nullptr, 0, bw.n2w, bw.n2b);
+            linear_pairs(hid, 2 * d, m, 2 * d, bw.l2.pairs, bw.l2.b, d, state, rows, kEpiResidual, state, d);
+            return;
+        }
+        if (d == 512) {
+            // Small 512-wide blocks: LN2 fused into the FFN's first product.
             linear(att, d, m, d, bw.out.w, bw.out.b, d, state, d, kEpiResidual, state, d);
             LnLinear f{};
             f.x = state, f.ldx = d, f.lnw = bw.n2w, f.lnb = bw.n2b, f.w = bw.l1.w, f.b = bw.l1.b, f.out = hid;
@@ -538,12 +564,7 @@ struct Stages {
             return;
         }
         linear(att, d, m, d, bw.out.w, bw.out.b, d, state, d, kEpiResidual, state, d);
-        if (d == 128) {
-            ln_linear128(state, m, bw.n2w, bw.n2b, norm, bw.l1.w, bw.l1.b, 2 * d, hid, 2 * d, kEpiGelu);
-        } else {
-            layer_norm(state, d, bw.n2w, bw.n2b, norm, d, m, d, s);
-            linear(norm, d, m, d, bw.l1.w, bw.l1.b, 2 * d, hid, 2 * d, kEpiGelu);
-        }
+        ln_linear128(state, m, bw.n2w, bw.n2b, norm, bw.l1.w, bw.l1.b, 2 * d, hid, 2 * d, kEpiGelu);
         linear(hid, 2 * d, m, 2 * d, bw.l2.w, bw.l2.b, d, state, d, kEpiResidual, state, d);
     }
 
@@ -674,7 +695,7 @@ struct Stages {
             if (!normed) layer_norm(x, 512, bw.n1w, bw.n1b, r.norm, 512, m, 512, s);
             // Q, head-major [b, 8, rows, 64].
             OutMap qmap{64, kHeads, 0, (long long)rows * 64, rows, (long long)kHeads * rows * 64, 64};
-            linear_map(r.norm, 512, m, 512, bw.in_w, bw.in_b, 512, r.qh, qmap);
+            linear_pairs(r.norm, 512, m, 512, bw.in_pairs, bw.in_b, 512, r.qh, qmap);
             // QASSMax: q * base * (1 + tanh(MLP(q))) per head (reference.rs:417-428).
             QassRows qa{};
             qa.q = r.qh, qa.w0 = bw.qm0.w, qa.b0 = bw.qm0.b, qa.w2 = bw.qm2.w, qa.b2 = bw.qm2.b, qa.base = base;
@@ -821,7 +842,27 @@ void weights_load(irx_weights *W, irx_tensor_lookup lookup, void *user) {
     L.take("icl_predictor.y_encoder.bias", 512, &W->yicl.b);
     W->arena.alloc(L.host.size() * sizeof(float));
     IRX_HIP(hipMemcpy(W->arena.p, L.host.data(), L.host.size() * sizeof(float), hipMemcpyHostToDevice));
-    W->bytes = W->arena.bytes;
+    // The ICL blocks' and the decoder's first matrices as FP16 pairs too.
+    constexpr size_t kBlockPairs = (size_t)(3 + 1 + 2 + 2) * 512 * 512;
+    W->pairs.alloc((kIclBlocks * kBlockPairs + 1024 * 512) * sizeof(float));
+    W->bytes = W->arena.bytes + W->pairs.bytes;
+    float *next_pairs = W->pairs.f();
+    auto pack = [&](const float **slot, int n, int k, const float **lnw = nullptr, const float **lnb = nullptr) {
+        const size_t offset = L.offset_of(slot);
+        const float *h = L.host.data();
+        const PairW p = pair_pack(h + offset, W->arena.f() + offset, n, k, lnw ? h + L.offset_of(lnw) : nullptr,
+                                  lnb ? h + L.offset_of(lnb) : nullptr, next_pairs, nullptr);
+        next_pairs += (size_t)n * k;
+        return p;
+    };
+    for (BlockW &b : W->icl) {
+        b.in_pairs = pack(&b.in_w, 1536, 512);
+        b.out.pairs = pack(&b.out.w, 512, 512);
+        b.l1.pairs = pack(&b.l1.w, 1024, 512, &b.n2w, &b.n2b);
+        b.l2.pairs = pack(&b.l2.w, 512, 1024);
+    }
+    W->dec0.pairs = pack(&W->dec0.w, 1024, 512, &W->ln_w, &W->ln_b);
+    IRX_HIP(hipDeviceSynchronize());
     for (auto &pend : L.pending) {
         if (pend.slot == &freqs) continue;
         *pend.slot = W->arena.f() + pend.offset;
@@ -1173,13 +1214,22 @@ void build_impl(irx_weights *W, const irx_build_inputs *in, irx_build_outputs *o
         {
             Stages::IclBuffers ib = Stages::icl_buffers(ws, N, 1, N, N, cus, f16);
             float *kv32 = f16 ? ws.take((size_t)2 * kHeads * N * 64) : nullptr;
+            auto project_kv = [&](const BlockW &bw, const float *norm, float *out, const OutMap &map) {
+                if (N > kPairRows) {
+                    PairW kv = bw.in_pairs;
+                    kv.pack += (size_t)512 * 512;  // past the query rows' fragments
+                    st.linear_pairs(norm, 512, N, 512, kv, bw.in_b + 512, 1024, out, map);
+                } else {
+                    st.linear_map(norm, 512, N, 512, bw.in_w + 512 * 512, bw.in_b + 512, 1024, out, map);
+                }
+            };
             for (int blk = 0; blk < kIclBlocks; ++blk) {
                 const BlockW &bw = W->icl[blk];
                 layer_norm(rows, 512, bw.n1w, bw.n1b, ib.norm, 512, N, 512, s);
                 if (!f16) {
                     float *kc = cache->icl[blk].f() + (long long)e * kHeads * N * 64;
                     OutMap kvmap = OutMap::head_major(64, kHeads, N, icl_plane);
-                    st.linear_map(ib.norm, 512, N, 512, bw.in_w + 512 * 512, bw.in_b + 512, 1024, kc, kvmap);
+                    project_kv(bw, ib.norm, kc, kvmap);
                     // The last block's row states are never read: only its K/V are kept.
                     if (blk + 1 < kIclBlocks)
                         st.icl_queries(blk, rows, 1, N, kc, kc + icl_plane, N, d_base + blk * 512, ib, nullptr,
@@ -1188,7 +1238,7 @@ void build_impl(irx_weights *W, const irx_build_inputs *in, irx_build_outputs *o
                     // FP32 K/V of this estimator, then packed into its part of the FP16 cache.
                     const long long p32 = (long long)kHeads * N * 64;
                     OutMap kvmap = OutMap::head_major(64, kHeads, N, p32);
-                    st.linear_map(ib.norm, 512, N, 512, bw.in_w + 512 * 512, bw.in_b + 512, 1024, kv32, kvmap);
+                    project_kv(bw, ib.norm, kv32, kvmap);
                     unsigned short *k16 = static_cast<unsigned short *>(cache->icl[blk].p) + e * est16;
                     unsigned short *v16 = k16 + plane16;
                     pack_icl16(kv32, kv32 + p32, false, N, kHeads, k16, v16, counter, s);
@@ -1350,14 +1400,14 @@ void issue_pass(irx_predictor *P, int slot, const PassBuffers &pb, const float *
         }
     }
     // Decoder (cached_icl_decoder, cpu.rs:2543-2580) into logits [B, Q, width].
-    if ((long long)B * R <= kLnLinearRows) {
+    if ((long long)B * R > kPairRows) {
+        st.linear_pairs(rows, 512, (long long)B * R, 512, W.dec0.pairs, W.dec0.b, 1024, ib.hid,
+                        OutMap::row_major(1024, 1024), kEpiGelu, nullptr, 0, W.ln_w, W.ln_b);
+    } else {
         LnLinear f{};
         f.x = rows, f.ldx = 512, f.lnw = W.ln_w, f.lnb = W.ln_b, f.w = W.dec0.w, f.b = W.dec0.b, f.out = ib.hid;
         f.ldo = 1024, f.m = B * R, f.n = 1024;
         ln_linear512(f, kLnGelu, s);
-    } else {
-        layer_norm(rows, 512, W.ln_w, W.ln_b, ib.norm, 512, (long long)B * R, 512, s);
-        st.linear(ib.norm, 512, (long long)B * R, 512, W.dec0.w, W.dec0.b, 1024, ib.hid, 1024, kEpiGelu);
     }
     OutMap lmap{width, 1, 0, 0, R, (long long)Q * width, width};
     st.linear_map(ib.hid, 1024, (long long)B * R, 1024, W.dec2.w, W.dec2.b, width, logits, lmap);
@@ -2325,6 +2375,31 @@ int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t 
         } else {
             ln_linear512(f, epilogue, nullptr);
         }
+        IRX_HIP(hipDeviceSynchronize());
+        IRX_HIP(hipMemcpy(out, dout.p, m * n * 4, hipMemcpyDeviceToHost));
+    });
+}
+
+int irx_test_pair_linear(irx_device *device, int epilogue, const float *x, size_t m, size_t k, const float *lnw,
+                         const float *lnb, const float *w, const float *b, size_t n, const float *residual, float *out) {
+    return guarded("irx_test_pair_linear", [&] {
+        if (!device || !x || !m || !w || !b || !out || n % 64 || !n || (k != 512 && k != 1024) || !lnw != !lnb ||
+            (lnw && k != 512) || epilogue < kEpiNone || epilogue > kEpiResidual || (epilogue == kEpiResidual && !residual))
+            fail(IRX_INVALID_ARGUMENT, "pair product arguments do not match");
+        set_device(device);
+        auto up = [](const float *h, size_t count) {
+            DevBuf d(count * 4);
+            if (h) IRX_HIP(hipMemcpy(d.p, h, count * 4, hipMemcpyHostToDevice));
+            return d;
+        };
+        DevBuf dx = up(x, m * k), dw = up(w, n * k), db = up(b, n), pack(n * k * 4), dout = up(residual, m * n);
+        DevBuf dlw = up(lnw, lnw ? 512 : 1), dlb = up(lnb, lnb ? 512 : 1);
+        PairLinear g{};
+        g.x = dx.f(), g.ldx = (long long)k, g.lnw = lnw ? dlw.f() : nullptr, g.lnb = lnb ? dlb.f() : nullptr;
+        g.w = pair_pack(w, dw.f(), (int)n, (int)k, lnw, lnb, pack.f(), nullptr);
+        g.bias = db.f(), g.residual = dout.f(), g.ldr = (long long)n, g.c = dout.f();
+        g.out = OutMap::row_major((int)n, (long long)n), g.m = (int)m, g.n = (int)n, g.k = (int)k, g.epilogue = epilogue;
+        pair_linear(g, nullptr);
         IRX_HIP(hipDeviceSynchronize());
         IRX_HIP(hipMemcpy(out, dout.p, m * n * 4, hipMemcpyDeviceToHost));
     });

@@ -834,21 +834,16 @@ void pack_pair(const float *w, int ld, int r0, int c0, float scale, float *dst) 
         }
 }
 
-// The exponent that brings magnitudes up to `largest` to at most 2^`top`.
-int scale_exponent(double largest, int top) {
-    if (!(largest > 0.0)) return 0;
-    return std::max(-60, std::min(60, top - 1 - std::ilogb(largest)));
-}
 int weight_exponent(const float *w, size_t count) {
     float largest = 0.f;
     for (size_t i = 0; i < count; ++i) largest = std::max(largest, std::fabs(w[i]));
-    return scale_exponent(largest, 14);
+    return pair_scale_exponent(largest, 14);
 }
 // The bound of a LayerNormed row's values: at most sqrt(128) of deviation.
 int ln_exponent(const float *w, const float *b) {
     float lw = 0.f, lb = 0.f;
     for (int i = 0; i < 128; ++i) lw = std::max(lw, std::fabs(w[i])), lb = std::max(lb, std::fabs(b[i]));
-    return scale_exponent(11.5 * lw + lb, 15);
+    return pair_scale_exponent(11.5 * lw + lb, 15);
 }
 
 }  // namespace
@@ -898,7 +893,7 @@ void tail128_pack(const float *wo, const float *n2w, const float *n2b, const flo
         hidden = std::max(hidden, 11.5 * std::sqrt(norm) + std::fabs(bias));
     }
     const int eo = weight_exponent(wo, 128 * 128), e1 = weight_exponent(w1, 256 * 128);
-    const int e2 = weight_exponent(w2, 128 * 256), el = ln_exponent(n2w, n2b), eh = scale_exponent(hidden, 15);
+    const int e2 = weight_exponent(w2, 128 * 256), el = ln_exponent(n2w, n2b), eh = pair_scale_exponent(hidden, 15);
     const float so = std::ldexp(1.f, eo), s1 = std::ldexp(1.f, e1), s2 = std::ldexp(1.f, e2);
     for (int kb = 0; kb < 4; ++kb)
         for (int ob = 0; ob < 8; ++ob) pack_pair(wo, 128, 16 * ob, 32 * kb, so, out + (kb * 8 + ob) * 512);

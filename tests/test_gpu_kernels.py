@@ -584,6 +584,40 @@ def test_ln_linear_gelu_matches_float64(device, m, n):
     np.testing.assert_allclose(out.reshape(m, n), want, rtol=1e-4, atol=2e-5)
 
 
+@pytest.mark.parametrize("m", [1, 65, 512, 1000, 9001])
+@pytest.mark.parametrize("epilogue,k,n,norm", [(0, 512, 64, False), (0, 512, 1024, False), (1, 512, 1024, True),
+                                               (2, 512, 512, False), (2, 1024, 512, False), (1, 1024, 64, False)])
+def test_pair_linear_matches_float64(device, m, epilogue, k, n, norm):
+    """The ICL products on FP16 pairs, at 16 and 32 rows per workgroup, rows of
+    sizes from 2^-20 to 2^20 where they are not LayerNormed (one of zeros) and
+    weights of 1e-3: every output within 2^-20 of the sum of its terms'
+    magnitudes (operands to 2^-23 each, sums of at most 32 steps), plus the
+    GELU's 1.2e-7 (1 + |x|)."""
+    rng = np.random.default_rng(m + k + n)
+    x = fast_values(m * k, 1, 2.0).reshape(m, k)
+    if not norm:
+        x *= np.exp2(rng.integers(-20, 21, (m, 1))).astype(np.float32)
+        x[m // 2] = 0.0
+    lnw, lnb = fast_values(512, 2, 0.2) + 1.0, fast_values(512, 3, 0.1)
+    w, b = fast_values(n * k, 4, 1e-3), fast_values(n, 5, 0.1)
+    res = fast_values(m * n, 6, 1.0)
+    out = np.zeros(m * n, np.float32)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_pair_linear(device.handle, epilogue, F(x), m, k, F(lnw) if norm else None,
+                                             F(lnb) if norm else None, F(w), F(b), n,
+                                             F(res) if epilogue == 2 else None, F(out)))
+    rows = sorted(set(rng.integers(0, m, 64)) | {0, m // 2, m - 1})
+    a = ln64(x[rows], lnw, lnb) if norm else x[rows].astype(np.float64)
+    wt = w.reshape(n, k).T.astype(np.float64)
+    want, size = a @ wt + b, np.abs(a) @ np.abs(wt) + np.abs(b)
+    if epilogue == 1:
+        size = size + 0.25 * (1.0 + np.abs(want))
+        want = gelu64(want)
+    if epilogue == 2:
+        want, size = want + res.reshape(m, n)[rows], size + np.abs(res.reshape(m, n)[rows])
+    assert (np.abs(out.reshape(m, n)[rows] - want) / size).max() < 2.0 ** -20
+
+
 @pytest.mark.parametrize("form,estimators,rows", [(2, 1, 1), (2, 1, 2), (2, 1, 5), (2, 8, 1), (2, 4, 2), (2, 3, 3),
                                                   (2, 1, 16), (2, 2, 8), (2, 3, 5), (2, 1, 32), (2, 4, 8), (2, 3, 11),
                                                   (2, 2, 250), (2, 3, 17), (3, 1, 1), (3, 3, 5), (3, 2, 250),
