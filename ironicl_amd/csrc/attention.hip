@@ -262,6 +262,37 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
     const int half = lane >> 5, r32 = lane & 31;
     const int qrow0 = qt * kIclQueries + qgroup * 64 + r32;
 
+    const float *kbase = p.k + pair * p.kv_pair_stride;
+    const float *vbase = p.v + pair * p.kv_pair_stride;
+    // Staging: thread t holds key t / 8's dims 8 (t % 8) .. +7 and dim `lane`
+    // of the eight keys at stored chunk `wave`. The loads go through buffer
+    // descriptors that end with the range: keys past it read as zeros (their
+    // scores are masked), and the addresses take no VALU work.
+    const int s_key = tid >> 3, s_chunk = tid & 7;
+    float kr[8], vr[8];
+    auto rsrc = [&](const float *base, int k0) {
+        const float *tile = base + (long long)k0 * 64;
+        const long long bytes = min((long long)(k_end - k0) * 256, 0x7fffffffLL);
+        return __builtin_amdgcn_make_buffer_rsrc((void *)tile, 0, (int)bytes, 0x00020000);
+    };
+    const int k_off = tid * 32, v_off = (16 * (wave >> 1) + 4 * (wave & 1)) * 256 + lane * 4;
+    auto load_k = [&](int k0) {
+        const auto r = rsrc(kbase, k0);
+        const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, k_off, 0, 0);
+        const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(r, k_off + 16, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kr[e] = __uint_as_float(a[e]), kr[4 + e] = __uint_as_float(b[e]);
+    };
+    auto load_v = [&](int k0) {
+        const auto r = rsrc(vbase, k0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            vr[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, v_off + ((i & 3) + 8 * (i >> 2)) * 256, 0, 0));
+    };
+    // The first tile's loads cross the queries' latency.
+    load_k(k_begin), load_v(k_begin);
+    __builtin_amdgcn_sched_barrier(0);
+
     // The lane's queries (row qrow0 + 32 j), dims 16 m + 8 half .. +7, as
     // scaled pairs; coef[j] takes a product of scaled queries and unscaled
     // keys to the exp2 domain.
@@ -302,33 +333,6 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
         }
     }
 
-    const float *kbase = p.k + pair * p.kv_pair_stride;
-    const float *vbase = p.v + pair * p.kv_pair_stride;
-    // Staging: thread t holds key t / 8's dims 8 (t % 8) .. +7 and dim `lane`
-    // of the eight keys at stored chunk `wave`. The loads go through buffer
-    // descriptors that end with the range: keys past it read as zeros (their
-    // scores are masked), and the addresses take no VALU work.
-    const int s_key = tid >> 3, s_chunk = tid & 7;
-    float kr[8], vr[8];
-    auto rsrc = [&](const float *base, int k0) {
-        const float *tile = base + (long long)k0 * 64;
-        const long long bytes = min((long long)(k_end - k0) * 256, 0x7fffffffLL);
-        return __builtin_amdgcn_make_buffer_rsrc((void *)tile, 0, (int)bytes, 0x00020000);
-    };
-    const int k_off = tid * 32, v_off = (16 * (wave >> 1) + 4 * (wave & 1)) * 256 + lane * 4;
-    auto load_k = [&](int k0) {
-        const auto r = rsrc(kbase, k0);
-        const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, k_off, 0, 0);
-        const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(r, k_off + 16, 0, 0);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) kr[e] = __uint_as_float(a[e]), kr[4 + e] = __uint_as_float(b[e]);
-    };
-    auto load_v = [&](int k0) {
-        const auto r = rsrc(vbase, k0);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            vr[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, v_off + ((i & 3) + 8 * (i >> 2)) * 256, 0, 0));
-    };
     bool special = false;
     q_largest = wave_magnitude(q_largest);
     if (lane == 0) lds.largest[wave] = q_largest;
@@ -531,7 +535,6 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
     // Tiles past the last repeat it; what is made of them is never used.
     const int k_last = k_begin + (tiles - 1) * kKeyTile;
     auto tile_at = [&](int u) { return min(k_begin + u * kKeyTile, k_last); };
-    load_k(k_begin), load_v(k_begin);
     update_scales();
     convert_k(0), convert_v(0, 0);
     load_k(tile_at(1)), load_v(tile_at(1));
@@ -1657,6 +1660,22 @@ IclLaunch plan_icl(int pairs, int q_rows, int kv_rows, int compute_units, bool f
     if (base < slots) {
         // Few queries: split the keys until one round of workgroups fills the chip.
         splits = std::min((int)ceil_div(slots, base), max_splits);
+        if (!f16) {
+            // FP32: as many ranges as pay for their merge. Microseconds, as
+            // measured: about 10 for a workgroup's start and end, 2.5 a 64-key
+            // tile, and for the merge 4 and its traffic (each partial row
+            // written and read, 520 bytes, at 4 TB/s). 33 queries x 1,024 keys x
+            // 16 pairs in 8 ranges 15.8 us (in 2: 28.1), 512 x 1,024 x 8 in 8 23.9
+            // (in 2: 33.9); 2,000 x 700 x 24 (192 units) unsplit 46 (in 2: 63).
+            const int tiles = (int)ceil_div(kv_rows, kKeyTile);
+            double best = 1e30;
+            for (int s = 1; s <= std::min((int)ceil_div(slots, base), std::max(1, tiles / 2)); ++s) {
+                const double rounds = (double)ceil_div(base * s, slots);
+                const double merge = s > 1 ? 4.0 + base * s * (kIclQueries * 520.0 / 4e6) : 0.0;
+                const double cost = rounds * (10.0 + 2.5 * (double)ceil_div(tiles, s)) + merge;
+                if (cost < best) best = cost, splits = s;
+            }
+        }
     } else {
         // Many: take the split count (up to 8) whose last round of workgroups is
         // fullest, preferring fewer splits unless more are clearly better.
@@ -1701,7 +1720,7 @@ IclPlan plan_icl_fp32(int pairs, int q_rows, int kv_rows, int compute_units) {
         IclLaunch &t = pl.tail;
         t = m;
         // At most 16 splits: the rows merge kernel's limit.
-        const long long max_splits = std::min(16, std::max(1, kv_rows / 512));
+        const long long max_splits = std::min(16, std::max(1, kv_rows / 128));
         const int want = (int)std::max<long long>(1, std::min(slots / rest, max_splits));
         t.keys_per_split = (int)ceil_div(ceil_div(kv_rows, want), kKeyTile) * kKeyTile;
         t.splits = (int)ceil_div(kv_rows, t.keys_per_split);
