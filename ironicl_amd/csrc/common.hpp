@@ -339,6 +339,9 @@ struct LnLinear {
     const float *qm0w, *qm0b, *qm2w, *qm2b;  // kLnQass: [64, 64], [64] each
     const float *base;                       // kLnQass: [8, 64]
     int rows;                                // kLnQass: rows per estimator
+    // kLnQass, more than 32 rows: w as FP16 pairs with its LayerNorm scale
+    // (pack null: FP32 products).
+    PairW pairs;
 };
 void ln_linear512(const LnLinear &a, int epilogue, hipStream_t stream);
 

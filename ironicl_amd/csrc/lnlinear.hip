@@ -19,7 +19,10 @@
 // transposed (D = W x^T: lane (m, g) = (lane % 16, lane / 16) holds row m's
 // columns 16 b + 4 g + r in register r of block b). Each wave loads its rows'
 // quarter of x in that layout, the row statistics are summed over the four
-// waves through LDS, and the partial products are summed there too.
+// waves through LDS, and the partial products are summed there too. The query
+// projection of passes of more than 32 rows multiplies FP16 pairs (PAIRS,
+// common.hpp; pair_pack's fragments have x's layout as their slots): 48 products
+// of 16 cycles a wave instead of 128 of 32.
 #include "common.hpp"
 
 #include <algorithm>
@@ -49,10 +52,11 @@ __device__ __forceinline__ auto tree_sum(F a) {
 // W: waves, each taking 512 / W of K (8 for the QASS form of passes of at
 // most 32 rows: half the products and weight loads per wave; waves 4-7 then
 // only pass the barriers of the epilogue).
-template <int EPI, int OB = 4, int W = 4>
+template <int EPI, int OB = 4, int W = 4, bool PAIRS = false>
 __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
     static_assert(OB == 4 || (OB == 2 && EPI == kLnGelu), "QASS needs a whole 64-wide head per workgroup");
     static_assert(W == 4 || W == 8, "four or eight waves");
+    static_assert(!PAIRS || (OB == 4 && W == 4), "pairs: the 16 x 64 form");
     constexpr int KB = 32 / W;  // 16-wide k-blocks per wave
     __shared__ float red[2][W][kRows];
     __shared__ __attribute__((aligned(16))) float part[W][kRows][68];
@@ -68,15 +72,27 @@ __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
     // x[row][k0 + 16 kb + 4 g + e], and every weight fragment of this wave's
     // quarter up front (columns col0 + 16 ob + lane % 16): the loads' latency
     // is paid once, under the LayerNorm.
-    f32x4 x[KB], wf[KB][OB];
+    f32x4 x[KB], wf[PAIRS ? 1 : KB][OB];
+    u32x4 wp[PAIRS ? KB / 2 : 1][OB][2];  // hi, lo of 32-deep step kb
     const float *xr = p.x + r * p.ldx + k0 + 4 * g;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) x[kb] = *reinterpret_cast<const f32x4 *>(xr + 16 * kb);
-    const float *wr = p.w + (long long)(col0 + m16) * 512 + k0 + 4 * g;
+    if constexpr (PAIRS) {
+        const float *pk = p.pairs.pack + ((size_t)(col0 / 16) * 16 + (KB / 2) * w) * 512 + lane * 4;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
+        for (int kb = 0; kb < KB / 2; ++kb)
 #pragma unroll
-        for (int ob = 0; ob < OB; ++ob) wf[kb][ob] = *reinterpret_cast<const f32x4 *>(wr + ob * 16 * 512 + 16 * kb);
+            for (int ob = 0; ob < OB; ++ob)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    wp[kb][ob][h] = *reinterpret_cast<const u32x4 *>(pk + ((size_t)ob * 16 + kb) * 512 + h * 256);
+    } else {
+        const float *wr = p.w + (long long)(col0 + m16) * 512 + k0 + 4 * g;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int ob = 0; ob < OB; ++ob) wf[kb][ob] = *reinterpret_cast<const f32x4 *>(wr + ob * 16 * 512 + 16 * kb);
+    }
     float s = 0.f;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) s += (x[kb][0] + x[kb][1]) + (x[kb][2] + x[kb][3]);
@@ -111,12 +127,31 @@ __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
     f32x4 acc[OB];
 #pragma unroll
     for (int ob = 0; ob < OB; ++ob) acc[ob] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (PAIRS) {
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
+        for (int kb = 0; kb < KB / 2; ++kb) {
+            float y[8];
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+            for (int e = 0; e < 8; ++e) y[e] = x[2 * kb + (e >> 2)][e & 3] * p.pairs.ln_scale;
+            half8 xh, xl;
+            pair8(y, xh, xl);
 #pragma unroll
-            for (int ob = 0; ob < OB; ++ob) acc[ob] = mfma(wf[kb][ob][e], x[kb][e], acc[ob]);
+            for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][1]), xh, acc[ob], 0, 0, 0);
+#pragma unroll
+            for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][0]), xl, acc[ob], 0, 0, 0);
+#pragma unroll
+            for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][0]), xh, acc[ob], 0, 0, 0);
+        }
+#pragma unroll
+        for (int ob = 0; ob < OB; ++ob) acc[ob] *= p.pairs.ln_inv;
+    } else {
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int ob = 0; ob < OB; ++ob) acc[ob] = mfma(wf[kb][ob][e], x[kb][e], acc[ob]);
+    }
 #pragma unroll
     for (int ob = 0; ob < OB; ++ob)
         *reinterpret_cast<f32x4 *>(&part[w][m16][16 * ob + 4 * g]) = acc[ob];
@@ -419,6 +454,9 @@ void ln_linear512(const LnLinear &a, int epilogue, hipStream_t stream) {
             launch_rows<kLnGelu>(a, stream);
     } else if (epilogue == kLnQass && a.m <= 32) {
         hipLaunchKernelGGL((ln_linear512_kernel<kLnQass, 4, 8>), grid, dim3(512), 0, stream, a);
+    } else if (epilogue == kLnQass && a.pairs.pack) {
+        if (reinterpret_cast<uintptr_t>(a.pairs.pack) & 15) fail(3, "ln_linear512: pairs must be 16-byte aligned");
+        hipLaunchKernelGGL((ln_linear512_kernel<kLnQass, 4, 4, true>), grid, dim3(256), 0, stream, a);
     } else if (epilogue == kLnQass) {
         hipLaunchKernelGGL(ln_linear512_kernel<kLnQass>, grid, dim3(256), 0, stream, a);
     } else if (a.m <= 32) {

@@ -689,7 +689,7 @@ struct Stages {
             LnLinear f{};
             f.x = x, f.ldx = 512, f.lnw = bw.n1w, f.lnb = bw.n1b, f.w = bw.in_w, f.b = bw.in_b, f.out = r.qg;
             f.m = (int)m, f.n = 512, f.qm0w = bw.qm0.w, f.qm0b = bw.qm0.b, f.qm2w = bw.qm2.w, f.qm2b = bw.qm2.b;
-            f.base = base, f.rows = rows;
+            f.base = base, f.rows = rows, f.pairs = bw.in_pairs;
             ln_linear512(f, kLnQass, s);
         } else {
             if (!normed) layer_norm(x, 512, bw.n1w, bw.n1b, r.norm, 512, m, 512, s);
@@ -856,7 +856,7 @@ void weights_load(irx_weights *W, irx_tensor_lookup lookup, void *user) {
         return p;
     };
     for (BlockW &b : W->icl) {
-        b.in_pairs = pack(&b.in_w, 1536, 512);
+        b.in_pairs = pack(&b.in_w, 1536, 512, &b.n1w, &b.n1b);
         b.out.pairs = pack(&b.out.w, 512, 512);
         b.l1.pairs = pack(&b.l1.w, 1024, 512, &b.n2w, &b.n2b);
         b.l2.pairs = pack(&b.l2.w, 512, 1024);
@@ -2339,7 +2339,7 @@ int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t 
                        const float *lnb, const float *w, const float *b, size_t n, const float *qm0w,
                        const float *qm0b, const float *qm2w, const float *qm2b, const float *base, float *out) {
     return guarded("irx_test_ln_linear", [&] {
-        const bool tiled = epilogue == 3, qass = epilogue == kLnQass || tiled;
+        const bool tiled = epilogue == 3, pairs = epilogue == 4, qass = epilogue == kLnQass || tiled || pairs;
         if (!device || !x || !m || !lnw || !lnb || !w || !b || !out || (epilogue != kLnGelu && !qass) ||
             (qass && (n != 512 || !rows || m % rows || !qm0w || !qm0b || !qm2w || !qm2b || !base)) || !n || n % 64)
             fail(IRX_INVALID_ARGUMENT, "LN-linear arguments do not match");
@@ -2357,6 +2357,8 @@ int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t 
         f.x = dx.f(), f.ldx = 512, f.lnw = dlw.f(), f.lnb = dlb.f(), f.w = dw.f(), f.b = db.f(), f.out = dout.f();
         f.ldo = (long long)n, f.m = (int)m, f.n = (int)n;
         if (qass) f.qm0w = d0w.f(), f.qm0b = d0b.f(), f.qm2w = d2w.f(), f.qm2b = d2b.f(), f.base = dbase.f(), f.rows = (int)rows;
+        DevBuf pack(pairs ? n * 512 * 4 : 0);
+        if (pairs) f.pairs = pair_pack(w, dw.f(), (int)n, 512, lnw, lnb, pack.f(), nullptr);
         if (tiled) {
             // The build's form (Stages::icl_queries with more rows than the fused form takes).
             DevBuf dnorm(m * 512 * 4), dq(m * 512 * 4);
@@ -2373,7 +2375,7 @@ int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t 
             qass_rows(qa, nullptr);
             IRX_HIP(hipDeviceSynchronize());
         } else {
-            ln_linear512(f, epilogue, nullptr);
+            ln_linear512(f, pairs ? kLnQass : epilogue, nullptr);
         }
         IRX_HIP(hipDeviceSynchronize());
         IRX_HIP(hipMemcpy(out, dout.p, m * n * 4, hipMemcpyDeviceToHost));

@@ -621,7 +621,7 @@ def test_pair_linear_matches_float64(device, m, epilogue, k, n, norm):
 @pytest.mark.parametrize("form,estimators,rows", [(2, 1, 1), (2, 1, 2), (2, 1, 5), (2, 8, 1), (2, 4, 2), (2, 3, 3),
                                                   (2, 1, 16), (2, 2, 8), (2, 3, 5), (2, 1, 32), (2, 4, 8), (2, 3, 11),
                                                   (2, 2, 250), (2, 3, 17), (3, 1, 1), (3, 3, 5), (3, 2, 250),
-                                                  (3, 1, 2049), (3, 3, 1001)])
+                                                  (3, 1, 2049), (3, 3, 1001), (4, 1, 33), (4, 3, 17), (4, 2, 250)])
 def test_ln_linear_qass_matches_float64(device, form, estimators, rows):
     """LN1 + Q projection + QASSMax (query MLP and gate per head), head-major:
     form 2 the prediction's fused kernel, form 3 the build's (LayerNorm, tiled
