@@ -1654,7 +1654,7 @@ IclLaunch plan_icl(int pairs, int q_rows, int kv_rows, int compute_units, bool f
     g.qtiles = (int)ceil_div(q_rows, kIclQueries);
     g.q_padded = g.qtiles * kIclQueries;
     const long long base = (long long)g.qtiles * pairs;
-    const long long slots = compute_units;  // one workgroup per CU (its waves use up to 512 registers)
+    const long long slots = compute_units;  // one workgroup per CU (two 250-register waves a SIMD)
     const int max_splits = std::max(1, kv_rows / 512);
     int splits = 1;
     if (base < slots) {

@@ -1,7 +1,11 @@
 // FP32 products on gfx950 matrix cores: C = epilogue(A W^T + bias).
 //
-// Every dense layer of the model (the role of linear64 / linear_reduce in the
-// reference's CUDA backend, src/kernels/cuda/kernels.rs:290-470) runs here.
+// The dense layers of the model (the role of linear64 / linear_reduce in the
+// reference's CUDA backend, src/kernels/cuda/kernels.rs:290-470) that no fused
+// kernel takes (tail.hip, lnlinear.hip) and that do not run on FP16 pairs
+// (pairlinear.hip: the ICL stage's above 64 rows): the 128-wide products of
+// small passes, the inducing points' keys and values, small ICL products, the
+// decoder's last layer.
 // A is [M, K] activations, W is [N, K] in PyTorch Linear layout, so both
 // operands are K-contiguous.
 //

@@ -3,10 +3,10 @@
 // FFN's hidden layer, normalized rows) or 512-wide rows LayerNormed in the
 // prologue (the FFN's first product, the decoder's).
 //
-// A workgroup of four waves takes 16 RG rows x 64 columns. Its waves first load
+// A workgroup of four waves takes 16 RG rows x 64 CB columns. Its waves first load
 // the rows (a wave per 4 RG rows, every load in flight at once), LayerNorm
 // them or find each row's scale, and leave them in LDS as pairs in operand
-// order; then wave w runs columns 16 w .. + 15 over the whole depth on
+// order; then wave w runs its CB blocks of 16 columns over the whole depth on
 // v_mfma_f32_16x16x32_f16, the weights as the A operand, straight from their
 // packed fragments in L2 four steps ahead. In the result, lane (m, g) =
 // (lane % 16, lane / 16) holds row m's columns 4 g .. 4 g + 3, one 16-byte store.
@@ -31,7 +31,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kAhead = 4;  // weight fragments in flight, in 32-deep steps
 
-template <int K, int RG, int EPI, bool LN>
+template <int K, int RG, int CB, int EPI, bool LN>
 __global__ __launch_bounds__(256) void pair_linear_kernel(PairLinear p, int col_groups, int per_xcd, int count) {
     constexpr int ROWS = 16 * RG, STRIDE = K / 2 + 4;  // words per LDS row: K halves and 16 bytes of padding
     constexpr int S = K / 512, STEPS = K / 32;
@@ -45,7 +45,7 @@ __global__ __launch_bounds__(256) void pair_linear_kernel(PairLinear p, int col_
     const int m16 = lane & 15, g = lane >> 4;
 
     // This wave's weight fragments, the first steps' in flight over the prologue.
-    const float *pk = p.w.pack + (size_t)(cg * 4 + w) * STEPS * 512 + lane * 4;
+    const float *pk = p.w.pack + (size_t)(cg * 4 + w) * CB * STEPS * 512 + lane * 4;
     u32x4 wh[kAhead], wl[kAhead];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
@@ -122,51 +122,54 @@ __global__ __launch_bounds__(256) void pair_linear_kernel(PairLinear p, int col_
     }
     __syncthreads();
 
-    f32x4 big[RG], small[RG];
+#pragma unroll 1
+    for (int cb = 0; cb < CB; ++cb, pk += STEPS * 512) {
+        f32x4 big[RG], small[RG];
 #pragma unroll
-    for (int r = 0; r < RG; ++r) big[r] = small[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int r = 0; r < RG; ++r) big[r] = small[r] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int kb = 0; kb < STEPS; ++kb) {
-        const half8 ah = as_half8(wh[kb % kAhead]), al = as_half8(wl[kb % kAhead]);
-        half8 bh[RG], bl[RG];
+        for (int kb = 0; kb < STEPS; ++kb) {
+            const half8 ah = as_half8(wh[kb % kAhead]), al = as_half8(wl[kb % kAhead]);
+            half8 bh[RG], bl[RG];
 #pragma unroll
-        for (int r = 0; r < RG; ++r) {
-            const int at = (16 * r + m16) * STRIDE + (kb * 4 + g) * 4;
-            bh[r] = *reinterpret_cast<const half8 *>(&hi[at]);
-            bl[r] = *reinterpret_cast<const half8 *>(&lo[at]);
+            for (int r = 0; r < RG; ++r) {
+                const int at = (16 * r + m16) * STRIDE + (kb * 4 + g) * 4;
+                bh[r] = *reinterpret_cast<const half8 *>(&hi[at]);
+                bl[r] = *reinterpret_cast<const half8 *>(&lo[at]);
+            }
+#pragma unroll
+            for (int r = 0; r < RG; ++r) {
+                small[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[r], small[r], 0, 0, 0);
+                big[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[r], big[r], 0, 0, 0);
+                small[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[r], small[r], 0, 0, 0);
+            }
+            if (kb + kAhead < STEPS || cb + 1 < CB) {
+                wh[kb % kAhead] = *reinterpret_cast<const u32x4 *>(pk + (kb + kAhead) * 512);
+                wl[kb % kAhead] = *reinterpret_cast<const u32x4 *>(pk + (kb + kAhead) * 512 + 256);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // keeps each load this far ahead of its use
         }
-#pragma unroll
-        for (int r = 0; r < RG; ++r) {
-            small[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[r], small[r], 0, 0, 0);
-            big[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh[r], big[r], 0, 0, 0);
-            small[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl[r], small[r], 0, 0, 0);
-        }
-        if (kb + kAhead < STEPS) {
-            wh[kb % kAhead] = *reinterpret_cast<const u32x4 *>(pk + (kb + kAhead) * 512);
-            wl[kb % kAhead] = *reinterpret_cast<const u32x4 *>(pk + (kb + kAhead) * 512 + 256);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // keeps each load this far ahead of its use
-    }
 
-    const int col = 64 * cg + 16 * w + 4 * g;
-    const f32x4 bias = *reinterpret_cast<const f32x4 *>(p.bias + col);
-    const OutMap &o = p.out;
-    const int seg = col / o.col_seg, plane = seg / o.heads, head = seg - plane * o.heads;
-    const long long coff = plane * o.plane_stride + head * o.head_stride + (col - seg * o.col_seg);
+        const int col = 64 * CB * cg + 16 * (CB * w + cb) + 4 * g;
+        const f32x4 bias = *reinterpret_cast<const f32x4 *>(p.bias + col);
+        const OutMap &o = p.out;
+        const int seg = col / o.col_seg, plane = seg / o.heads, head = seg - plane * o.heads;
+        const long long coff = plane * o.plane_stride + head * o.head_stride + (col - seg * o.col_seg);
 #pragma unroll
-    for (int r = 0; r < RG; ++r) {
-        const long long row = row0 + 16 * r + m16;
-        if (row >= p.m) continue;
-        const float inv = LN ? p.w.ln_inv : p.w.inv * row_inv[16 * r + m16];
-        f32x4 v;
+        for (int r = 0; r < RG; ++r) {
+            const long long row = row0 + 16 * r + m16;
+            if (row >= p.m) continue;
+            const float inv = LN ? p.w.ln_inv : p.w.inv * row_inv[16 * r + m16];
+            f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = fmaf(big[r][e] + small[r][e], inv, bias[e]);
-            if constexpr (EPI == kEpiGelu) v[e] = gelu_erf(v[e]);
+            for (int e = 0; e < 4; ++e) {
+                v[e] = fmaf(big[r][e] + small[r][e], inv, bias[e]);
+                if constexpr (EPI == kEpiGelu) v[e] = gelu_erf(v[e]);
+            }
+            if constexpr (EPI == kEpiResidual) v += *reinterpret_cast<const f32x4 *>(p.residual + row * p.ldr + col);
+            const long long grp = row / o.rows_per_group;
+            *reinterpret_cast<f32x4 *>(p.c + grp * o.group_stride + (row - grp * o.rows_per_group) * o.ldc + coff) = v;
         }
-        if constexpr (EPI == kEpiResidual) v += *reinterpret_cast<const f32x4 *>(p.residual + row * p.ldr + col);
-        const long long grp = row / o.rows_per_group;
-        *reinterpret_cast<f32x4 *>(p.c + grp * o.group_stride + (row - grp * o.rows_per_group) * o.ldc + coff) = v;
     }
 }
 
@@ -236,34 +239,41 @@ void pair_linear(const PairLinear &a, hipStream_t stream) {
     KernelTimer timer(kFamGemm, stream, 2.0 * m * n * k,
                       4.0 * (m * k + n * k + m * n + (a.epilogue == kEpiResidual ? m * n : 0.0)));
     // 32 rows a workgroup once that fills the chip (half the weight reads of
-    // 16); at depth 1,024 the rows' pairs take the LDS of 16.
-    const int cgs = a.n / 64;
-    const int rg = a.k == 512 && (long long)ceil_div(a.m, 32) * cgs >= 256 ? 2 : 1;
-    const long long count = (long long)ceil_div(a.m, 16 * rg) * cgs, per_xcd = (count + 7) / 8;
+    // 16; at depth 1,024 the rows' pairs take the LDS of 16), and 256 columns
+    // rather than 64 once that leaves two workgroups a CU: the prologue, several
+    // times a 64-column product's time, is then paid by a fourth of them.
+    const int rg = a.k == 512 && (long long)ceil_div(a.m, 32) * (a.n / 64) >= 256 ? 2 : 1;
+    const long long groups = ceil_div(a.m, 16 * rg);
+    const bool wide = a.n % 256 == 0 && groups * (a.n / 256) >= 512;
+    const int cgs = a.n / (wide ? 256 : 64);
+    const long long count = groups * cgs, per_xcd = (count + 7) / 8;
     if (per_xcd * 8 > 0x7fffffffLL) fail(3, "pair_linear: too many rows");
-    auto go = [&]<int K, int RG, int EPI, bool LN>() {
-        hipLaunchKernelGGL((pair_linear_kernel<K, RG, EPI, LN>), dim3((unsigned)(per_xcd * 8)), dim3(256), 0, stream, a,
-                           cgs, (int)per_xcd, (int)count);
+    auto go = [&]<int K, int RG, int CB, bool LN>() {
+        const dim3 grid((unsigned)(per_xcd * 8)), block(256);
+        if (a.epilogue == kEpiNone)
+            hipLaunchKernelGGL((pair_linear_kernel<K, RG, CB, kEpiNone, LN>), grid, block, 0, stream, a, cgs, (int)per_xcd, (int)count);
+        else if (a.epilogue == kEpiGelu)
+            hipLaunchKernelGGL((pair_linear_kernel<K, RG, CB, kEpiGelu, LN>), grid, block, 0, stream, a, cgs, (int)per_xcd, (int)count);
+        else
+            hipLaunchKernelGGL((pair_linear_kernel<K, RG, CB, kEpiResidual, LN>), grid, block, 0, stream, a, cgs, (int)per_xcd, (int)count);
         IRX_HIP(hipGetLastError());
     };
-    auto epilogue = [&]<int K, int RG, bool LN>() {
-        if (a.epilogue == kEpiNone)
-            go.template operator()<K, RG, kEpiNone, LN>();
-        else if (a.epilogue == kEpiGelu)
-            go.template operator()<K, RG, kEpiGelu, LN>();
+    auto width = [&]<int K, int RG, bool LN>() {
+        if (wide)
+            go.template operator()<K, RG, 4, LN>();
         else
-            go.template operator()<K, RG, kEpiResidual, LN>();
+            go.template operator()<K, RG, 1, LN>();
     };
     if (a.k == 1024)
-        epilogue.template operator()<1024, 1, false>();
+        width.template operator()<1024, 1, false>();
     else if (ln && rg == 2)
-        epilogue.template operator()<512, 2, true>();
+        width.template operator()<512, 2, true>();
     else if (ln)
-        epilogue.template operator()<512, 1, true>();
+        width.template operator()<512, 1, true>();
     else if (rg == 2)
-        epilogue.template operator()<512, 2, false>();
+        width.template operator()<512, 2, false>();
     else
-        epilogue.template operator()<512, 1, false>();
+        width.template operator()<512, 1, false>();
 }
 
 }  // namespace irx
