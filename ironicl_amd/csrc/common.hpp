@@ -199,18 +199,17 @@ void gemm(const GemmArgs &args, hipStream_t stream);
 // m x n product with K = 128 and plain row-major output.
 bool gemm_fuses_ln(long long m, int n);
 
-// A weight matrix [n, k] packed as FP16 pairs (pair_pack, pairlinear.hip), the
-// inverse of its scale, and the scale of LayerNormed rows with the inverse of
-// that product's.
+// A weight matrix [n, k] packed as FP16 pairs (pair_pack, pairlinear.hip), each
+// row's inverse scale [n], and the scale of LayerNormed rows and its inverse.
 struct PairW {
-    const float *pack = nullptr;
-    float inv = 0.f, ln_scale = 0.f, ln_inv = 0.f;
+    const float *pack = nullptr, *row_inv = nullptr;
+    float ln_scale = 0.f, ln_inv = 0.f;
 };
-// Packs W (host copy for its largest value, device copy to read) into `out`
-// (n k floats on the device); lnw / lnb: host copies of the LayerNorm taken in
-// the product's prologue, or null. n a multiple of 16, k of 512.
-PairW pair_pack(const float *host, const float *device, int n, int k, const float *lnw, const float *lnb, float *out,
-                hipStream_t stream);
+constexpr size_t pair_pack_floats(int n, int k) { return (size_t)n * k + n; }
+// Packs W [n, k] (device) into `out` (pair_pack_floats on the device); lnw /
+// lnb: host copies of the LayerNorm taken in the product's prologue, or null.
+// n a multiple of 16, k of 512.
+PairW pair_pack(const float *w, int n, int k, const float *lnw, const float *lnb, float *out, hipStream_t stream);
 // The exponent that brings magnitudes up to `largest` to at most 2^`top`.
 int pair_scale_exponent(double largest, int top);
 // c = epilogue(A W^T + bias), A [m, k] (k = 512 or 1,024) or LN(A) (lnw / lnb
@@ -235,7 +234,7 @@ void pair_linear(const PairLinear &a, hipStream_t stream);
 // `pack` holds Wo [128,128], W1 [256,128] and W2 [128,256] as packed by
 // tail128_pack (host code, kTail128PackFloats floats): FP16 pairs, then
 // kPackScales words of scales.
-constexpr size_t kPackScales = 64;
+constexpr size_t kPackScales = 576;
 constexpr size_t kTail128PackFloats = 10 * 8192 + kPackScales;
 struct Tail128 {
     const float *att;  // [m, 128], row stride lda

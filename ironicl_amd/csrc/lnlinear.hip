@@ -143,7 +143,8 @@ __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
             for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][0]), xh, acc[ob], 0, 0, 0);
         }
 #pragma unroll
-        for (int ob = 0; ob < OB; ++ob) acc[ob] *= p.pairs.ln_inv;
+        for (int ob = 0; ob < OB; ++ob)
+            acc[ob] *= *reinterpret_cast<const f32x4 *>(p.pairs.row_inv + col0 + 16 * ob + 4 * g) * p.pairs.ln_inv;
     } else {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)

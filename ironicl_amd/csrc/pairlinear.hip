@@ -13,7 +13,8 @@
 // hi.hi products and the two small ones go to separate accumulators, so two
 // chains run per row group.
 //
-// Scales: a weight matrix by a power of two set when it is packed, LayerNormed
+// Scales: each row of a weight matrix by a power of two set when it is packed
+// (an output's error is then that of its own terms), LayerNormed
 // rows by one from the LayerNorm's weights (a value is at most sqrt(512) times
 // the largest weight plus the largest bias), other rows each by its largest.
 //
@@ -152,6 +153,7 @@ __global__ __launch_bounds__(256) void pair_linear_kernel(PairLinear p, int col_
 
         const int col = 64 * CB * cg + 16 * (CB * w + cb) + 4 * g;
         const f32x4 bias = *reinterpret_cast<const f32x4 *>(p.bias + col);
+        const f32x4 w_inv = *reinterpret_cast<const f32x4 *>(p.w.row_inv + col);
         const OutMap &o = p.out;
         const int seg = col / o.col_seg, plane = seg / o.heads, head = seg - plane * o.heads;
         const long long coff = plane * o.plane_stride + head * o.head_stride + (col - seg * o.col_seg);
@@ -159,11 +161,11 @@ __global__ __launch_bounds__(256) void pair_linear_kernel(PairLinear p, int col_
         for (int r = 0; r < RG; ++r) {
             const long long row = row0 + 16 * r + m16;
             if (row >= p.m) continue;
-            const float inv = LN ? p.w.ln_inv : p.w.inv * row_inv[16 * r + m16];
+            const float inv = LN ? p.w.ln_inv : row_inv[16 * r + m16];
             f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v[e] = fmaf(big[r][e] + small[r][e], inv, bias[e]);
+                v[e] = fmaf(big[r][e] + small[r][e], w_inv[e] * inv, bias[e]);
                 if constexpr (EPI == kEpiGelu) v[e] = gelu_erf(v[e]);
             }
             if constexpr (EPI == kEpiResidual) v += *reinterpret_cast<const f32x4 *>(p.residual + row * p.ldr + col);
@@ -175,13 +177,15 @@ __global__ __launch_bounds__(256) void pair_linear_kernel(PairLinear p, int col_
 
 // A thread per (16-column block, 32-deep step, lane) of a [n, k] matrix: the
 // lane's eight values, hi then (1 KB further) lo parts.
-__global__ __launch_bounds__(256) void pair_pack_kernel(const float *w, int k, long long lanes, float scale, float *out) {
+__global__ __launch_bounds__(256) void pair_pack_kernel(const float *w, int k, long long lanes, const float *row_inv,
+                                                        float *out) {
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= lanes) return;
     const int lane = (int)(i & 63), steps = k / 32;
     const long long frag = i >> 6, cb = frag / steps;
     const float *src = w + (cb * 16 + (lane & 15)) * k + (frag - cb * steps) * 32 + 4 * (lane >> 4);
     const f32x4 a = *reinterpret_cast<const f32x4 *>(src), b = *reinterpret_cast<const f32x4 *>(src + 16);
+    const float scale = 1.0f / row_inv[cb * 16 + (lane & 15)];
     float y[8];
 #pragma unroll
     for (int e = 0; e < 4; ++e) y[e] = a[e] * scale, y[4 + e] = b[e] * scale;
@@ -189,6 +193,18 @@ __global__ __launch_bounds__(256) void pair_pack_kernel(const float *w, int k, l
     pair8(y, h, l);
     *reinterpret_cast<half8 *>(out + frag * 512 + lane * 4) = h;
     *reinterpret_cast<half8 *>(out + frag * 512 + 256 + lane * 4) = l;
+}
+
+// A wave per row: the inverse of the power of two that brings the row's
+// largest magnitude into [2^13, 2^14) (within 2^-60 .. 2^60; 1 for zeros).
+__global__ __launch_bounds__(256) void pair_rows_kernel(const float *w, int n, int k, float *row_inv) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (row >= n) return;
+    float m = 0.f;
+    for (int i = lane; i < k; i += 64) m = fmaxf(m, fabsf(w[(long long)row * k + i]));
+    m = wave_max(m);
+    const int e = m > 0.f ? max(-60, min(60, pair_exponent(m))) : 0;
+    if (lane == 0) row_inv[row] = pow2(-e);
 }
 
 float largest_magnitude(const float *w, size_t count) {
@@ -207,19 +223,19 @@ int pair_scale_exponent(double largest, int top) {
     return std::max(-60, std::min(60, top - 1 - std::ilogb(largest)));
 }
 
-PairW pair_pack(const float *host, const float *device, int n, int k, const float *lnw, const float *lnb, float *out,
-                hipStream_t stream) {
+PairW pair_pack(const float *w, int n, int k, const float *lnw, const float *lnb, float *out, hipStream_t stream) {
     if (n % 16 || k % 512) fail(3, "pair_pack: unsupported shape");
-    const int ew = pair_scale_exponent(largest_magnitude(host, (size_t)n * k), 14);
+    float *row_inv = out + (size_t)n * k;
     PairW p;
-    p.pack = out, p.inv = std::ldexp(1.f, -ew);
+    p.pack = out, p.row_inv = row_inv;
     if (lnw) {
         const int el = pair_scale_exponent(22.7 * largest_magnitude(lnw, k) + largest_magnitude(lnb, k), 15);
-        p.ln_scale = std::ldexp(1.f, el), p.ln_inv = std::ldexp(1.f, -el - ew);
+        p.ln_scale = std::ldexp(1.f, el), p.ln_inv = std::ldexp(1.f, -el);
     }
     const long long lanes = (long long)n / 16 * (k / 32) * 64;
-    hipLaunchKernelGGL(pair_pack_kernel, dim3((unsigned)ceil_div(lanes, 256LL)), dim3(256), 0, stream, device, k, lanes,
-                       std::ldexp(1.f, ew), out);
+    hipLaunchKernelGGL(pair_rows_kernel, dim3(ceil_div((size_t)n, 4)), dim3(256), 0, stream, w, n, k, row_inv);
+    hipLaunchKernelGGL(pair_pack_kernel, dim3((unsigned)ceil_div(lanes, 256LL)), dim3(256), 0, stream, w, k, lanes,
+                       row_inv, out);
     IRX_HIP(hipGetLastError());
     return p;
 }
@@ -228,11 +244,11 @@ void pair_linear(const PairLinear &a, hipStream_t stream) {
     if (a.m <= 0) return;
     const bool ln = a.lnw != nullptr;
     auto aligned = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    if (!a.x || !a.c || !a.w.pack || !a.bias || a.n % 64 || (a.k != 512 && a.k != 1024) || (ln && (a.k != 512 || !a.lnb)) ||
+    if (!a.x || !a.c || !a.w.pack || !a.w.row_inv || !a.bias || a.n % 64 || (a.k != 512 && a.k != 1024) || (ln && (a.k != 512 || !a.lnb)) ||
         (a.epilogue == kEpiResidual && !a.residual) || a.out.col_seg % 4)
         fail(3, "pair_linear: unsupported arguments");
     if ((a.ldx & 3) || (a.ldr & 3) || (a.out.ldc & 3) || (a.out.head_stride & 3) || (a.out.plane_stride & 3) ||
-        (a.out.group_stride & 3) || !aligned(a.x) || !aligned(a.c) || !aligned(a.w.pack) || !aligned(a.bias) ||
+        (a.out.group_stride & 3) || !aligned(a.x) || !aligned(a.c) || !aligned(a.w.pack) || !aligned(a.w.row_inv) || !aligned(a.bias) ||
         !aligned(a.residual) || !aligned(a.lnw) || !aligned(a.lnb))
         fail(3, "pair_linear: rows must be 16-byte aligned");
     const double m = a.m, n = a.n, k = a.k;

@@ -843,16 +843,17 @@ void weights_load(irx_weights *W, irx_tensor_lookup lookup, void *user) {
     W->arena.alloc(L.host.size() * sizeof(float));
     IRX_HIP(hipMemcpy(W->arena.p, L.host.data(), L.host.size() * sizeof(float), hipMemcpyHostToDevice));
     // The ICL blocks' and the decoder's first matrices as FP16 pairs too.
-    constexpr size_t kBlockPairs = (size_t)(3 + 1 + 2 + 2) * 512 * 512;
-    W->pairs.alloc((kIclBlocks * kBlockPairs + 1024 * 512) * sizeof(float));
+    constexpr size_t kBlockPairs = pair_pack_floats(1536, 512) + pair_pack_floats(512, 512) +
+                                   pair_pack_floats(1024, 512) + pair_pack_floats(512, 1024);
+    W->pairs.alloc((kIclBlocks * kBlockPairs + pair_pack_floats(1024, 512)) * sizeof(float));
     W->bytes = W->arena.bytes + W->pairs.bytes;
     float *next_pairs = W->pairs.f();
     auto pack = [&](const float **slot, int n, int k, const float **lnw = nullptr, const float **lnb = nullptr) {
         const size_t offset = L.offset_of(slot);
         const float *h = L.host.data();
-        const PairW p = pair_pack(h + offset, W->arena.f() + offset, n, k, lnw ? h + L.offset_of(lnw) : nullptr,
+        const PairW p = pair_pack(W->arena.f() + offset, n, k, lnw ? h + L.offset_of(lnw) : nullptr,
                                   lnb ? h + L.offset_of(lnb) : nullptr, next_pairs, nullptr);
-        next_pairs += (size_t)n * k;
+        next_pairs += pair_pack_floats(n, k);
         return p;
     };
     for (BlockW &b : W->icl) {
@@ -1217,7 +1218,7 @@ void build_impl(irx_weights *W, const irx_build_inputs *in, irx_build_outputs *o
             auto project_kv = [&](const BlockW &bw, const float *norm, float *out, const OutMap &map) {
                 if (N > kPairRows) {
                     PairW kv = bw.in_pairs;
-                    kv.pack += (size_t)512 * 512;  // past the query rows' fragments
+                    kv.pack += (size_t)512 * 512, kv.row_inv += 512;  // past the query rows
                     st.linear_pairs(norm, 512, N, 512, kv, bw.in_b + 512, 1024, out, map);
                 } else {
                     st.linear_map(norm, 512, N, 512, bw.in_w + 512 * 512, bw.in_b + 512, 1024, out, map);
@@ -2357,8 +2358,8 @@ int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t 
         f.x = dx.f(), f.ldx = 512, f.lnw = dlw.f(), f.lnb = dlb.f(), f.w = dw.f(), f.b = db.f(), f.out = dout.f();
         f.ldo = (long long)n, f.m = (int)m, f.n = (int)n;
         if (qass) f.qm0w = d0w.f(), f.qm0b = d0b.f(), f.qm2w = d2w.f(), f.qm2b = d2b.f(), f.base = dbase.f(), f.rows = (int)rows;
-        DevBuf pack(pairs ? n * 512 * 4 : 0);
-        if (pairs) f.pairs = pair_pack(w, dw.f(), (int)n, 512, lnw, lnb, pack.f(), nullptr);
+        DevBuf pack(pairs ? pair_pack_floats((int)n, 512) * 4 : 0);
+        if (pairs) f.pairs = pair_pack(dw.f(), (int)n, 512, lnw, lnb, pack.f(), nullptr);
         if (tiled) {
             // The build's form (Stages::icl_queries with more rows than the fused form takes).
             DevBuf dnorm(m * 512 * 4), dq(m * 512 * 4);
@@ -2394,11 +2395,11 @@ int irx_test_pair_linear(irx_device *device, int epilogue, const float *x, size_
             if (h) IRX_HIP(hipMemcpy(d.p, h, count * 4, hipMemcpyHostToDevice));
             return d;
         };
-        DevBuf dx = up(x, m * k), dw = up(w, n * k), db = up(b, n), pack(n * k * 4), dout = up(residual, m * n);
+        DevBuf dx = up(x, m * k), dw = up(w, n * k), db = up(b, n), pack(pair_pack_floats((int)n, (int)k) * 4), dout = up(residual, m * n);
         DevBuf dlw = up(lnw, lnw ? 512 : 1), dlb = up(lnb, lnb ? 512 : 1);
         PairLinear g{};
         g.x = dx.f(), g.ldx = (long long)k, g.lnw = lnw ? dlw.f() : nullptr, g.lnb = lnb ? dlb.f() : nullptr;
-        g.w = pair_pack(w, dw.f(), (int)n, (int)k, lnw, lnb, pack.f(), nullptr);
+        g.w = pair_pack(dw.f(), (int)n, (int)k, lnw, lnb, pack.f(), nullptr);
         g.bias = db.f(), g.residual = dout.f(), g.ldr = (long long)n, g.c = dout.f();
         g.out = OutMap::row_major((int)n, (long long)n), g.m = (int)m, g.n = (int)n, g.k = (int)k, g.epilogue = epilogue;
         pair_linear(g, nullptr);

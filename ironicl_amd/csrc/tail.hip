@@ -18,8 +18,8 @@
 // lanes. The same per-lane layout is used to load att and state and to store
 // the result.
 //
-// Scales. Weights are packed times a power of two that brings the matrix's
-// largest into [2^13, 2^14). LayerNormed rows are bounded by sqrt(128) times
+// Scales. Each row of a weight matrix is packed times a power of two that
+// brings its largest into [2^13, 2^14). LayerNormed rows are bounded by sqrt(128) times
 // the weights' largest plus the biases', the hidden layer by its weights' row
 // norms, so their scales are fixed when the weights are packed; attention
 // outputs, which can come from an imported cache, are scaled by row.
@@ -37,6 +37,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 namespace irx {
 namespace {
@@ -122,13 +123,14 @@ __device__ __forceinline__ int row_exponent(const f32x4 (&x)[8]) {
     return pair_exponent(m);
 }
 
-// Words of scales after a pack's fragments. Tail: the out-projection's inverse
-// weight scale; LN2's scale and the inverse of its product's; the hidden
-// layer's and the inverse of its product's. Head: LN1's and the inverse of its
-// product's.
+// Words of scales after a pack's fragments. Tail: LN2's scale and the hidden
+// layer's, then per output the inverse of its product's scale: out-projection
+// (weights only: attention outputs are scaled by row), W1, W2. Head: LN1's
+// scale, then per output the inverse.
 constexpr size_t kTailScales = 10 * 8192;
-enum { kTailOutInv, kTailLn, kTailLnInv, kTailHid, kTailHidInv };
-enum { kHeadLn, kHeadInv };
+enum { kTailLn = 0, kTailHid = 1, kTailOutInv = 16, kTailLnInv = kTailOutInv + 128, kTailHidInv = kTailLnInv + 256 };
+enum { kHeadLn = 0, kHeadInv = 16 };
+static_assert(kTailHidInv + 128 <= (int)kPackScales && kHeadInv + 384 <= (int)kPackScales);
 
 __device__ __forceinline__ f32x4 lds4(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
 
@@ -148,7 +150,7 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
     // Out-projection: half-chunk hc holds 32-wide k-block hc's fragments of the
     // eight output blocks.
     const int ea = row_exponent(x);
-    const float a_scale = pow2(ea), a_inv = sc[kTailOutInv] * pow2(-ea);
+    const float a_scale = pow2(ea), a_inv = pow2(-ea);
     Pair xp[4];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) xp[kb] = pair_of(x[2 * kb], x[2 * kb + 1], a_scale);
@@ -164,9 +166,10 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
         const f32x4 bo = *reinterpret_cast<const f32x4 *>(t.bo + 16 * b + 4 * g);
+        const f32x4 wi = lds4(sc + kTailOutInv + 16 * b + 4 * g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            s1[b][e] = s1[b][e] + __builtin_fmaf(acc[b][e], a_inv, bo[e]);
+            s1[b][e] = s1[b][e] + __builtin_fmaf(acc[b][e], wi[e] * a_inv, bo[e]);
             sum += s1[b][e];
         }
     }
@@ -197,7 +200,7 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
     // 16 hb + 4 g + e from half-chunk 4 + 2 c (even and odd k-blocks in
     // separate accumulators, four independent chains), then acc += W2 h from
     // half-chunk 5 + 2 c.
-    const float ln_scale = sc[kTailLn], ln_inv = sc[kTailLnInv], hid_scale = sc[kTailHid], hid_inv = sc[kTailHidInv];
+    const float ln_scale = sc[kTailLn], hid_scale = sc[kTailHid];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) xp[kb] = pair_of(x[2 * kb], x[2 * kb + 1], ln_scale);
 #pragma unroll 1
@@ -215,9 +218,10 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
             const f32x4 b1 = *reinterpret_cast<const f32x4 *>(t.b1 + 32 * c + 16 * hb + 4 * g);
+            const f32x4 wi = lds4(sc + kTailLnInv + 32 * c + 16 * hb + 4 * g);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                hg[hb][e] = gelu_erf(__builtin_fmaf(h[0][hb][e] + h[1][hb][e], ln_inv, b1[e]));
+                hg[hb][e] = gelu_erf(__builtin_fmaf(h[0][hb][e] + h[1][hb][e], wi[e], b1[e]));
         }
         const Pair hp = pair_of(hg[0], hg[1], hid_scale);
         const float *frag2 = next(h0 + 5 + 2 * c);
@@ -228,9 +232,10 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
 #pragma unroll
     for (int b = 0; b < 8; ++b) {
         const f32x4 b2 = *reinterpret_cast<const f32x4 *>(t.b2 + 16 * b + 4 * g);
+        const f32x4 wi = lds4(sc + kTailHidInv + 16 * b + 4 * g);
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[b][e], hid_inv, b2[e]) + s1[b][e];
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[b][e], wi[e], b2[e]) + s1[b][e];
         *reinterpret_cast<f32x4 *>(out + 16 * b) = v;
     }
 }
@@ -370,7 +375,7 @@ __global__ __launch_bounds__(256, 3) void column_block_kernel(ColumnBlock p, int
     // q: lane (m, g) holds head h's dims 4 g .. 4 g + 3 of row m in q[h],
     // scaled into the exp2 domain (1 / sqrt(16) = 0.25).
     const float *qsc = p.qpack + head128_pack_floats(128) - kPackScales;
-    const float ln_scale = qsc[kHeadLn], q_inv = qsc[kHeadInv];
+    const float ln_scale = qsc[kHeadLn];
     f32x4 q[8];
 #pragma unroll
     for (int ob = 0; ob < 8; ++ob) q[ob] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -384,8 +389,9 @@ __global__ __launch_bounds__(256, 3) void column_block_kernel(ColumnBlock p, int
 #pragma unroll
     for (int ob = 0; ob < 8; ++ob) {
         const f32x4 qb = *reinterpret_cast<const f32x4 *>(p.qb + 16 * ob + 4 * g);
+        const f32x4 wi = lds4(qsc + kHeadInv + 16 * ob + 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q[ob][e] = __builtin_fmaf(q[ob][e], q_inv, qb[e]) * scale;
+        for (int e = 0; e < 4; ++e) q[ob][e] = __builtin_fmaf(q[ob][e], wi[e], qb[e]) * scale;
     }
 
     // Per head: S^T = K Q^T (lane (m, g) holds keys 16 kb + 4 g + r of row
@@ -464,15 +470,16 @@ __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[
     // Out-projection of output blocks 2 w + j; s1 = state + (acc + bo) to LDS.
     f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
     const int ea = row_exponent(x);
-    const float a_scale = pow2(ea), a_inv = sc[kTailOutInv] * pow2(-ea);
+    const float a_scale = pow2(ea), a_inv = pow2(-ea);
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) pair_mfma<2>(fo[kb], pair_of(x[2 * kb], x[2 * kb + 1], a_scale), acc);
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int c0 = 16 * (2 * w + j) + 4 * g;
         const f32x4 bo = *reinterpret_cast<const f32x4 *>(t.bo + c0);
+        const f32x4 wi = lds4(sc + kTailOutInv + c0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s1[j][e] = s1[j][e] + __builtin_fmaf(acc[j][e], a_inv, bo[e]);
+        for (int e = 0; e < 4; ++e) s1[j][e] = s1[j][e] + __builtin_fmaf(acc[j][e], wi[e] * a_inv, bo[e]);
         *reinterpret_cast<f32x4 *>(&s1s[m16 * kS1Stride + c0]) = s1[j];
     }
     __syncthreads();
@@ -509,7 +516,7 @@ __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[
     }
 
     // Hidden slices c = 2 w + sl: gelu(W1 x + b1) to LDS.
-    const float ln_scale = sc[kTailLn], ln_inv = sc[kTailLnInv], hid_scale = sc[kTailHid], hid_inv = sc[kTailHidInv];
+    const float ln_scale = sc[kTailLn], hid_scale = sc[kTailHid];
     Pair xp[4];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) xp[kb] = pair_of(xn[2 * kb], xn[2 * kb + 1], ln_scale);
@@ -524,9 +531,10 @@ __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb) {
             const f32x4 b1 = *reinterpret_cast<const f32x4 *>(t.b1 + 32 * c + 16 * hb + 4 * g);
+            const f32x4 wi = lds4(sc + kTailLnInv + 32 * c + 16 * hb + 4 * g);
             f32x4 hg;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) hg[e] = gelu_erf(__builtin_fmaf(h[0][hb][e] + h[1][hb][e], ln_inv, b1[e]));
+            for (int e = 0; e < 4; ++e) hg[e] = gelu_erf(__builtin_fmaf(h[0][hb][e] + h[1][hb][e], wi[e], b1[e]));
             *reinterpret_cast<f32x4 *>(&hs[m16 * kHidStride + 32 * c + 16 * hb + 4 * g]) = hg;
         }
     }
@@ -550,9 +558,10 @@ __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[
     for (int j = 0; j < 2; ++j) {
         const int c0 = 16 * (2 * w + j);
         const f32x4 b2 = *reinterpret_cast<const f32x4 *>(t.b2 + c0 + 4 * g);
+        const f32x4 wi = lds4(sc + kTailHidInv + c0 + 4 * g);
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc2[j][e], hid_inv, b2[e]) + s1[j][e];
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc2[j][e], wi[e], b2[e]) + s1[j][e];
         *reinterpret_cast<f32x4 *>(out + c0) = v;
     }
 }
@@ -666,15 +675,16 @@ __global__ __launch_bounds__(256) void column_block_rows16_kernel(ColumnBlock p,
     }
     f32x4 q[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
     const float *qsc = p.qpack + head128_pack_floats(128) - kPackScales;
-    const float q_scale = qsc[kHeadLn], q_inv = qsc[kHeadInv];
+    const float q_scale = qsc[kHeadLn];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) pair_mfma<2>(fq[kb], pair_of(x[2 * kb], x[2 * kb + 1], q_scale), q);
     const float scale = 0.25f * kLog2e;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const f32x4 qb = *reinterpret_cast<const f32x4 *>(p.qb + 16 * (2 * w + j) + 4 * g);
+        const f32x4 wi = lds4(qsc + kHeadInv + 16 * (2 * w + j) + 4 * g);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) q[j][e] = __builtin_fmaf(q[j][e], q_inv, qb[e]) * scale;
+        for (int e = 0; e < 4; ++e) q[j][e] = __builtin_fmaf(q[j][e], wi[e], qb[e]) * scale;
     }
 
     // The tail's fragments for this wave and its state blocks, in flight
@@ -791,7 +801,7 @@ __global__ __launch_bounds__(256, 3) void head128_kernel(Head128 p) {
     }
 
     const float *sc = p.pack + head128_pack_floats(16 * NB) - kPackScales;
-    const float ln_scale = sc[kHeadLn], inv = sc[kHeadInv];
+    const float ln_scale = sc[kHeadLn];
     Pair xp[4];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) xp[kb] = pair_of(x[2 * kb], x[2 * kb + 1], ln_scale);
@@ -813,31 +823,37 @@ __global__ __launch_bounds__(256, 3) void head128_kernel(Head128 p) {
 #pragma unroll
     for (int ob = 0; ob < NB; ++ob) {
         const f32x4 b = *reinterpret_cast<const f32x4 *>(p.b + 16 * ob + 4 * g);
+        const f32x4 wi = lds4(sc + kHeadInv + 16 * ob + 4 * g);
         f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[ob][e], inv, b[e]);
+        for (int e = 0; e < 4; ++e) v[e] = __builtin_fmaf(acc[ob][e], wi[e], b[e]);
         *reinterpret_cast<f32x4 *>(out + 16 * ob) = v;
     }
 }
 
 // Fragment pair (rows r0.., columns c0 .. c0 + 31) of a row-major [.., ld]
-// matrix times `scale`: lane (n, g) = (l % 16, l / 16) slot e holds row r0 + n,
+// matrix, row r times 2^e[r]: lane (n, g) = (l % 16, l / 16) slot e holds row r0 + n,
 // column c0 + 16 (e / 4) + 4 g + e % 4; 1 KB of hi parts, then of lo parts.
-void pack_pair(const float *w, int ld, int r0, int c0, float scale, float *dst) {
+void pack_pair(const float *w, int ld, int r0, int c0, const std::vector<int> &e2, float *dst) {
     _Float16 *hi = reinterpret_cast<_Float16 *>(dst), *lo = reinterpret_cast<_Float16 *>(dst + 256);
     for (int l = 0; l < 64; ++l)
         for (int e = 0; e < 8; ++e) {
-            const float x = w[(long long)(r0 + (l & 15)) * ld + c0 + 16 * (e >> 2) + 4 * (l >> 4) + (e & 3)] * scale;
+            const int r = r0 + (l & 15);
+            const float x = std::ldexp(w[(long long)r * ld + c0 + 16 * (e >> 2) + 4 * (l >> 4) + (e & 3)], e2[r]);
             const _Float16 h = (_Float16)x;
             hi[l * 8 + e] = h;
             lo[l * 8 + e] = (_Float16)(x - (float)h);
         }
 }
 
-int weight_exponent(const float *w, size_t count) {
-    float largest = 0.f;
-    for (size_t i = 0; i < count; ++i) largest = std::max(largest, std::fabs(w[i]));
-    return pair_scale_exponent(largest, 14);
+std::vector<int> row_exponents(const float *w, int rows, int ld) {
+    std::vector<int> e(rows);
+    for (int r = 0; r < rows; ++r) {
+        float largest = 0.f;
+        for (int i = 0; i < ld; ++i) largest = std::max(largest, std::fabs(w[(long long)r * ld + i]));
+        e[r] = pair_scale_exponent(largest, 14);
+    }
+    return e;
 }
 // The bound of a LayerNormed row's values: at most sqrt(128) of deviation.
 int ln_exponent(const float *w, const float *b) {
@@ -851,12 +867,14 @@ int ln_exponent(const float *w, const float *b) {
 void head128_pack(const float *lnw, const float *lnb, const float *w, int outputs, float *out) {
     const int nb = outputs / 16;
     std::fill(out, out + head128_pack_floats(outputs), 0.f);
-    const int ew = weight_exponent(w, (size_t)outputs * 128), el = ln_exponent(lnw, lnb);
+    const std::vector<int> ew = row_exponents(w, outputs, 128);
+    const int el = ln_exponent(lnw, lnb);
     for (int kb = 0; kb < 4; ++kb)
         for (int ob = 0; ob < nb; ++ob)
-            pack_pair(w, 128, 16 * ob, 32 * kb, std::ldexp(1.f, ew), out + (size_t)(kb * nb + ob) * 512);
+            pack_pair(w, 128, 16 * ob, 32 * kb, ew, out + (size_t)(kb * nb + ob) * 512);
     float *sc = out + head128_pack_floats(outputs) - kPackScales;
-    sc[kHeadLn] = std::ldexp(1.f, el), sc[kHeadInv] = std::ldexp(1.f, -el - ew);
+    sc[kHeadLn] = std::ldexp(1.f, el);
+    for (int r = 0; r < outputs; ++r) sc[kHeadInv + r] = std::ldexp(1.f, -el - ew[r]);
 }
 
 void head128(const Head128 &h, hipStream_t stream) {
@@ -892,9 +910,8 @@ void tail128_pack(const float *wo, const float *n2w, const float *n2b, const flo
         }
         hidden = std::max(hidden, 11.5 * std::sqrt(norm) + std::fabs(bias));
     }
-    const int eo = weight_exponent(wo, 128 * 128), e1 = weight_exponent(w1, 256 * 128);
-    const int e2 = weight_exponent(w2, 128 * 256), el = ln_exponent(n2w, n2b), eh = pair_scale_exponent(hidden, 15);
-    const float so = std::ldexp(1.f, eo), s1 = std::ldexp(1.f, e1), s2 = std::ldexp(1.f, e2);
+    const std::vector<int> so = row_exponents(wo, 128, 128), s1 = row_exponents(w1, 256, 128), s2 = row_exponents(w2, 128, 256);
+    const int el = ln_exponent(n2w, n2b), eh = pair_scale_exponent(hidden, 15);
     for (int kb = 0; kb < 4; ++kb)
         for (int ob = 0; ob < 8; ++ob) pack_pair(wo, 128, 16 * ob, 32 * kb, so, out + (kb * 8 + ob) * 512);
     for (int c = 0; c < 8; ++c) {
@@ -904,9 +921,10 @@ void tail128_pack(const float *wo, const float *n2w, const float *n2b, const flo
         for (int ob = 0; ob < 8; ++ob) pack_pair(w2, 256, 16 * ob, 32 * c, s2, chunk + 4096 + ob * 512);
     }
     float *sc = out + kTailScales;
-    sc[kTailOutInv] = std::ldexp(1.f, -eo);
-    sc[kTailLn] = std::ldexp(1.f, el), sc[kTailLnInv] = std::ldexp(1.f, -el - e1);
-    sc[kTailHid] = std::ldexp(1.f, eh), sc[kTailHidInv] = std::ldexp(1.f, -eh - e2);
+    sc[kTailLn] = std::ldexp(1.f, el), sc[kTailHid] = std::ldexp(1.f, eh);
+    for (int r = 0; r < 128; ++r)
+        sc[kTailOutInv + r] = std::ldexp(1.f, -so[r]), sc[kTailHidInv + r] = std::ldexp(1.f, -eh - s2[r]);
+    for (int r = 0; r < 256; ++r) sc[kTailLnInv + r] = std::ldexp(1.f, -el - s1[r]);
 }
 
 void tail128(const Tail128 &t, hipStream_t stream, bool rows16) {

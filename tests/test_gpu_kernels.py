@@ -590,7 +590,7 @@ def test_ln_linear_gelu_matches_float64(device, m, n):
 def test_pair_linear_matches_float64(device, m, epilogue, k, n, norm):
     """The ICL products on FP16 pairs, at 16 and 32 rows per workgroup, rows of
     sizes from 2^-20 to 2^20 where they are not LayerNormed (one of zeros) and
-    weights of 1e-3: every output within 2^-20 of the sum of its terms'
+    rows of weights of 1e-3 times as much: every output within 2^-20 of the sum of its terms'
     magnitudes (operands to 2^-23 each, sums of at most 32 steps), plus the
     GELU's 1.2e-7 (1 + |x|)."""
     rng = np.random.default_rng(m + k + n)
@@ -599,7 +599,8 @@ def test_pair_linear_matches_float64(device, m, epilogue, k, n, norm):
         x *= np.exp2(rng.integers(-20, 21, (m, 1))).astype(np.float32)
         x[m // 2] = 0.0
     lnw, lnb = fast_values(512, 2, 0.2) + 1.0, fast_values(512, 3, 0.1)
-    w, b = fast_values(n * k, 4, 1e-3), fast_values(n, 5, 0.1)
+    w, b = fast_values(n * k, 4, 1e-3), fast_values(n, 5, 1e-6)
+    w = (w.reshape(n, k) * np.exp2(rng.integers(-20, 21, (n, 1)))).astype(np.float32).ravel()
     res = fast_values(m * n, 6, 1.0)
     out = np.zeros(m * n, np.float32)
     F = hip.fptr
