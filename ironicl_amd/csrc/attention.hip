@@ -163,6 +163,11 @@ __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 constexpr int kPairWaves = 8;
 constexpr float kPairHigh = 32768.0f, kPairLow = 2048.0f;
 
+// A finite softmax reference below every score, for rows that have met no key:
+// keys that score -inf weigh exp2(-inf - kLowest) = 0 against it, where a
+// reference of -inf would make that -inf - -inf.
+constexpr float kLowest = -3.402823466e38f;
+
 // One query against `keys` keys in plain FP32 by a pair of threads (32 dims
 // each) with a running maximum: the unnormalized output, its sum and reference.
 __device__ __forceinline__ void icl_row_fp32(const float *q, const float *k, const float *v, int keys, int part,
@@ -170,7 +175,7 @@ __device__ __forceinline__ void icl_row_fp32(const float *q, const float *k, con
     float qr[32];
 #pragma unroll
     for (int d = 0; d < 32; ++d) qr[d] = q[32 * part + d] * (0.125f * kLog2e), o[d] = 0.f;
-    m = -INFINITY, l = 0.f;
+    m = kLowest, l = 0.f;
     for (int key = 0; key < keys; ++key) {
         const float *kr = k + (long long)key * 64 + 32 * part, *vr = v + (long long)key * 64 + 32 * part;
         float s = 0.f;
@@ -178,7 +183,7 @@ __device__ __forceinline__ void icl_row_fp32(const float *q, const float *k, con
         for (int d = 0; d < 32; ++d) s = __builtin_fmaf(qr[d], kr[d], s);
         s += __shfl_xor(s, 1, 64);
         const float mn = fmaxf(m, s);
-        const float a = key ? __builtin_amdgcn_exp2f(m - mn) : 0.f, w = __builtin_amdgcn_exp2f(s - mn);
+        const float a = __builtin_amdgcn_exp2f(m - mn), w = __builtin_amdgcn_exp2f(s - mn);
         l = l * a + w;
 #pragma unroll
         for (int d = 0; d < 32; ++d) o[d] = o[d] * a + w * vr[d];
@@ -397,7 +402,6 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[d][j][r] = 0.f;
-    constexpr float kLowest = -3.0e38f;  // a finite reference below every score
     float m_ref[2] = {kLowest, kLowest}, l_run[2] = {0.f, 0.f};
     f32x16 s[2];    // scores of the tile (raw products)
     half8 ph[2][2], pl[2][2];  // its probabilities, [query block][step]
@@ -594,8 +598,11 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
             dst = p.partial + prow * 64;
             if (part == 0) p.partial[(long long)g.splits * g.part_rows * 64 + prow] = m + log2f(l);
         }
+        // A range whose keys all score -inf adds nothing to the row's other
+        // ranges; a row of nothing else has no softmax.
+        const float inv = SPLIT && !(l > 0.f) ? 0.f : 1.0f / l;
 #pragma unroll
-        for (int d = 0; d < 32; ++d) dst[32 * part + d] = out[d] / l;
+        for (int d = 0; d < 32; ++d) dst[32 * part + d] = out[d] * inv;
         return;
     }
     if (khalf == 0) flush(!flushed);
@@ -1527,7 +1534,7 @@ __global__ __launch_bounds__(64) void icl_merge_kernel(IclAttention p, int split
     const long long step = (long long)p.pairs * q_padded;  // rows between splits
     const long long row0 = (long long)pair * q_padded + qrow;
     const float *lse = p.partial + (long long)splits * step * 64 + row0;
-    float m_run = -INFINITY, den = 0.f;
+    float m_run = kLowest, den = 0.f;
     f32x4 num = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = sg; s0 < splits; s0 += 4 * kMergePerGroup) {
         float l8[kMergePerGroup];
@@ -1544,7 +1551,7 @@ __global__ __launch_bounds__(64) void icl_merge_kernel(IclAttention p, int split
         float m_new = m_run;
 #pragma unroll
         for (int j = 0; j < kMergePerGroup; ++j) m_new = fmaxf(m_new, l8[j]);
-        const float a = __builtin_amdgcn_exp2f(m_run - m_new);  // 0 while m_run is -inf
+        const float a = __builtin_amdgcn_exp2f(m_run - m_new);
         num *= a, den *= a;
 #pragma unroll
         for (int j = 0; j < kMergePerGroup; ++j) {
@@ -1561,12 +1568,10 @@ __global__ __launch_bounds__(64) void icl_merge_kernel(IclAttention p, int split
 #pragma unroll
         for (int e = 0; e < 4; ++e) num_o[e] = __shfl_xor(num[e], off, 64);
         const float m_new = fmaxf(m_run, m_o);
-        if (m_new != -INFINITY) {  // both groups empty: nothing to combine
-            const float a = __builtin_amdgcn_exp2f(m_run - m_new), b = __builtin_amdgcn_exp2f(m_o - m_new);
-            num = a * num + b * num_o;
-            den = a * den + b * den_o;
-            m_run = m_new;
-        }
+        const float a = __builtin_amdgcn_exp2f(m_run - m_new), b = __builtin_amdgcn_exp2f(m_o - m_new);
+        num = a * num + b * num_o;
+        den = a * den + b * den_o;
+        m_run = m_new;
     }
     if (sg != 0) return;
     const int b = pair / kHeads, head = pair - b * kHeads;
@@ -1612,9 +1617,9 @@ __global__ __launch_bounds__(256) void icl_merge_rows_kernel(IclAttention p, Icl
         v[s] = *reinterpret_cast<const f32x4 *>(p.partial + (row0 + sl * step) * 64 + d);
         l[s] = s < splits ? ls : -INFINITY;
     }
-    float m = l[0];
+    float m = kLowest;
 #pragma unroll
-    for (int s = 1; s < MAXS; ++s) m = fmaxf(m, l[s]);
+    for (int s = 0; s < MAXS; ++s) m = fmaxf(m, l[s]);
     f32x4 num = {0.f, 0.f, 0.f, 0.f};
     float den = 0.f;
 #pragma unroll

@@ -171,6 +171,31 @@ def test_icl_attention_beyond_the_scaled_products(device, query_rows, rows):
         assert np.abs(out[pair] - want).max() < 1e-5
 
 
+@pytest.mark.parametrize("query_rows,rows", [(33, 200), (300, 9001)])
+@pytest.mark.parametrize("hidden", ["1 of 64", "2 of 64", "40 of 64", "first half"])
+@pytest.mark.parametrize("kind", ["overflow", "lowest", "infinite"])
+def test_icl_attention_hidden_keys_lead_a_range(device, query_rows, rows, hidden, kind):
+    """More than 32 rows: keys that score -inf (the type's lowest value against queries of 8,
+    whose products overflow; infinite keys) or the lowest finite score weigh
+    nothing wherever they stand: first in every 64-key tile, and so first in
+    every key range, or filling whole ranges."""
+    pairs = 8
+    rng = np.random.default_rng(rows)
+    q, k, v = (rng.standard_normal((pairs, n, 64)).astype(np.float32) for n in (query_rows, rows, rows))
+    q[:, :, 0] = 1.0 if kind == "lowest" else 8.0
+    k[:, :, 0] = 0.0
+    index = np.arange(rows)
+    out_of_sight = index < rows // 2 if hidden == "first half" else index % 64 < int(hidden.split()[0])
+    k[:, out_of_sight] = 0.0
+    k[:, out_of_sight, 0] = -np.inf if kind == "infinite" else np.finfo(np.float32).min
+    out = np.zeros_like(q)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_icl_attention(device.handle, F(q), F(k), F(v), pairs, query_rows, rows, F(out)))
+    for pair in (0, 7):
+        want = attention64(q[pair], k[pair, ~out_of_sight], v[pair, ~out_of_sight], 0.125)
+        assert np.abs(out[pair] - want).max() < 1e-5
+
+
 @pytest.mark.parametrize("rows", [1, 63, 64, 65, 2000, 10007])
 def test_icl_attention_matches_float64(device, rows):
     pairs = 64
