@@ -149,8 +149,8 @@ constexpr int kFlushTiles = 64;
 //
 // Infinite keys or values, values all below 2^-47, and keys so large that
 // scores could pass 2^20 (where one scale would serve neither those keys nor
-// their neighbours) are left to a plain FP32 loop over the workgroup's
-// queries (icl_row_fp32).
+// their neighbours) are left to FP32 products over the workgroup's queries
+// (icl_range_fp32), at once if the first tile shows it and else after the loop.
 struct IclPairTile {
     u32x4 h[kKeyTile * 8], l[kKeyTile * 8];  // K: [key][8 chunks of 8 dims]; V: [dim][8 chunks of 8 keys]
 };
@@ -168,26 +168,141 @@ constexpr float kPairHigh = 32768.0f, kPairLow = 2048.0f;
 // reference of -inf would make that -inf - -inf.
 constexpr float kLowest = -3.402823466e38f;
 
-// One query against `keys` keys in plain FP32 by a pair of threads (32 dims
-// each) with a running maximum: the unnormalized output, its sum and reference.
-__device__ __forceinline__ void icl_row_fp32(const float *q, const float *k, const float *v, int keys, int part,
-                                           float *o, float &m, float &l) {
-    float qr[32];
+// A workgroup's 256 queries against its key range on the FP32 matrix cores
+// (v_mfma_f32_32x32x2f32), for operands that scaled FP16 pairs do not serve.
+// Wave w takes queries 32 w .. + 31, and lane (q, half) = (lane % 32, lane / 32):
+//   S^T (key x query), step 4 c + e: A = K[key][dim 32 half + 4 c + e], B = the
+//     lane's query, same dim; register r of block b is key 32 b + 8 (r / 4) +
+//     4 half + r % 4;
+//   O^T (dim x query), step r: B = that register's probability, A = V[its key],
+//     even dims in o[0] and odd ones in o[1] (one 8-byte read serves both).
+// Sums are taken in two levels, as in the kernel below. 512 queries x 50,000
+// keys x 8 pairs take 490 us so, 107 of the FP32 matrix cores' 157 TFLOP/s (a
+// scalar loop with a query to a pair of threads took 5,560).
+struct IclFp32Tile {
+    float k[kKeyTile * 64];  // 16-byte chunk c of key r at chunk c ^ (r % 16)
+    float v[kKeyTile * 64];
+};
+
+template <bool SPLIT, class Rsrc>
+__device__ __forceinline__ void icl_range_fp32(const IclAttention &p, const IclLaunch &g, IclFp32Tile &t, Rsrc &&rsrc,
+                                               int wave, int pair, int qt, int split, int tail_unit, int k_begin,
+                                               int k_end) {
+    // (The lane counted anew: held through the caller's loop it would spill.)
+    const int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), tid = 64 * wave + lane;
+    const int half = lane >> 5, r32 = lane & 31, row = 32 * wave + r32;
+    const int qrow = qt * kIclQueries + row;
+    float q[32];
+    const float *src = p.q + pair * p.q_pair_stride + (long long)min(qrow, p.q_rows - 1) * 64 + 32 * half;
 #pragma unroll
-    for (int d = 0; d < 32; ++d) qr[d] = q[32 * part + d] * (0.125f * kLog2e), o[d] = 0.f;
-    m = kLowest, l = 0.f;
-    for (int key = 0; key < keys; ++key) {
-        const float *kr = k + (long long)key * 64 + 32 * part, *vr = v + (long long)key * 64 + 32 * part;
-        float s = 0.f;
+    for (int c = 0; c < 8; ++c) {
+        const f32x4 x = *reinterpret_cast<const f32x4 *>(src + 4 * c);
 #pragma unroll
-        for (int d = 0; d < 32; ++d) s = __builtin_fmaf(qr[d], kr[d], s);
-        s += __shfl_xor(s, 1, 64);
-        const float mn = fmaxf(m, s);
-        const float a = __builtin_amdgcn_exp2f(m - mn), w = __builtin_amdgcn_exp2f(s - mn);
-        l = l * a + w;
+        for (int e = 0; e < 4; ++e) q[4 * c + e] = x[e] * (0.125f * kLog2e);
+    }
+    // Thread t stages dims 8 (t % 8) .. +7 of key t / 8; rows past the range are zeros.
+    const int s_key = tid >> 3, s_chunk = 2 * (tid & 7);
+    u32x4 kr[2], vr[2];
+    auto load = [&](int k0) {
+        const auto kd = rsrc(p.k + pair * p.kv_pair_stride, k0), vd = rsrc(p.v + pair * p.kv_pair_stride, k0);
 #pragma unroll
-        for (int d = 0; d < 32; ++d) o[d] = o[d] * a + w * vr[d];
-        m = mn;
+        for (int i = 0; i < 2; ++i) {
+            kr[i] = __builtin_amdgcn_raw_buffer_load_b128(kd, tid * 32 + 16 * i, 0, 0);
+            vr[i] = __builtin_amdgcn_raw_buffer_load_b128(vd, tid * 32 + 16 * i, 0, 0);
+        }
+    };
+    float m = kLowest, l = 0.f, l_total = 0.f;
+    f32x16 o[2], total[2];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) total[0][r] = total[1][r] = 0.f;
+    load(k_begin);
+#pragma unroll 1
+    for (int k0 = k_begin; k0 < k_end;) {
+        const int stop = min(k_end, k0 + kFlushTiles * kKeyTile);
+        l = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[0][r] = o[1][r] = 0.f;
+#pragma unroll 1
+        for (; k0 < stop; k0 += kKeyTile) {
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                *reinterpret_cast<u32x4 *>(&t.k[s_key * 64 + 4 * ((s_chunk + i) ^ (s_key & 15))]) = kr[i];
+                *reinterpret_cast<u32x4 *>(&t.v[s_key * 64 + 4 * (s_chunk + i)]) = vr[i];
+            }
+            __syncthreads();
+            if (k0 + kKeyTile < k_end) load(k0 + kKeyTile);
+            f32x16 s[2];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[0][r] = s[1][r] = 0.f;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const int at = r32 * 64 + 4 * ((8 * half + c) ^ (r32 & 15));
+                const f32x4 a0 = *reinterpret_cast<const f32x4 *>(&t.k[at]);
+                const f32x4 a1 = *reinterpret_cast<const f32x4 *>(&t.k[at + 32 * 64]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    s[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], q[4 * c + e], s[0], 0, 0, 0);
+                    s[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], q[4 * c + e], s[1], 0, 0, 0);
+                }
+                if (c % 2) __builtin_amdgcn_sched_barrier(0);  // (all reads at once spill)
+            }
+            float mt = kLowest;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    if (k0 + 32 * b + 8 * (r >> 2) + 4 * half + (r & 3) >= k_end) s[b][r] = -INFINITY;
+                    mt = fmaxf(mt, s[b][r]);
+                }
+            const float m_new = fmaxf(m, halves_max(mt)), alpha = __builtin_amdgcn_exp2f(m - m_new);
+            m = m_new, l *= alpha, l_total *= alpha;
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                o[0][r] *= alpha, o[1][r] *= alpha, total[0][r] *= alpha, total[1][r] *= alpha;
+            float sum = 0.f;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s[b][r] = __builtin_amdgcn_exp2f(s[b][r] - m);
+                    sum += s[b][r];
+                }
+            l += sum;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int key = 32 * b + 8 * (r >> 2) + 4 * half + (r & 3);
+                    const f32x2 a = *reinterpret_cast<const f32x2 *>(&t.v[key * 64 + 2 * r32]);
+                    o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[0], s[b][r], o[0], 0, 0, 0);
+                    o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[1], s[b][r], o[1], 0, 0, 0);
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+                }
+        }
+        l_total += l;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) total[0][r] += o[0][r], total[1][r] += o[1][r];
+    }
+    l = halves_sum(l_total);
+    if (qrow >= p.q_rows) return;
+    float *dst;
+    if constexpr (!SPLIT) {
+        const int b = pair / kHeads, head = pair - b * kHeads;
+        dst = p.o + ((long long)b * p.q_rows + qrow) * p.ldo + head * 64;
+    } else {
+        const long long prow = g.tail_units ? split * g.part_rows + (long long)tail_unit * kIclQueries + row
+                                            : split * g.part_rows + (long long)pair * g.q_padded + qrow;
+        dst = p.partial + prow * 64;
+        if (half == 0) p.partial[(long long)g.splits * g.part_rows * 64 + prow] = m + log2f(l);
+    }
+    // A range whose keys all score -inf adds nothing to the row's other
+    // ranges; a row of nothing else has no softmax.
+    const float inv = SPLIT && !(l > 0.f) ? 0.f : 1.0f / l;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const f32x2 v = {total[0][r] * inv, total[1][r] * inv};
+        *reinterpret_cast<f32x2 *>(dst + 2 * (8 * (r >> 2) + 4 * half + (r & 3))) = v;
     }
 }
 
@@ -541,7 +656,16 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
     update_scales();
     convert_k(0), convert_v(0, 0);
     load_k(tile_at(1)), load_v(tile_at(1));
+    if (lane == 0) lds.special[wave] = special;
     phase_barrier();
+    auto any_special = [&]() {
+        unsigned any = 0;
+#pragma unroll
+        for (int w = 0; w < kPairWaves; ++w) any |= lds.special[w];
+        return __builtin_amdgcn_readfirstlane(any) != 0;
+    };
+    // (Where the first tile shows that the range is left to FP32, no loop.)
+    const int paired = any_special() ? 0 : tiles;
     scores(0);
     if (khalf) {
         // Half 1 runs a phase behind half 0, and writes K a tile ahead of it.
@@ -552,7 +676,7 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
     }
     bool flushed = false;
     int since = 0;
-    for (int t = 0, vb = 0; t < tiles; ++t) {
+    for (int t = 0, vb = 0; t < paired; ++t) {
         const int vb_next = vb == 2 ? 0 : vb + 1;
         // VALU phase.
         if constexpr (FLUSH) {
@@ -576,33 +700,10 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
     if (khalf == 0) phase_barrier();
     if (lane == 0) lds.special[wave] = special;
     __syncthreads();
-    unsigned any_special = 0;
-#pragma unroll
-    for (int w = 0; w < kPairWaves; ++w) any_special |= lds.special[w];
-    if (__builtin_amdgcn_readfirstlane(any_special)) {
-        // Plain FP32 for the whole range: thread pairs (2 i, 2 i + 1) take query i.
-        const int row = tid >> 1, part = tid & 1, qrow = qt * kIclQueries + row;
-        const int safe = min(qrow, p.q_rows - 1);
-        float out[32], m, l;
-        icl_row_fp32(p.q + pair * p.q_pair_stride + (long long)safe * 64, kbase + (long long)k_begin * 64,
-                      vbase + (long long)k_begin * 64, k_end - k_begin, part, out, m, l);
-        if (qrow >= p.q_rows) return;
-        float *dst;
-        if constexpr (!SPLIT) {
-            const int b = pair / kHeads, head = pair - b * kHeads;
-            dst = p.o + ((long long)b * p.q_rows + qrow) * p.ldo + head * 64;
-        } else {
-            const long long prow =
-                g.tail_units ? split * g.part_rows + (long long)tail_unit * kIclQueries + row
-                             : split * g.part_rows + (long long)pair * g.q_padded + qrow;
-            dst = p.partial + prow * 64;
-            if (part == 0) p.partial[(long long)g.splits * g.part_rows * 64 + prow] = m + log2f(l);
-        }
-        // A range whose keys all score -inf adds nothing to the row's other
-        // ranges; a row of nothing else has no softmax.
-        const float inv = SPLIT && !(l > 0.f) ? 0.f : 1.0f / l;
-#pragma unroll
-        for (int d = 0; d < 32; ++d) dst[32 * part + d] = out[d] * inv;
+    if (any_special()) {
+        // FP32 products for the whole range.
+        icl_range_fp32<SPLIT>(p, g, reinterpret_cast<IclFp32Tile &>(lds.data.tiles), rsrc, wave, pair, qt, split,
+                              tail_unit, k_begin, k_end);
         return;
     }
     if (khalf == 0) flush(!flushed);

@@ -171,6 +171,28 @@ def test_icl_attention_beyond_the_scaled_products(device, query_rows, rows):
         assert np.abs(out[pair] - want).max() < 1e-5
 
 
+def test_icl_attention_beyond_the_scaled_products_long_range(device):
+    """50,000 keys in one range with one key taking all but 1.3e-3 of each
+    row's weight, the others 2.5e-8 each, in operands left to FP32 products
+    (a dim of 1e7 in every key that no query has): what the 49,999 add must
+    not be rounded away, so sums are taken in two levels."""
+    pairs, query_rows, rows = 8, 8192, 50000
+    rng = np.random.default_rng(5)
+    q = np.zeros((pairs, query_rows, 64), np.float32)
+    q[:, :, 0] = 8.0
+    k = np.zeros((pairs, rows, 64), np.float32)
+    k[:, :, 1] = rng.standard_normal((pairs, rows))
+    k[:, :, 63] = 1e7
+    k[:, 3, 0] = 17.5
+    v = rng.standard_normal((pairs, rows, 64), dtype=np.float32)
+    out = np.zeros_like(q)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_icl_attention(device.handle, F(q), F(k), F(v), pairs, query_rows, rows, F(out)))
+    for pair in (0, 7):
+        want = attention64(q[pair, :1], k[pair], v[pair], 0.125)
+        assert np.abs(out[pair] - want).max() < 1e-5
+
+
 @pytest.mark.parametrize("query_rows,rows", [(33, 200), (300, 9001)])
 @pytest.mark.parametrize("hidden", ["1 of 64", "2 of 64", "40 of 64", "first half"])
 @pytest.mark.parametrize("kind", ["overflow", "lowest", "infinite"])
