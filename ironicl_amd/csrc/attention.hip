@@ -460,8 +460,9 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
     for (int w = 0; w < kPairWaves; ++w) q_largest = fmaxf(q_largest, lds.largest[w]);
     q_largest = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(q_largest)));
     // The wave's scales, 2^ek and 2^ev, brought up to date with the staged
-    // values (rarely anything to do).
-    int ek = 0, ev = 0;
+    // values (rarely anything to do). They start as those of a share of zeros,
+    // which no first share keeps whose scores could pass the bound.
+    int ek = 126, ev = 60;
     auto update_scales = [&]() {
         float km = 0.f, vm = 0.f;
 #pragma unroll

@@ -193,6 +193,23 @@ def test_icl_attention_beyond_the_scaled_products_long_range(device):
         assert np.abs(out[pair] - want).max() < 1e-5
 
 
+@pytest.mark.parametrize("query_rows,rows", [(33, 1), (33, 40), (300, 9001)])
+def test_icl_attention_huge_scores_from_the_first_tile(device, query_rows, rows):
+    """Operands of 2^12 .. 2^13 need no scaling as FP16 pairs, and their scores
+    reach 2^29, where an FP32 ulp is 64: more than any margin a scaled
+    probability has. Each row's weight is all on the last key (the next one
+    scores 2^15 less), so the output is that key's value."""
+    pairs = 8
+    q = np.full((pairs, query_rows, 64), 8192.0, np.float32)
+    k = np.empty((pairs, rows, 64), np.float32)
+    k[:] = (4096.0 + 0.5 * np.arange(rows, dtype=np.float32))[None, :, None]
+    v = np.random.default_rng(rows).uniform(-8192, 8192, (pairs, rows, 64)).astype(np.float32)
+    out = np.zeros_like(q)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_icl_attention(device.handle, F(q), F(k), F(v), pairs, query_rows, rows, F(out)))
+    assert np.abs(out - v[:, -1:]).max() <= 8192 * 2.0 ** -22
+
+
 @pytest.mark.parametrize("query_rows,rows", [(33, 200), (300, 9001)])
 @pytest.mark.parametrize("hidden", ["1 of 64", "2 of 64", "40 of 64", "first half"])
 @pytest.mark.parametrize("kind", ["overflow", "lowest", "infinite"])
