@@ -79,9 +79,9 @@ __device__ __forceinline__ float halves_sum(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-// Maximum over a wave of magnitudes (x >= 0), in every lane: rotations within
-// rows of 16 lanes, then the rows.
-__device__ __forceinline__ float wave_magnitude(float x) {
+// Maximum over a wave, in every lane: rotations within rows of 16 lanes, then
+// the rows.
+__device__ __forceinline__ float wave_max_all(float x) {
 #define IRX_ROTATE(n) \
     x = fmaxf(x, __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + n, 0xf, 0xf, true)))
     IRX_ROTATE(8);
@@ -139,18 +139,27 @@ constexpr int kFlushTiles = 64;
 //
 // Scales, all powers of two. Queries: per row, in registers. Keys and values:
 // per wave's share of a tile (8 keys x 64 dims), kept while the share's
-// largest scaled magnitude stays in [2^11, 2^15] and else set to bring it into
-// [2^13, 2^14): an operand is held to 2^-23 of itself or 2^-36 of the largest
-// of its eight keys. The key scale joins the softmax's multiply (four keys of
+// largest scaled magnitude stays below 2^15 (keys' at 2^11 or more) and else
+// set to bring it into [2^13, 2^14): a pair holds an operand to 2^-24 of itself, or to 2^-25
+// absolute (scaled) below that. The key scale joins the softmax's multiply (four keys of
 // it to a register group); the value scale joins the exponent, so that the
 // probability carries its inverse, and is taken out of the row sum. The
 // reference the exponent is taken against is raised, to 8 (base 2) below the
 // running maximum, when a scaled probability would pass 2^15.
 //
-// Infinite keys or values, values all below 2^-47, and keys so large that
-// scores could pass 2^20 (where one scale would serve neither those keys nor
-// their neighbours) are left to FP32 products over the workgroup's queries
-// (icl_range_fp32), at once if the first tile shows it and else after the loop.
+// What the absolute part cannot hold is left to FP32 products over the
+// workgroup's queries (icl_range_fp32), at once if the first tile shows it and
+// else after the loop:
+//   infinite keys or values, and values all below 2^-47;
+//   keys so large that scores could pass 2^17 where their scale is set (as
+//     8 |q| |k| of the largest magnitudes). Below it the absolute parts of the
+//     64 products of q and k add up to at most 2^-21 of score;
+//   values that spread too far: a share's smallest key times its smallest dim
+//     (zeros aside, each by its largest value) over the largest, the size of a
+//     value that is small both ways, must be 1/2 or more scaled, so that every
+//     value is held to 2^-24 of the size its key and dim have. That each dim's
+//     largest value reaches 2^7, and that some dim's smallest does, shows it in
+//     most tiles (2^7 2^7 / 2^15) and keeps the scale.
 struct IclPairTile {
     u32x4 h[kKeyTile * 8], l[kKeyTile * 8];  // K: [key][8 chunks of 8 dims]; V: [dim][8 chunks of 8 keys]
 };
@@ -161,7 +170,8 @@ struct IclPairTiles {
 // lanes read or write at one chunk cover all 64 LDS banks.
 __device__ __forceinline__ int pair_swizzle(int row) { return (row >> 1) & 7; }
 constexpr int kPairWaves = 8;
-constexpr float kPairHigh = 32768.0f, kPairLow = 2048.0f;
+constexpr int kPairHigh = 15, kPairLow = 11, kPairEven = 7;  // powers of two
+constexpr float kPairScore = 131072.0f;
 
 // A finite softmax reference below every score, for rows that have met no key:
 // keys that score -inf weigh exp2(-inf - kLowest) = 0 against it, where a
@@ -453,7 +463,7 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
     }
 
     bool special = false;
-    q_largest = wave_magnitude(q_largest);
+    q_largest = wave_max_all(q_largest);
     if (lane == 0) lds.largest[wave] = q_largest;
     __syncthreads();
 #pragma unroll
@@ -463,25 +473,45 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
     // values (rarely anything to do). They start as those of a share of zeros,
     // which no first share keeps whose scores could pass the bound.
     int ek = 126, ev = 60;
+    // Unscaled limits: kPairHigh and kPairLow of keys, kPairHigh and kPairEven
+    // of values.
+    auto limit = [](int e) { return pow2(min(e, 127)); };
+    float k_high = limit(kPairHigh - ek), k_low = limit(kPairLow - ek);
+    float v_high = limit(kPairHigh - ev), v_even = limit(kPairEven - ev);
     auto update_scales = [&]() {
-        float km = 0.f, vm = 0.f;
+        float km = 0.f, vm = 0.f, vl = fabsf(vr[0]);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) km = fmaxf(km, fabsf(kr[i])), vm = fmaxf(vm, fabsf(vr[i]));
-        const float ks = km * pow2(ek), vs = vm * pow2(ev);
-        const unsigned long long high = __ballot(fmaxf(ks, vs) > kPairHigh);
-        const unsigned long long k_ok = __ballot(ks >= kPairLow), v_ok = __ballot(vs >= kPairLow);
-        if (__builtin_expect(high != 0 || k_ok == 0 || v_ok == 0, 0)) {
-            km = wave_magnitude(km), vm = wave_magnitude(vm);
-            const unsigned kb = __builtin_amdgcn_readfirstlane(__float_as_uint(km));
-            const unsigned vb = __builtin_amdgcn_readfirstlane(__float_as_uint(vm));
+        for (int i = 0; i < 8; ++i)
+            km = fmaxf(km, fabsf(kr[i])), vm = fmaxf(vm, fabsf(vr[i])), vl = fminf(vl, fabsf(vr[i]));
+        // (Bitwise: one branch for it all.) Every dim reaches v_even, and every
+        // key does (in some dim).
+        auto uneven = [&]() { return int(__ballot(vm >= v_even) != ~0ull) | int(__ballot(vl >= v_even) == 0); };
+        const unsigned long long high = __ballot(km >= k_high) | __ballot(vm >= v_high);
+        if (__builtin_expect(int(high != 0) | int(__ballot(km >= k_low) == 0) | uneven(), 0)) {
+            const float k_largest = wave_max_all(km), v_largest = wave_max_all(vm);
+            const unsigned kb = __builtin_amdgcn_readfirstlane(__float_as_uint(k_largest));
+            const unsigned vb = __builtin_amdgcn_readfirstlane(__float_as_uint(v_largest));
             // 8 |q| |k| bounds a score (64 dims, times 1/8).
-            if (kb >= 0x7f800000u || vb >= 0x7f800000u || __uint_as_float(kb) * 8.0f * q_largest > 1048576.0f ||
+            if (kb >= 0x7f800000u || vb >= 0x7f800000u || __uint_as_float(kb) * 8.0f * q_largest > kPairScore ||
                 (vb && __uint_as_float(vb) < 7e-15f))
                 special = true;
             if (kb && kb < 0x7f800000u) ek = pair_exponent(__uint_as_float(kb));
             // (A share of zeros takes the scale of the smallest values, so that
             // its probabilities do not set the reference.)
             if (vb < 0x7f800000u) ev = vb ? min(60, pair_exponent(__uint_as_float(vb))) : 60;
+            k_high = limit(kPairHigh - ek), k_low = limit(kPairLow - ek);
+            v_high = limit(kPairHigh - ev), v_even = limit(kPairEven - ev);
+            if (vb && vb < 0x7f800000u && uneven()) {
+                // The smallest nonzero key and dim, each by its largest value.
+                float key = -INFINITY;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float m = wave_max_all(fabsf(vr[i]));
+                    key = fmaxf(key, m > 0.f ? -m : -INFINITY);
+                }
+                const float dim = wave_max_all(vm > 0.f ? -vm : -INFINITY), up = pow2(ev);
+                if (dim * up * (key * up) < 0.5f * (v_largest * up)) special = true;
+            }
         }
     };
     // The staged tiles, u of K and w of V (to buffer `vb`), to LDS. Every lane

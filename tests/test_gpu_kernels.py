@@ -210,6 +210,41 @@ def test_icl_attention_huge_scores_from_the_first_tile(device, query_rows, rows)
     assert np.abs(out - v[:, -1:]).max() <= 8192 * 2.0 ** -22
 
 
+@pytest.mark.parametrize("query_rows,rows", [(33, 2), (64, 129), (257, 700)])
+@pytest.mark.parametrize("kind", ["key", "dim", "both"])
+@pytest.mark.parametrize("octaves", [6, 11, 14, 20, 30])
+def test_icl_attention_value_spread(device, query_rows, rows, kind, octaves):
+    """Values far below the largest of their eight keys, across the spread at
+    which scaled FP16 pairs no longer hold them: every 8th key 2^octaves
+    larger, at a score that gives it no weight; every 5th dim 2^octaves
+    smaller; both. Scores are below 1, so a term p v carries a few roundings
+    (the pair of p 2^-24, that of v 2^-24 of v or of the size its key and dim
+    have, the exponent's sum and exp2 2^-22, the accumulated sums' 2^-22 over
+    700 keys): 2^-20 of the sum of p and those sizes."""
+    pairs = 8
+    rng = np.random.default_rng(octaves)
+    q, k, v = (rng.standard_normal((pairs, n, 64)).astype(np.float32) for n in (query_rows, rows, rows))
+    q[:] = np.abs(q) * np.float32(0.25)
+    k *= np.float32(0.25)
+    size = np.ones((rows, 64), np.float32)
+    if kind != "dim":
+        k[:, ::8] = -400.0
+        size[::8] *= np.float32(2.0 ** octaves)
+    if kind != "key":
+        size[:, ::5] *= np.float32(2.0 ** -octaves)
+    v *= size
+    out = np.zeros_like(q)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_icl_attention(device.handle, F(q), F(k), F(v), pairs, query_rows, rows, F(out)))
+    for pair in (0, 7):
+        scores = q[pair].astype(np.float64) @ k[pair].astype(np.float64).T / 8.0
+        p = np.exp(scores - scores.max(axis=1, keepdims=True))
+        p /= p.sum(axis=1, keepdims=True)
+        bound = p @ np.maximum(np.abs(v[pair]), size).astype(np.float64)
+        worst = (np.abs(out[pair] - p @ v[pair].astype(np.float64)) / bound).max()
+        assert worst < 2.0 ** -20, (pair, worst * 2.0 ** 20)
+
+
 @pytest.mark.parametrize("query_rows,rows", [(33, 200), (300, 9001)])
 @pytest.mark.parametrize("hidden", ["1 of 64", "2 of 64", "40 of 64", "first half"])
 @pytest.mark.parametrize("kind", ["overflow", "lowest", "infinite"])
