@@ -144,7 +144,7 @@ __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
         }
 #pragma unroll
         for (int ob = 0; ob < OB; ++ob)
-            acc[ob] *= *reinterpret_cast<const f32x4 *>(p.pairs.row_inv + col0 + 16 * ob + 4 * g) * p.pairs.ln_inv;
+            acc[ob] = acc[ob] * *reinterpret_cast<const f32x4 *>(p.pairs.row_inv + col0 + 16 * ob + 4 * g) * p.pairs.ln_inv;
     } else {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)

@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void pair_linear_kernel(PairLinear p, int col_
             f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v[e] = fmaf(big[r][e] + small[r][e], w_inv[e] * inv, bias[e]);
+                v[e] = fmaf((big[r][e] + small[r][e]) * w_inv[e], inv, bias[e]);
                 if constexpr (EPI == kEpiGelu) v[e] = gelu_erf(v[e]);
             }
             if constexpr (EPI == kEpiResidual) v += *reinterpret_cast<const f32x4 *>(p.residual + row * p.ldr + col);
@@ -196,14 +196,14 @@ __global__ __launch_bounds__(256) void pair_pack_kernel(const float *w, int k, l
 }
 
 // A wave per row: the inverse of the power of two that brings the row's
-// largest magnitude into [2^13, 2^14) (within 2^-60 .. 2^60; 1 for zeros).
+// largest magnitude into [2^13, 2^14) (1 for zeros).
 __global__ __launch_bounds__(256) void pair_rows_kernel(const float *w, int n, int k, float *row_inv) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (row >= n) return;
     float m = 0.f;
     for (int i = lane; i < k; i += 64) m = fmaxf(m, fabsf(w[(long long)row * k + i]));
     m = wave_max(m);
-    const int e = m > 0.f ? max(-60, min(60, pair_exponent(m))) : 0;
+    const int e = m > 0.f ? pair_exponent(m) : 0;
     if (lane == 0) row_inv[row] = pow2(-e);
 }
 
@@ -220,7 +220,7 @@ float largest_magnitude(const float *w, size_t count) {
 
 int pair_scale_exponent(double largest, int top) {
     if (!(largest > 0.0)) return 0;
-    return std::max(-60, std::min(60, top - 1 - std::ilogb(largest)));
+    return std::max(-126, std::min(126, top - 1 - std::ilogb(largest)));
 }
 
 PairW pair_pack(const float *w, int n, int k, const float *lnw, const float *lnb, float *out, hipStream_t stream) {

@@ -169,7 +169,7 @@ __device__ __forceinline__ void tail_chain(f32x4 (&x)[8], f32x4 (&s1)[8], Next &
         const f32x4 wi = lds4(sc + kTailOutInv + 16 * b + 4 * g);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            s1[b][e] = s1[b][e] + __builtin_fmaf(acc[b][e], wi[e] * a_inv, bo[e]);
+            s1[b][e] = s1[b][e] + __builtin_fmaf(acc[b][e] * wi[e], a_inv, bo[e]);
             sum += s1[b][e];
         }
     }
@@ -479,7 +479,7 @@ __device__ __forceinline__ void rows16_chain(const Tail128 &t, const f32x4 (&x)[
         const f32x4 bo = *reinterpret_cast<const f32x4 *>(t.bo + c0);
         const f32x4 wi = lds4(sc + kTailOutInv + c0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s1[j][e] = s1[j][e] + __builtin_fmaf(acc[j][e], wi[e] * a_inv, bo[e]);
+        for (int e = 0; e < 4; ++e) s1[j][e] = s1[j][e] + __builtin_fmaf(acc[j][e] * wi[e], a_inv, bo[e]);
         *reinterpret_cast<f32x4 *>(&s1s[m16 * kS1Stride + c0]) = s1[j];
     }
     __syncthreads();
@@ -846,12 +846,14 @@ void pack_pair(const float *w, int ld, int r0, int c0, const std::vector<int> &e
         }
 }
 
-std::vector<int> row_exponents(const float *w, int rows, int ld) {
+// The rows' exponents; `with` is that of the operand they multiply, whose sum
+// with each stays a float's.
+std::vector<int> row_exponents(const float *w, int rows, int ld, int with = 0) {
     std::vector<int> e(rows);
     for (int r = 0; r < rows; ++r) {
         float largest = 0.f;
         for (int i = 0; i < ld; ++i) largest = std::max(largest, std::fabs(w[(long long)r * ld + i]));
-        e[r] = pair_scale_exponent(largest, 14);
+        e[r] = std::max(-126 - with, std::min(126 - with, pair_scale_exponent(largest, 14)));
     }
     return e;
 }
@@ -867,8 +869,8 @@ int ln_exponent(const float *w, const float *b) {
 void head128_pack(const float *lnw, const float *lnb, const float *w, int outputs, float *out) {
     const int nb = outputs / 16;
     std::fill(out, out + head128_pack_floats(outputs), 0.f);
-    const std::vector<int> ew = row_exponents(w, outputs, 128);
     const int el = ln_exponent(lnw, lnb);
+    const std::vector<int> ew = row_exponents(w, outputs, 128, el);
     for (int kb = 0; kb < 4; ++kb)
         for (int ob = 0; ob < nb; ++ob)
             pack_pair(w, 128, 16 * ob, 32 * kb, ew, out + (size_t)(kb * nb + ob) * 512);
@@ -910,8 +912,9 @@ void tail128_pack(const float *wo, const float *n2w, const float *n2b, const flo
         }
         hidden = std::max(hidden, 11.5 * std::sqrt(norm) + std::fabs(bias));
     }
-    const std::vector<int> so = row_exponents(wo, 128, 128), s1 = row_exponents(w1, 256, 128), s2 = row_exponents(w2, 128, 256);
     const int el = ln_exponent(n2w, n2b), eh = pair_scale_exponent(hidden, 15);
+    const std::vector<int> so = row_exponents(wo, 128, 128), s1 = row_exponents(w1, 256, 128, el);
+    const std::vector<int> s2 = row_exponents(w2, 128, 256, eh);
     for (int kb = 0; kb < 4; ++kb)
         for (int ob = 0; ob < 8; ++ob) pack_pair(wo, 128, 16 * ob, 32 * kb, so, out + (kb * 8 + ob) * 512);
     for (int c = 0; c < 8; ++c) {

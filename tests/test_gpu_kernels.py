@@ -555,6 +555,30 @@ def test_block_tail_operand_ranges(device, fused, att_size, wo_size, ln_size, ff
     assert (np.abs(out.reshape(rows, 128) - want) / size).max() < 2.0 ** -19
 
 
+@pytest.mark.parametrize("fused", [1, 2])
+@pytest.mark.parametrize("att,wo,ln,w1,w2", [(-80, 80, 0, 0, 0), (80, -80, 0, 0, 0), (0, 0, -80, 80, 0),
+                                            (0, 0, 80, -80, 0), (0, 0, 0, 80, -80), (0, 0, 0, -80, 80)])
+def test_block_tail_weights_of_any_size(device, fused, att, wo, ln, w1, w2):
+    """Each product's operands 2^80 apart (as powers of two here): weights are
+    scaled by row over nearly all of FP32's range. 2^-18 of the result's
+    largest: the bounds above, over 256 hidden units of like size."""
+    rows = 70
+    def up(x, e):
+        return x * np.float32(2.0 ** e)
+    a, state = up(fast_values(rows * 128, 1), att), fast_values(rows * 128, 2, 3.0)
+    wo, bo = up(fast_values(128 * 128, 3, 0.09), wo), fast_values(128, 4, 0.1)
+    n2w, n2b = up(fast_values(128, 5, 0.2) + 1.0, ln), up(fast_values(128, 6, 0.1), ln)
+    w1, b1 = up(fast_values(256 * 128, 7, 0.09), w1), up(fast_values(256, 8, 0.1), ln + w1)
+    w2, b2 = up(fast_values(128 * 256, 9, 0.06), w2), fast_values(128, 10, 0.1)
+    out = np.zeros_like(state)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_block_tail(device.handle, fused, F(a), F(state), rows, F(wo), F(bo), F(n2w), F(n2b),
+                                            F(w1), F(b1), F(w2), F(b2), 1, F(out)))
+    want = block_tail64(a.reshape(rows, 128), state.reshape(rows, 128), wo.reshape(128, 128), bo, n2w, n2b,
+                        w1.reshape(256, 128), b1, w2.reshape(128, 256), b2)
+    assert np.abs(out.reshape(rows, 128) - want).max() < 2.0 ** -18 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("rows", [1, 16, 33, 1000])
 def test_block_tail_small_pass_form_equals_tail128(device, rows):
     """The 16-rows-per-workgroup tail takes every product in tail128's order:
@@ -716,6 +740,30 @@ def test_pair_linear_matches_float64(device, m, epilogue, k, n, norm):
     if epilogue == 2:
         want, size = want + res.reshape(m, n)[rows], size + np.abs(res.reshape(m, n)[rows])
     assert (np.abs(out.reshape(m, n)[rows] - want) / size).max() < 2.0 ** -20
+
+
+@pytest.mark.parametrize("m,k,norm", [(5, 512, False), (70, 1024, False), (5, 512, True), (1000, 512, True)])
+@pytest.mark.parametrize("octaves", [-80, 80])
+def test_pair_linear_weights_of_any_size(device, m, k, norm, octaves):
+    """Weights far below and above one against rows (or LayerNorm weights) far
+    above and below: the same products and bounds as at ordinary sizes."""
+    n = 64
+    x = fast_values(m * k, 1, 2.0).reshape(m, k)
+    lnw, lnb = fast_values(512, 2, 0.2) + 1.0, fast_values(512, 3, 0.1)
+    down = np.float32(2.0 ** -octaves)
+    if norm:
+        lnw, lnb = lnw * down, lnb * down
+    else:
+        x *= down
+    w, b = fast_values(n * k, 4, 0.05) * np.float32(2.0 ** octaves), fast_values(n, 5, 0.1)
+    out = np.zeros(m * n, np.float32)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_pair_linear(device.handle, 0, F(x), m, k, F(lnw) if norm else None,
+                                             F(lnb) if norm else None, F(w), F(b), n, None, F(out)))
+    a = ln64(x, lnw, lnb) if norm else x.astype(np.float64)
+    wt = w.reshape(n, k).T.astype(np.float64)
+    size = np.abs(a) @ np.abs(wt) + np.abs(b)
+    assert (np.abs(out.reshape(m, n) - (a @ wt + b)) / size).max() < 2.0 ** -20
 
 
 @pytest.mark.parametrize("form,estimators,rows", [(2, 1, 1), (2, 1, 2), (2, 1, 5), (2, 8, 1), (2, 4, 2), (2, 3, 3),
