@@ -417,13 +417,19 @@ int irx_test_pair_linear(irx_device *device, int epilogue, const float *x, size_
  * q * base[head] * (1 + tanh(gelu(q qm0w^T + qm0b) qm2w^T + qm2b)), into out
  * head-major [m / rows, 8, rows, 64] (StaticExecutor::qass, cpu.rs:3798-3853);
  * epilogue 3: the same result as the build computes it for many query rows
- * (LayerNorm, a tiled head-major Q projection, then the QASS MLP and gate
- * over the projected rows); epilogue 4: epilogue 2 with w as FP16 pairs, as
- * passes of more than 32 rows run it. */
+ * (LayerNorm, a head-major Q projection on FP16 pairs, then the QASS MLP and
+ * gate over the projected rows); epilogue 4: epilogue 2 (which takes w as FP16
+ * pairs from 33 rows). */
 int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t m, size_t rows,
                        const float *lnw, const float *lnb, const float *w, const float *b, size_t n,
                        const float *qm0w, const float *qm0b, const float *qm2w, const float *qm2b,
                        const float *base, float *out);
+/* K and V of an ICL block's normalized rows x [rows, 512] as the build projects
+ * them into a context of several estimators: w [1,536, 512] and b [1,536] are
+ * the block's whole in_proj, out [2, estimators, 8, rows, 64] the block's K and
+ * V planes, of which the named estimator's parts are written. */
+int irx_test_icl_kv(irx_device *device, const float *x, size_t rows, const float *w, const float *b,
+                    size_t estimators, size_t estimator, float *out);
 /* GELU, 0.5 x (1 + erf(x / sqrt 2)), of count floats as every kernel here
  * computes it (src/kernels/reference.rs:52-54). */
 int irx_test_gelu(irx_device *device, const float *x, size_t count, float *out);

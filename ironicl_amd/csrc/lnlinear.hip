@@ -455,11 +455,11 @@ void ln_linear512(const LnLinear &a, int epilogue, hipStream_t stream) {
             launch_rows<kLnGelu>(a, stream);
     } else if (epilogue == kLnQass && a.m <= 32) {
         hipLaunchKernelGGL((ln_linear512_kernel<kLnQass, 4, 8>), grid, dim3(512), 0, stream, a);
-    } else if (epilogue == kLnQass && a.pairs.pack) {
-        if (reinterpret_cast<uintptr_t>(a.pairs.pack) & 15) fail(3, "ln_linear512: pairs must be 16-byte aligned");
-        hipLaunchKernelGGL((ln_linear512_kernel<kLnQass, 4, 4, true>), grid, dim3(256), 0, stream, a);
     } else if (epilogue == kLnQass) {
-        hipLaunchKernelGGL(ln_linear512_kernel<kLnQass>, grid, dim3(256), 0, stream, a);
+        if (!a.pairs.pack || !a.pairs.row_inv ||
+            ((reinterpret_cast<uintptr_t>(a.pairs.pack) | reinterpret_cast<uintptr_t>(a.pairs.row_inv)) & 15))
+            fail(3, "ln_linear512: more than 32 rows need 16-byte aligned pairs");
+        hipLaunchKernelGGL((ln_linear512_kernel<kLnQass, 4, 4, true>), grid, dim3(256), 0, stream, a);
     } else if (a.m <= 32) {
         const dim3 narrow((unsigned)ceil_div((size_t)a.m, kRows), (unsigned)(a.n / 32));
         hipLaunchKernelGGL((ln_linear512_kernel<kLnGelu, 2>), narrow, dim3(256), 0, stream, a);

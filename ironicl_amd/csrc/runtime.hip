@@ -674,6 +674,43 @@ struct Stages {
         return r;
     }
 
+    // LN1, the Q projection and QASSMax of an ICL block's `b` x `rows` rows, into
+    // qg head-major [b, 8, rows, 64]: one launch (fused), else through `norm`
+    // (normed: already there) and the projected rows in qh.
+    void icl_query_rows(const BlockW &bw, const float *x, int b, int rows, const float *base, float *norm, float *qh,
+                        float *qg, bool normed, bool fused) const {
+        const long long m = (long long)b * rows;
+        if (fused) {
+            LnLinear f{};
+            f.x = x, f.ldx = 512, f.lnw = bw.n1w, f.lnb = bw.n1b, f.w = bw.in_w, f.b = bw.in_b, f.out = qg;
+            f.m = (int)m, f.n = 512, f.qm0w = bw.qm0.w, f.qm0b = bw.qm0.b, f.qm2w = bw.qm2.w, f.qm2b = bw.qm2.b;
+            f.base = base, f.rows = rows, f.pairs = bw.in_pairs;
+            ln_linear512(f, kLnQass, s);
+            return;
+        }
+        if (!normed) layer_norm(x, 512, bw.n1w, bw.n1b, norm, 512, m, 512, s);
+        // Q, head-major [b, 8, rows, 64].
+        OutMap qmap{64, kHeads, 0, (long long)rows * 64, rows, (long long)kHeads * rows * 64, 64};
+        linear_pairs(norm, 512, m, 512, bw.in_pairs, bw.in_b, 512, qh, qmap);
+        // QASSMax: q * base * (1 + tanh(MLP(q))) per head (reference.rs:417-428).
+        QassRows qa{};
+        qa.q = qh, qa.w0 = bw.qm0.w, qa.b0 = bw.qm0.b, qa.w2 = bw.qm2.w, qa.b2 = bw.qm2.b, qa.base = base;
+        qa.out = qg, qa.m = m * kHeads, qa.rows = rows, qa.compute_units = cus;
+        qass_rows(qa, s);
+    }
+
+    // K and V of an ICL block's n normalized rows, in two planes of head-major rows.
+    void icl_kv_rows(const BlockW &bw, const float *norm, int n, float *out, long long plane) const {
+        const OutMap map = OutMap::head_major(64, kHeads, n, plane);
+        if (n > kPairRows) {
+            PairW kv = bw.in_pairs;
+            kv.pack += (size_t)512 * 512, kv.row_inv += 512;  // past the query rows
+            linear_pairs(norm, 512, n, 512, kv, bw.in_b + 512, 1024, out, map);
+        } else {
+            linear_map(norm, 512, n, 512, bw.in_w + 512 * 512, bw.in_b + 512, 1024, out, map);
+        }
+    }
+
     // Query half of ICL block `blk` (cached_block with QASS, cpu.rs:2587-2850,
     // 3798-3853) for `b` estimators x `rows` query rows [b*rows, 512], against
     // K/V [b, 8, kv_rows, 64] (or the FP16 cache k16 / v16). normed: r.norm
@@ -684,24 +721,7 @@ struct Stages {
                      const unsigned short *v16 = nullptr, const Icl8Block *c8 = nullptr, bool normed = false) const {
         const BlockW &bw = w.icl[blk];
         const long long m = (long long)b * rows;
-        if (m <= kLnLinearRows) {
-            // LN1, Q projection and QASSMax in one launch, into qg head-major.
-            LnLinear f{};
-            f.x = x, f.ldx = 512, f.lnw = bw.n1w, f.lnb = bw.n1b, f.w = bw.in_w, f.b = bw.in_b, f.out = r.qg;
-            f.m = (int)m, f.n = 512, f.qm0w = bw.qm0.w, f.qm0b = bw.qm0.b, f.qm2w = bw.qm2.w, f.qm2b = bw.qm2.b;
-            f.base = base, f.rows = rows, f.pairs = bw.in_pairs;
-            ln_linear512(f, kLnQass, s);
-        } else {
-            if (!normed) layer_norm(x, 512, bw.n1w, bw.n1b, r.norm, 512, m, 512, s);
-            // Q, head-major [b, 8, rows, 64].
-            OutMap qmap{64, kHeads, 0, (long long)rows * 64, rows, (long long)kHeads * rows * 64, 64};
-            linear_pairs(r.norm, 512, m, 512, bw.in_pairs, bw.in_b, 512, r.qh, qmap);
-            // QASSMax: q * base * (1 + tanh(MLP(q))) per head (reference.rs:417-428).
-            QassRows qa{};
-            qa.q = r.qh, qa.w0 = bw.qm0.w, qa.b0 = bw.qm0.b, qa.w2 = bw.qm2.w, qa.b2 = bw.qm2.b, qa.base = base;
-            qa.out = r.qg, qa.m = m * kHeads, qa.rows = rows, qa.compute_units = cus;
-            qass_rows(qa, s);
-        }
+        icl_query_rows(bw, x, b, rows, base, r.norm, r.qh, r.qg, normed, m <= kLnLinearRows);
         IclAttention at{};
         at.q = r.qg, at.q_pair_stride = (long long)rows * 64, at.k = k, at.v = v;
         at.kv_pair_stride = (long long)kv_rows * 64, at.o = r.att, at.ldo = 512;
@@ -1215,22 +1235,12 @@ void build_impl(irx_weights *W, const irx_build_inputs *in, irx_build_outputs *o
         {
             Stages::IclBuffers ib = Stages::icl_buffers(ws, N, 1, N, N, cus, f16);
             float *kv32 = f16 ? ws.take((size_t)2 * kHeads * N * 64) : nullptr;
-            auto project_kv = [&](const BlockW &bw, const float *norm, float *out, const OutMap &map) {
-                if (N > kPairRows) {
-                    PairW kv = bw.in_pairs;
-                    kv.pack += (size_t)512 * 512, kv.row_inv += 512;  // past the query rows
-                    st.linear_pairs(norm, 512, N, 512, kv, bw.in_b + 512, 1024, out, map);
-                } else {
-                    st.linear_map(norm, 512, N, 512, bw.in_w + 512 * 512, bw.in_b + 512, 1024, out, map);
-                }
-            };
             for (int blk = 0; blk < kIclBlocks; ++blk) {
                 const BlockW &bw = W->icl[blk];
                 layer_norm(rows, 512, bw.n1w, bw.n1b, ib.norm, 512, N, 512, s);
                 if (!f16) {
                     float *kc = cache->icl[blk].f() + (long long)e * kHeads * N * 64;
-                    OutMap kvmap = OutMap::head_major(64, kHeads, N, icl_plane);
-                    project_kv(bw, ib.norm, kc, kvmap);
+                    st.icl_kv_rows(bw, ib.norm, N, kc, icl_plane);
                     // The last block's row states are never read: only its K/V are kept.
                     if (blk + 1 < kIclBlocks)
                         st.icl_queries(blk, rows, 1, N, kc, kc + icl_plane, N, d_base + blk * 512, ib, nullptr,
@@ -1238,8 +1248,7 @@ void build_impl(irx_weights *W, const irx_build_inputs *in, irx_build_outputs *o
                 } else {
                     // FP32 K/V of this estimator, then packed into its part of the FP16 cache.
                     const long long p32 = (long long)kHeads * N * 64;
-                    OutMap kvmap = OutMap::head_major(64, kHeads, N, p32);
-                    project_kv(bw, ib.norm, kv32, kvmap);
+                    st.icl_kv_rows(bw, ib.norm, N, kv32, p32);
                     unsigned short *k16 = static_cast<unsigned short *>(cache->icl[blk].p) + e * est16;
                     unsigned short *v16 = k16 + plane16;
                     pack_icl16(kv32, kv32 + p32, false, N, kHeads, k16, v16, counter, s);
@@ -2340,7 +2349,7 @@ int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t 
                        const float *lnb, const float *w, const float *b, size_t n, const float *qm0w,
                        const float *qm0b, const float *qm2w, const float *qm2b, const float *base, float *out) {
     return guarded("irx_test_ln_linear", [&] {
-        const bool tiled = epilogue == 3, pairs = epilogue == 4, qass = epilogue == kLnQass || tiled || pairs;
+        const bool tiled = epilogue == 3, qass = epilogue == kLnQass || tiled || epilogue == 4;
         if (!device || !x || !m || !lnw || !lnb || !w || !b || !out || (epilogue != kLnGelu && !qass) ||
             (qass && (n != 512 || !rows || m % rows || !qm0w || !qm0b || !qm2w || !qm2b || !base)) || !n || n % 64)
             fail(IRX_INVALID_ARGUMENT, "LN-linear arguments do not match");
@@ -2351,35 +2360,54 @@ int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t 
             return d;
         };
         DevBuf dx = up(x, m * 512), dlw = up(lnw, 512), dlb = up(lnb, 512), dw = up(w, n * 512), db = up(b, n);
-        DevBuf d0w, d0b, d2w, d2b, dbase;
-        if (qass) d0w = up(qm0w, 64 * 64), d0b = up(qm0b, 64), d2w = up(qm2w, 64 * 64), d2b = up(qm2b, 64), dbase = up(base, 512);
         DevBuf dout(m * n * 4);
-        LnLinear f{};
-        f.x = dx.f(), f.ldx = 512, f.lnw = dlw.f(), f.lnb = dlb.f(), f.w = dw.f(), f.b = db.f(), f.out = dout.f();
-        f.ldo = (long long)n, f.m = (int)m, f.n = (int)n;
-        if (qass) f.qm0w = d0w.f(), f.qm0b = d0b.f(), f.qm2w = d2w.f(), f.qm2b = d2b.f(), f.base = dbase.f(), f.rows = (int)rows;
-        DevBuf pack(pairs ? pair_pack_floats((int)n, 512) * 4 : 0);
-        if (pairs) f.pairs = pair_pack(dw.f(), (int)n, 512, lnw, lnb, pack.f(), nullptr);
-        if (tiled) {
-            // The build's form (Stages::icl_queries with more rows than the fused form takes).
-            DevBuf dnorm(m * 512 * 4), dq(m * 512 * 4);
-            layer_norm(dx.f(), 512, dlw.f(), dlb.f(), dnorm.f(), 512, (long long)m, 512, nullptr);
-            GemmArgs g{};
-            g.a = dnorm.f(), g.lda = 512, g.w = dw.f(), g.bias = db.f(), g.c = dq.f();
-            const long long hr = (long long)rows;
-            g.out = OutMap{64, kHeads, 0, hr * 64, (int)hr, (long long)kHeads * hr * 64, 64};
-            g.m = (int)m, g.n = 512, g.k = 512, g.epilogue = kEpiNone;
-            gemm(g, nullptr);
-            QassRows qa{};
-            qa.q = dq.f(), qa.w0 = d0w.f(), qa.b0 = d0b.f(), qa.w2 = d2w.f(), qa.b2 = d2b.f(), qa.base = dbase.f();
-            qa.out = dout.f(), qa.m = (long long)m * kHeads, qa.rows = (int)rows, qa.compute_units = device->compute_units;
-            qass_rows(qa, nullptr);
+        if (qass) {
+            DevBuf d0w = up(qm0w, 64 * 64), d0b = up(qm0b, 64), d2w = up(qm2w, 64 * 64), d2b = up(qm2b, 64);
+            DevBuf dbase = up(base, 512), pack(pair_pack_floats(512, 512) * 4);
+            DevBuf dnorm(tiled ? m * 512 * 4 : 0), dq(tiled ? m * 512 * 4 : 0);
+            BlockW bw{};
+            bw.dim = 512, bw.n1w = dlw.f(), bw.n1b = dlb.f(), bw.in_w = dw.f(), bw.in_b = db.f();
+            bw.in_pairs = pair_pack(dw.f(), 512, 512, lnw, lnb, pack.f(), nullptr);
+            bw.qm0 = {d0w.f(), d0b.f()}, bw.qm2 = {d2w.f(), d2b.f()};
+            irx_weights none;
+            Stages st{none, nullptr, device->compute_units};
+            st.icl_query_rows(bw, dx.f(), (int)(m / rows), (int)rows, dbase.f(), dnorm.f(), dq.f(), dout.f(), false,
+                              !tiled);
             IRX_HIP(hipDeviceSynchronize());
         } else {
-            ln_linear512(f, pairs ? kLnQass : epilogue, nullptr);
+            LnLinear f{};
+            f.x = dx.f(), f.ldx = 512, f.lnw = dlw.f(), f.lnb = dlb.f(), f.w = dw.f(), f.b = db.f(), f.out = dout.f();
+            f.ldo = (long long)n, f.m = (int)m, f.n = (int)n;
+            ln_linear512(f, kLnGelu, nullptr);
         }
         IRX_HIP(hipDeviceSynchronize());
         IRX_HIP(hipMemcpy(out, dout.p, m * n * 4, hipMemcpyDeviceToHost));
+    });
+}
+
+int irx_test_icl_kv(irx_device *device, const float *x, size_t rows, const float *w, const float *b,
+                    size_t estimators, size_t estimator, float *out) {
+    return guarded("irx_test_icl_kv", [&] {
+        if (!device || !x || !rows || !w || !b || !out || !estimators || estimator >= estimators ||
+            rows > (1u << 20) || estimators > 64)
+            fail(IRX_INVALID_ARGUMENT, "K/V projection arguments do not match");
+        set_device(device);
+        auto up = [](const float *h, size_t count) {
+            DevBuf d(count * 4);
+            IRX_HIP(hipMemcpy(d.p, h, count * 4, hipMemcpyHostToDevice));
+            return d;
+        };
+        const size_t part = rows * 512, plane = estimators * part;
+        DevBuf dx = up(x, part), dw = up(w, 1536 * 512), db = up(b, 1536), dout = up(out, 2 * plane);
+        DevBuf pack(pair_pack_floats(1536, 512) * 4);
+        BlockW bw{};
+        bw.dim = 512, bw.in_w = dw.f(), bw.in_b = db.f();
+        bw.in_pairs = pair_pack(dw.f(), 1536, 512, nullptr, nullptr, pack.f(), nullptr);
+        irx_weights none;
+        Stages st{none, nullptr, device->compute_units};
+        st.icl_kv_rows(bw, dx.f(), (int)rows, dout.f() + estimator * part, (long long)plane);
+        IRX_HIP(hipDeviceSynchronize());
+        IRX_HIP(hipMemcpy(out, dout.p, 2 * plane * 4, hipMemcpyDeviceToHost));
     });
 }
 

@@ -124,6 +124,7 @@ SIGNATURES = {
                                             _F]),
     "irx_test_ln_linear": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, _CF, _sz, _sz, _CF, _CF, _CF, _CF, _sz, _CF,
                                           _CF, _CF, _CF, _CF, _F]),
+    "irx_test_icl_kv": (ctypes.c_int, [ctypes.c_void_p, _CF, _sz, _CF, _CF, _sz, _sz, _F]),
     "irx_test_layer_norm": (ctypes.c_int, [ctypes.c_void_p, _CF, _CF, _CF, _sz, _sz, _F]),
     "irx_test_gelu": (ctypes.c_int, [ctypes.c_void_p, _CF, _sz, _F]),
     "irx_test_copy": (ctypes.c_int, [ctypes.c_void_p, _sz]),

@@ -772,9 +772,10 @@ def test_pair_linear_weights_of_any_size(device, m, k, norm, octaves):
                                                   (3, 1, 2049), (3, 3, 1001), (4, 1, 33), (4, 3, 17), (4, 2, 250)])
 def test_ln_linear_qass_matches_float64(device, form, estimators, rows):
     """LN1 + Q projection + QASSMax (query MLP and gate per head), head-major:
-    form 2 the prediction's fused kernel, form 3 the build's (LayerNorm, tiled
-    projection, then the MLP and gate over the projected rows, whose waves each
-    take a contiguous share of 16-row tasks; 3 x 1001 x 8 rows end mid-task)."""
+    forms 2 and 4 the prediction's fused kernels (FP16 pairs from 33 rows), form
+    3 the build's (LayerNorm, projection on FP16 pairs, then the MLP and gate
+    over the projected rows, whose waves each take a contiguous share of 16-row
+    tasks; 3 x 1001 x 8 rows end mid-task)."""
     m = estimators * rows
     x = fast_values(m * 512, 6, 3.0) - 0.1
     lnw, lnb = fast_values(512, 7, 0.2) + 1.0, fast_values(512, 8, 0.1)
@@ -792,6 +793,24 @@ def test_ln_linear_qass_matches_float64(device, form, estimators, rows):
     g = h @ m2w.reshape(64, 64).T.astype(np.float64) + m2b
     want = q * base.reshape(1, 8, 1, 64) * (1 + np.tanh(g))
     np.testing.assert_allclose(out.reshape(estimators, 8, rows, 64), want, rtol=1e-4, atol=2e-5)
+
+
+@pytest.mark.parametrize("rows", [1, 64, 65, 1000, 4097])
+@pytest.mark.parametrize("estimators,estimator", [(1, 0), (3, 1)])
+def test_icl_kv_matches_float64(device, rows, estimators, estimator):
+    """The build's K and V projection (FP16 pairs above 64 rows): the weights'
+    rows past the query's, into two planes of head-major rows of one estimator;
+    the other estimators' parts stay as they were."""
+    x = fast_values(rows * 512, 1, 2.0)
+    w, b = fast_values(1536 * 512, 2, 0.05), fast_values(1536, 3, 0.1)
+    out = np.full((2, estimators, 8, rows, 64), 7.0, np.float32)
+    F = hip.fptr
+    hip.check(hip.lib().irx_test_icl_kv(device.handle, F(x), rows, F(w), F(b), estimators, estimator, F(out)))
+    a, wt = x.reshape(rows, 512).astype(np.float64), w.reshape(1536, 512)[512:].T.astype(np.float64)
+    want = (a @ wt + b[512:]).reshape(rows, 2, 8, 64).transpose(1, 2, 0, 3)
+    size = (np.abs(a) @ np.abs(wt) + np.abs(b[512:])).reshape(rows, 2, 8, 64).transpose(1, 2, 0, 3)
+    assert (np.abs(out[:, estimator] - want) / size).max() < 2.0 ** -20
+    assert (np.delete(out, estimator, axis=1) == 7.0).all()
 
 
 def test_gelu_matches_float64(device):
