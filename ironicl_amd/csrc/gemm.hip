@@ -9,7 +9,7 @@
 // A is [M, K] activations, W is [N, K] in PyTorch Linear layout, so both
 // operands are K-contiguous.
 //
-// Two kernels, both on v_mfma_f32_32x32x2f32: tiled (BM x BN per workgroup,
+// Two kernels, both on v_mfma_f32_32x32x2f32: tiled (64 x 64 per workgroup,
 // 32-deep K steps through double-buffered LDS, one barrier per step, the next
 // step's global loads in flight during the MFMAs; LDS rows padded to 36
 // floats so a half-wave's 16-byte reads hit distinct banks) for products with
@@ -21,18 +21,13 @@
 // of M, whose A rows then stay in that XCD's L2 for all N tiles.
 #include "common.hpp"
 
-#include <atomic>
-
 namespace irx {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kBK = 32;
-// Workgroups per CU of the 128 x 128 tiles with 32-deep K steps (73.7 KB of
-// LDS) and with 16-deep ones (40 KB, 128 registers).
-constexpr long long kDeepPerCu = 2, kShallowPerCu = 4;
+constexpr int kTile = 64, kBK = 32;
 
 __device__ __forceinline__ long long col_offset(const OutMap &o, int n) {
     int seg = n / o.col_seg;
@@ -122,15 +117,21 @@ __device__ __forceinline__ void store_rows(const GemmArgs &p, int row0, int col,
     }
 }
 
-// Large products: a BM x BN tile per 256-thread workgroup (2 x 2 waves of
-// (BM/2) x (BN/2)), K in 32-deep steps through double-buffered LDS. Within a
+// Large products: a 64 x 64 tile per 256-thread workgroup (2 x 2 waves of
+// 32 x 32), K in 32-deep steps through double-buffered LDS. Within a
 // step lanes 0-31 feed k = 0..15 and lanes 32-63 k = 16..31, one k from each
 // half per MFMA, so a lane reads its 16 operands as four 16-byte LDS loads.
-template <int BM, int BN, int EPI, bool GROUPED, int BK = kBK>
-__global__ __launch_bounds__(256, BK == 16 ? 3 : 2) void gemm_kernel(GemmArgs p, int tiles_m, int tiles_n, int per_xcd) {
-    constexpr int MI = BM / 64, NI = BN / 64;
-    constexpr int STRIDE = BK + 4, KQ = BK / 8;  // LDS row floats; 16-byte operand loads per lane and block
-    constexpr int A_LOADS = BM * BK / 4 / 256, B_LOADS = BN * BK / 4 / 256;
+//
+// The products left to it are 128-deep (the inducing points' keys and values,
+// the CLS queries) or the decoder's last layer; 128 x 128 tiles gain nothing
+// there: 76,800 x 128 -> 256 60.5 us in 64 x 64 tiles, 66.5 in 128 x 128 ones and a
+// rest in 64 x 64, 262,144 x 128 -> 128 with a residual 105 (114), 16,384 x 1,024
+// -> 999 350 (347), 20,000 x 1,024 -> 999 431 (436).
+template <int EPI, bool GROUPED>
+__global__ __launch_bounds__(256, 2) void gemm_kernel(GemmArgs p, int tiles_m, int tiles_n, int per_xcd) {
+    constexpr int BM = kTile, BN = kTile, BK = kBK;
+    constexpr int STRIDE = BK + 4, KQ = BK / 8;  // LDS row floats; 16-byte operand loads per lane
+    constexpr int LOADS = BM * BK / 4 / 256;
     __shared__ __attribute__((aligned(16))) float As[2][BM * STRIDE];
     __shared__ __attribute__((aligned(16))) float Bs[2][BN * STRIDE];
 
@@ -144,43 +145,32 @@ __global__ __launch_bounds__(256, BK == 16 ? 3 : 2) void gemm_kernel(GemmArgs p,
     const int half = lane >> 5, r32 = lane & 31;
 
     // Global loads: thread t covers float4 (row = idx / 8, k4 = idx % 8), idx = t + 256 i.
-    const float *a_src[A_LOADS];
-    int a_lds[A_LOADS];
+    const float *a_src[LOADS], *b_src[LOADS];
+    int dst[LOADS];
 #pragma unroll
-    for (int i = 0; i < A_LOADS; ++i) {
+    for (int i = 0; i < LOADS; ++i) {
         int idx = tid + 256 * i, row = idx / (BK / 4), k4 = idx % (BK / 4);
         a_src[i] = p.a + (long long)min(m0 + row, p.m - 1) * p.lda + k4 * 4;
-        a_lds[i] = row * STRIDE + k4 * 4;
-    }
-    const float *b_src[B_LOADS];
-    int b_lds[B_LOADS];
-#pragma unroll
-    for (int i = 0; i < B_LOADS; ++i) {
-        int idx = tid + 256 * i, row = idx / (BK / 4), k4 = idx % (BK / 4);
         b_src[i] = p.w + (long long)min(n0 + row, p.n - 1) * p.k + k4 * 4;
-        b_lds[i] = row * STRIDE + k4 * 4;
+        dst[i] = row * STRIDE + k4 * 4;
     }
-    f32x4 a_reg[A_LOADS], b_reg[B_LOADS];
+    f32x4 a_reg[LOADS], b_reg[LOADS];
     auto load_tile = [&](int k0) {
 #pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) a_reg[i] = *reinterpret_cast<const f32x4 *>(a_src[i] + k0);
+        for (int i = 0; i < LOADS; ++i) a_reg[i] = *reinterpret_cast<const f32x4 *>(a_src[i] + k0);
 #pragma unroll
-        for (int i = 0; i < B_LOADS; ++i) b_reg[i] = *reinterpret_cast<const f32x4 *>(b_src[i] + k0);
+        for (int i = 0; i < LOADS; ++i) b_reg[i] = *reinterpret_cast<const f32x4 *>(b_src[i] + k0);
     };
     auto store_tile = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < A_LOADS; ++i) *reinterpret_cast<f32x4 *>(&As[buf][a_lds[i]]) = a_reg[i];
+        for (int i = 0; i < LOADS; ++i) *reinterpret_cast<f32x4 *>(&As[buf][dst[i]]) = a_reg[i];
 #pragma unroll
-        for (int i = 0; i < B_LOADS; ++i) *reinterpret_cast<f32x4 *>(&Bs[buf][b_lds[i]]) = b_reg[i];
+        for (int i = 0; i < LOADS; ++i) *reinterpret_cast<f32x4 *>(&Bs[buf][dst[i]]) = b_reg[i];
     };
 
-    f32x16 acc[MI][NI];
+    f32x16 acc;
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
 
     const int ktiles = p.k / BK;
     load_tile(0);
@@ -192,48 +182,30 @@ __global__ __launch_bounds__(256, BK == 16 ? 3 : 2) void gemm_kernel(GemmArgs p,
         const int buf = kt & 1;
         const bool more = kt + 1 < ktiles;
         if (more) load_tile((kt + 1) * BK);
-        f32x4 af[MI][KQ], bf[NI][KQ];
+        f32x4 af[KQ], bf[KQ];
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+        for (int c = 0; c < KQ; ++c) af[c] = *reinterpret_cast<const f32x4 *>(&As[buf][a_row + 4 * c]);
 #pragma unroll
-            for (int c = 0; c < KQ; ++c)
-                af[i][c] = *reinterpret_cast<const f32x4 *>(&As[buf][a_row + i * 32 * STRIDE + 4 * c]);
-#pragma unroll
-        for (int j = 0; j < NI; ++j)
-#pragma unroll
-            for (int c = 0; c < KQ; ++c)
-                bf[j][c] = *reinterpret_cast<const f32x4 *>(&Bs[buf][b_row + j * 32 * STRIDE + 4 * c]);
+        for (int c = 0; c < KQ; ++c) bf[c] = *reinterpret_cast<const f32x4 *>(&Bs[buf][b_row + 4 * c]);
 #pragma unroll
         for (int t = 0; t < 4 * KQ; ++t)
-#pragma unroll
-            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                for (int j = 0; j < NI; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][t >> 2][t & 3],
-                                                                     bf[j][t >> 2][t & 3], acc[i][j], 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(af[t >> 2][t & 3], bf[t >> 2][t & 3], acc, 0, 0, 0);
         if (more) store_tile(buf ^ 1);
         __syncthreads();
     }
 
     // Epilogue. Lane (r32, half) holds column r32 and rows half*4 + (r&3) + 8*(r>>2).
+    const int col = n0 + wn * (BN / 2) + r32, row0 = m0 + wm * (BM / 2) + half * 4;
+    if (col >= p.n) return;
+    const long long coff = col_offset(p.out, col);
+    const float bias = p.bias ? p.bias[col] : 0.f;
+    if constexpr (!GROUPED) {
+        store_rows<EPI>(p, row0, col, coff, bias, acc, m0 + BM <= p.m);
+    } else {
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-        const int col = n0 + wn * (BN / 2) + j * 32 + r32;
-        if (col >= p.n) continue;
-        const long long coff = col_offset(p.out, col);
-        const float bias = p.bias ? p.bias[col] : 0.f;
-#pragma unroll
-        for (int i = 0; i < MI; ++i) {
-            const int row0 = m0 + wm * (BM / 2) + i * 32 + half * 4;
-            if constexpr (!GROUPED) {
-                store_rows<EPI>(p, row0, col, coff, bias, acc[i][j], m0 + BM <= p.m);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = row0 + (r & 3) + 8 * (r >> 2);
-                    if (row < p.m) store_out<EPI, GROUPED>(p, row, col, coff, bias, acc[i][j][r]);
-                }
-            }
+        for (int r = 0; r < 16; ++r) {
+            const int row = row0 + (r & 3) + 8 * (r >> 2);
+            if (row < p.m) store_out<EPI, GROUPED>(p, row, col, coff, bias, acc[r]);
         }
     }
 }
@@ -466,25 +438,6 @@ __global__ __launch_bounds__(256) void gemm_rows_kernel(GemmArgs p) {
     }
 }
 
-// Compute units of the current device, looked up once per device ordinal.
-int device_compute_units() {
-    constexpr int kMaxDevices = 64;
-    static std::atomic<int> cached[kMaxDevices] = {};
-    int ordinal = 0;
-    if (hipGetDevice(&ordinal) != hipSuccess || ordinal < 0 || ordinal >= kMaxDevices) {
-        (void)hipGetLastError();
-        return 256;
-    }
-    int cus = cached[ordinal].load(std::memory_order_relaxed);
-    if (cus > 0) return cus;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ordinal) != hipSuccess || cus <= 0) {
-        (void)hipGetLastError();
-        return 256;
-    }
-    cached[ordinal].store(cus, std::memory_order_relaxed);
-    return cus;
-}
-
 struct Flops {
     double flops, bytes;
 };
@@ -518,12 +471,9 @@ void dispatch_epilogue(const GemmArgs &args, dim3 grid, hipStream_t stream, int 
     fail(3, "gemm: unknown epilogue");
 }
 
-template <int BM, int BN, int BK>
+template <int E, bool G>
 struct Tiled {
-    template <int E, bool G>
-    struct K {
-        static constexpr auto kernel = gemm_kernel<BM, BN, E, G, BK>;
-    };
+    static constexpr auto kernel = gemm_kernel<E, G>;
 };
 
 template <int E, bool G>
@@ -550,11 +500,10 @@ struct SplitK8 {
     };
 };
 
-template <int BM, int BN, int BK = kBK>
-void launch(const GemmArgs &args, hipStream_t stream) {
-    int tiles_m = (int)ceil_div(args.m, BM), tiles_n = (int)ceil_div(args.n, BN);
+void launch_tiled(const GemmArgs &args, hipStream_t stream) {
+    int tiles_m = (int)ceil_div(args.m, kTile), tiles_n = (int)ceil_div(args.n, kTile);
     int per_xcd = (tiles_m * tiles_n + 7) / 8;
-    dispatch_epilogue<Tiled<BM, BN, BK>::template K>(args, dim3(per_xcd * 8), stream, tiles_m, tiles_n, per_xcd);
+    dispatch_epilogue<Tiled>(args, dim3(per_xcd * 8), stream, tiles_m, tiles_n, per_xcd);
 }
 
 // gemm_rows_kernel for m <= 8 rows and K = 128, 256, 512 or 1,024 (plain
@@ -635,49 +584,11 @@ void gemm(const GemmArgs &args, hipStream_t stream) {
         fail(3, "gemm: K must be a positive multiple of 64 with 16-byte aligned rows");
     if (args.epilogue == kEpiResidual && !args.residual)
         fail(3, "gemm: residual epilogue without a residual");
-    // Products with few 64 x 64 tiles split K over a workgroup's waves; those
-    // with four or more 128 x 128 tiles per CU take them (GELU ones, whose
-    // epilogue is long, from two per CU), the rest 64 x 64 (measured on the
-    // prediction pass's products).
-    const long long big_tiles = (long long)ceil_div(args.m, 128) * ceil_div(args.n, 128);
+    // Products with few 64 x 64 tiles split K over a workgroup's waves.
     if (small_product(args.m, args.n)) {
         if (!launch_rows(args, stream)) launch_splitk(args, stream);
-    } else if (big_tiles >= 1024 || (args.epilogue == kEpiGelu && big_tiles >= 512)) {
-        // 128 x 128 tiles: 16-deep K steps (40 KB of LDS, 128 registers: four
-        // workgroups per CU) when there are at least two such rounds of
-        // tiles, else 32-deep steps at two per CU (the 50,000-row build's
-        // products: N = 1,024 and 1,536 take the first, N = 512 the second,
-        // whose 1,564 tiles are 1.5 rounds of four per CU). When the last
-        // round would be mostly empty (at N = 512: 3.05 rounds of two per CU)
-        // the whole rounds take the first rows and the rows left over run as
-        // 64 x 64 tiles, a quarter of the work each, spread over the chip.
-        const long long cus = device_compute_units();
-        const bool deep = big_tiles < 2 * kShallowPerCu * cus;
-        const long long slots = (deep ? kDeepPerCu : kShallowPerCu) * cus;
-        const long long tiles_n = ceil_div(args.n, 128);
-        const long long main_tm = big_tiles / slots * slots / tiles_n;
-        const bool plain_rows = args.out.rows_per_group >= args.m;
-        auto big = [&](const GemmArgs &a) {
-            if (deep)
-                launch<128, 128, 32>(a, stream);
-            else
-                launch<128, 128, 16>(a, stream);
-        };
-        if (plain_rows && big_tiles % slots < slots / 2 && main_tm > 0 && main_tm * 128 < args.m) {
-            GemmArgs head = args, rest = args;
-            const long long rows = main_tm * 128;
-            head.m = (int)rows;
-            rest.m = args.m - (int)rows;
-            rest.a = args.a + rows * args.lda;
-            rest.c = args.c + rows * args.out.ldc;
-            if (args.residual) rest.residual = args.residual + rows * args.ldr;
-            big(head);
-            launch<64, 64>(rest, stream);
-        } else {
-            big(args);
-        }
     } else {
-        launch<64, 64>(args, stream);
+        launch_tiled(args, stream);
     }
 }
 

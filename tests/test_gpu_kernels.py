@@ -72,11 +72,9 @@ def test_products_match_float64(device, m, n, k, n2):
 
 
 def test_large_products_with_a_split_last_round(device):
-    """70,000 rows: 2,188 tiles of 128 x 128 fill whole rounds on 256 CUs up to
-    row 65,536 (two rounds of four workgroups per CU, or four of two), so both
-    products (GELU, then residual) run those rows as 128 x 128 tiles and the
-    4,464 rows after them as 64 x 64 tiles. Rows on both sides of that
-    boundary and the last rows against float64."""
+    """70,000 rows: 1,094 x 8 tiles of 64 x 64, whose last row of tiles holds 48
+    rows (GELU, then residual), against float64 at both ends and on both sides
+    of row 65,536."""
     m, n, k = 70_000, 512, 512
     x = fast_values(m * k, 11)
     w1, b1 = fast_values(n * k, 12, 0.05), fast_values(n, 13)
