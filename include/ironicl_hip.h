@@ -418,8 +418,8 @@ int irx_test_pair_linear(irx_device *device, int epilogue, const float *x, size_
  * head-major [m / rows, 8, rows, 64] (StaticExecutor::qass, cpu.rs:3798-3853);
  * epilogue 3: the same result as the build computes it for many query rows
  * (LayerNorm, a head-major Q projection on FP16 pairs, then the QASS MLP and
- * gate over the projected rows); epilogue 4: epilogue 2 (which takes w as FP16
- * pairs from 33 rows). */
+ * gate over the projected rows); epilogue 4: epilogue 2. 1 and 2 take w as FP16
+ * pairs from nine rows. */
 int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t m, size_t rows,
                        const float *lnw, const float *lnb, const float *w, const float *b, size_t n,
                        const float *qm0w, const float *qm0b, const float *qm2w, const float *qm2b,

@@ -199,6 +199,17 @@ void gemm(const GemmArgs &args, hipStream_t stream);
 // m x n product with K = 128 and plain row-major output.
 bool gemm_fuses_ln(long long m, int n);
 
+// Rows up to which the ICL stage's and the decoder's 512-wide products run in
+// FP32, a column to 16 lanes; above they run on FP16 pairs, the LayerNorm in
+// the prologue. A cached prediction's whole call, against 1,024 x 54 and 10,000
+// x 100, in us: 4 rows 600 and 753 in FP32, 661 and 850 on pairs; 9 rows on FP32
+// MFMAs (the only other form) 746 / 898, on pairs 668 / 872; 16 rows 768 / 925 and
+// 680 / 890; 32 rows 830 / 1,016 and 733 / 960; 64 rows 910 / 1,138 and 811 /
+// 1,072. At 5 to 8 rows pairs are faster too (8 rows 762 / 929 and 668 / 868) but
+// less exact than these FP32 sums (logits 3.8e-7 from float64 against 3.4e-7; 16 to
+// 64 rows, against FP32 MFMAs: 4.2e-7 and 4.4e-7).
+constexpr int kFewRows = 8;
+
 // A weight matrix [n, k] packed as FP16 pairs (pair_pack, pairlinear.hip), each
 // row's inverse scale [n], and the scale of LayerNormed rows and its inverse.
 struct PairW {
@@ -325,7 +336,8 @@ void regression_summary(const RegressionSummary &s, hipStream_t stream);
 // epilogue(LN(x) W^T + b) over 512-wide rows x [m, 512] (W [n, 512]), the
 // LayerNorm in the product's prologue: kLnGelu writes gelu() row-major [m, n];
 // kLnQass (n = 512) runs each head's QASS query MLP and gate and writes
-// head-major [m / rows, 8, rows, 64]. For prediction-sized m.
+// head-major [m / rows, 8, rows, 64]. For prediction-sized m, kLnGelu for at
+// most kFewRows.
 enum LnEpilogue : int { kLnGelu = 1, kLnQass = 2 };
 struct LnLinear {
     const float *x;
@@ -338,9 +350,7 @@ struct LnLinear {
     const float *qm0w, *qm0b, *qm2w, *qm2b;  // kLnQass: [64, 64], [64] each
     const float *base;                       // kLnQass: [8, 64]
     int rows;                                // kLnQass: rows per estimator
-    // kLnQass, more than 32 rows: w as FP16 pairs with its LayerNorm scale
-    // (pack null: FP32 products).
-    PairW pairs;
+    PairW pairs;                             // kLnQass, more than kFewRows: w as FP16 pairs
 };
 void ln_linear512(const LnLinear &a, int epilogue, hipStream_t stream);
 

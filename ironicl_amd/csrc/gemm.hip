@@ -3,9 +3,9 @@
 // The dense layers of the model (the role of linear64 / linear_reduce in the
 // reference's CUDA backend, src/kernels/cuda/kernels.rs:290-470) that no fused
 // kernel takes (tail.hip, lnlinear.hip) and that do not run on FP16 pairs
-// (pairlinear.hip: the ICL stage's above 64 rows): the 128-wide products of
-// small passes, the inducing points' keys and values, small ICL products, the
-// decoder's last layer.
+// (pairlinear.hip: the ICL stage's above kFewRows rows): the 128-wide products
+// of small passes, the inducing points' keys and values, the ICL products of
+// passes of few rows, the decoder's last layer.
 // A is [M, K] activations, W is [N, K] in PyTorch Linear layout, so both
 // operands are K-contiguous.
 //
@@ -313,15 +313,15 @@ __global__ __launch_bounds__(256) void gemm_splitk_kernel(GemmArgs p, int tiles_
     }
 }
 
-// Small products with K = 512 or 1,024 and a few dozen rows (the 512-wide
-// out-projection and FFN down of passes of 9-64 rows): the split-K tile over
-// eight waves, each taking an eighth of K with all of its operand loads
-// issued before the first product, so a tile costs one memory round trip
-// rather than one per 16-deep step (the four-wave kernel's 8-16 dependent
-// steps). Each wave finishes two of the
+// Small products with K = 1,024 and a few dozen rows (the decoder's last layer
+// in passes of 9-64 rows): the split-K tile over eight waves, each taking an
+// eighth of K with all of its operand loads issued before the first product, so
+// a tile costs one memory round trip rather than one per 16-deep step (the
+// four-wave kernel's 8-16 dependent steps). Each wave finishes two of the
 // sixteen accumulator registers: rows (2w % 4) + 8 (w / 2) + 4 half + rr.
-template <int EPI, bool GROUPED, int KW>  // KW: K per wave
+template <int EPI, bool GROUPED>
 __global__ __launch_bounds__(512) void gemm_splitk8_kernel(GemmArgs p, int tiles_m, int tiles_n, int per_xcd) {
+    constexpr int KW = 128;  // K per wave
     constexpr int S = KW / 16;
     __shared__ float red[8][16][64];
     const int bid = blockIdx.x;
@@ -486,18 +486,14 @@ struct SplitKLn {
     static constexpr auto kernel = gemm_splitk_kernel<E, G, true>;
 };
 
-// Rows up to which K = 512 and 1,024 products take the eight-wave split-K:
-// passes of a few dozen rows gain (16-row pass 1.29 -> 1.27 ms), but beside
-// the other stream's attention a 512-row pass's 512-thread, 150-register
-// workgroups cost more than they save (the two-stream step 43.8 -> 46.5 ms).
+// Rows up to which K = 1,024 products take the eight-wave split-K: beside the
+// other stream's attention a 512-row pass's 512-thread, 150-register
+// workgroups cost more than they save.
 constexpr int kSplitK8Rows = 64;
 
-template <int KW>
+template <int E, bool G>
 struct SplitK8 {
-    template <int E, bool G>
-    struct K {
-        static constexpr auto kernel = gemm_splitk8_kernel<E, G, KW>;
-    };
+    static constexpr auto kernel = gemm_splitk8_kernel<E, G>;
 };
 
 void launch_tiled(const GemmArgs &args, hipStream_t stream) {
@@ -557,10 +553,8 @@ void launch_splitk(const GemmArgs &args, hipStream_t stream) {
     int per_xcd = (tiles_m * tiles_n + 7) / 8;
     if (args.ln_w)
         dispatch_epilogue<SplitKLn>(args, dim3(per_xcd * 8), stream, tiles_m, tiles_n, per_xcd);
-    else if (args.m <= kSplitK8Rows && args.k == 512)
-        dispatch_epilogue<SplitK8<64>::template K>(args, dim3(per_xcd * 8), stream, tiles_m, tiles_n, per_xcd, 512);
     else if (args.m <= kSplitK8Rows && args.k == 1024)
-        dispatch_epilogue<SplitK8<128>::template K>(args, dim3(per_xcd * 8), stream, tiles_m, tiles_n, per_xcd, 512);
+        dispatch_epilogue<SplitK8>(args, dim3(per_xcd * 8), stream, tiles_m, tiles_n, per_xcd, 512);
     else
         dispatch_epilogue<SplitK>(args, dim3(per_xcd * 8), stream, tiles_m, tiles_n, per_xcd);
 }

@@ -12,17 +12,18 @@
 //            cpu.rs:3798-3853; qassmax_f32, reference.rs:417-428).
 // It replaces, per ICL block of a prediction pass, LayerNorm + Q projection +
 // two QASS products (four launches), and LayerNorm + FFN up (two launches).
-// Passes of at most eight rows take ln_rows512_kernel instead.
+// Passes of at most kFewRows rows take ln_rows512_kernel, larger ones the
+// 16-row kernel below for kLnQass and pair_linear for the rest.
 //
-// A workgroup of four waves computes 16 rows x 64 columns; wave w reduces over
-// K = 128 w .. 128 w + 127 on v_mfma_f32_16x16x4f32 with the product
+// In the 16-row kernel a workgroup of four waves computes 16 rows x one head's
+// 64 columns on FP16 pairs (common.hpp); wave w reduces over
+// K = 128 w .. 128 w + 127 on v_mfma_f32_16x16x32_f16 with the product
 // transposed (D = W x^T: lane (m, g) = (lane % 16, lane / 16) holds row m's
 // columns 16 b + 4 g + r in register r of block b). Each wave loads its rows'
-// quarter of x in that layout, the row statistics are summed over the four
-// waves through LDS, and the partial products are summed there too. The query
-// projection of passes of more than 32 rows multiplies FP16 pairs (PAIRS,
-// common.hpp; pair_pack's fragments have x's layout as their slots): 48 products
-// of 16 cycles a wave instead of 128 of 32.
+// quarter of x in that layout (pair_pack's fragments have it as their slots),
+// the row statistics are summed over the four waves through LDS, and the
+// partial products are summed there too. FP32 products took 128 MFMAs of 32
+// cycles a wave, pairs take 48 of 16.
 #include "common.hpp"
 
 #include <algorithm>
@@ -38,29 +39,17 @@ __device__ __forceinline__ f32x4 mfma(float a, float b, const f32x4 &acc) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0);
 }
 
-// Sum of a[0..W-1] as a pairwise tree ((a0 + a1) + (a2 + a3)) + ...
-template <int W, typename F>
+// Sum of a(0) .. a(3) as a pairwise tree.
+template <typename F>
 __device__ __forceinline__ auto tree_sum(F a) {
-    if constexpr (W == 4)
-        return (a(0) + a(1)) + (a(2) + a(3));
-    else
-        return ((a(0) + a(1)) + (a(2) + a(3))) + ((a(4) + a(5)) + (a(6) + a(7)));
+    return (a(0) + a(1)) + (a(2) + a(3));
 }
 
-// OB: 16-column output blocks per workgroup (4, or 2 for the GELU form of
-// passes of at most 32 rows, which then spread over twice the workgroups).
-// W: waves, each taking 512 / W of K (8 for the QASS form of passes of at
-// most 32 rows: half the products and weight loads per wave; waves 4-7 then
-// only pass the barriers of the epilogue).
-template <int EPI, int OB = 4, int W = 4, bool PAIRS = false>
-__global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
-    static_assert(OB == 4 || (OB == 2 && EPI == kLnGelu), "QASS needs a whole 64-wide head per workgroup");
-    static_assert(W == 4 || W == 8, "four or eight waves");
-    static_assert(!PAIRS || (OB == 4 && W == 4), "pairs: the 16 x 64 form");
-    constexpr int KB = 32 / W;  // 16-wide k-blocks per wave
-    __shared__ float red[2][W][kRows];
-    __shared__ __attribute__((aligned(16))) float part[W][kRows][68];
-    __shared__ __attribute__((aligned(16))) float tile[2][kRows][68];  // QASS: q, then the hidden layer
+__global__ __launch_bounds__(256) void ln_qass512_kernel(LnLinear p) {
+    constexpr int KB = 8, OB = 4;  // a wave's 16-wide k-blocks; 16-column output blocks
+    __shared__ float red[2][4][kRows];
+    __shared__ __attribute__((aligned(16))) float part[4][kRows][68];
+    __shared__ __attribute__((aligned(16))) float tile[2][kRows][68];  // q, then the hidden layer
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int m16 = lane & 15, g = lane >> 4;
     const long long row0 = (long long)blockIdx.x * kRows;
@@ -72,27 +61,19 @@ __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
     // x[row][k0 + 16 kb + 4 g + e], and every weight fragment of this wave's
     // quarter up front (columns col0 + 16 ob + lane % 16): the loads' latency
     // is paid once, under the LayerNorm.
-    f32x4 x[KB], wf[PAIRS ? 1 : KB][OB];
-    u32x4 wp[PAIRS ? KB / 2 : 1][OB][2];  // hi, lo of 32-deep step kb
+    f32x4 x[KB];
+    u32x4 wp[KB / 2][OB][2];  // hi, lo of 32-deep step kb
     const float *xr = p.x + r * p.ldx + k0 + 4 * g;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) x[kb] = *reinterpret_cast<const f32x4 *>(xr + 16 * kb);
-    if constexpr (PAIRS) {
-        const float *pk = p.pairs.pack + ((size_t)(col0 / 16) * 16 + (KB / 2) * w) * 512 + lane * 4;
+    const float *pk = p.pairs.pack + ((size_t)(col0 / 16) * 16 + (KB / 2) * w) * 512 + lane * 4;
 #pragma unroll
-        for (int kb = 0; kb < KB / 2; ++kb)
+    for (int kb = 0; kb < KB / 2; ++kb)
 #pragma unroll
-            for (int ob = 0; ob < OB; ++ob)
+        for (int ob = 0; ob < OB; ++ob)
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    wp[kb][ob][h] = *reinterpret_cast<const u32x4 *>(pk + ((size_t)ob * 16 + kb) * 512 + h * 256);
-    } else {
-        const float *wr = p.w + (long long)(col0 + m16) * 512 + k0 + 4 * g;
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-            for (int ob = 0; ob < OB; ++ob) wf[kb][ob] = *reinterpret_cast<const f32x4 *>(wr + ob * 16 * 512 + 16 * kb);
-    }
+            for (int h = 0; h < 2; ++h)
+                wp[kb][ob][h] = *reinterpret_cast<const u32x4 *>(pk + ((size_t)ob * 16 + kb) * 512 + h * 256);
     float s = 0.f;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) s += (x[kb][0] + x[kb][1]) + (x[kb][2] + x[kb][3]);
@@ -100,7 +81,7 @@ __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
     s += __shfl_xor(s, 32, 64);
     if (g == 0) red[0][w][m16] = s;
     __syncthreads();
-    const float mean = tree_sum<W>([&](int i) { return red[0][i][m16]; }) / 512.f;
+    const float mean = tree_sum([&](int i) { return red[0][i][m16]; }) / 512.f;
     float sq = 0.f;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb)
@@ -113,7 +94,7 @@ __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
     sq += __shfl_xor(sq, 32, 64);
     if (g == 0) red[1][w][m16] = sq;
     __syncthreads();
-    const float var = tree_sum<W>([&](int i) { return red[1][i][m16]; }) / 512.f;
+    const float var = tree_sum([&](int i) { return red[1][i][m16]; }) / 512.f;
     const float rstd = 1.0f / sqrtf(var + 1e-5f);
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
@@ -127,98 +108,71 @@ __global__ __launch_bounds__(64 * W) void ln_linear512_kernel(LnLinear p) {
     f32x4 acc[OB];
 #pragma unroll
     for (int ob = 0; ob < OB; ++ob) acc[ob] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (PAIRS) {
 #pragma unroll
-        for (int kb = 0; kb < KB / 2; ++kb) {
-            float y[8];
+    for (int kb = 0; kb < KB / 2; ++kb) {
+        float y[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) y[e] = x[2 * kb + (e >> 2)][e & 3] * p.pairs.ln_scale;
-            half8 xh, xl;
-            pair8(y, xh, xl);
+        for (int e = 0; e < 8; ++e) y[e] = x[2 * kb + (e >> 2)][e & 3] * p.pairs.ln_scale;
+        half8 xh, xl;
+        pair8(y, xh, xl);
 #pragma unroll
-            for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][1]), xh, acc[ob], 0, 0, 0);
+        for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][1]), xh, acc[ob], 0, 0, 0);
 #pragma unroll
-            for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][0]), xl, acc[ob], 0, 0, 0);
+        for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][0]), xl, acc[ob], 0, 0, 0);
 #pragma unroll
-            for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][0]), xh, acc[ob], 0, 0, 0);
-        }
-#pragma unroll
-        for (int ob = 0; ob < OB; ++ob)
-            acc[ob] = acc[ob] * *reinterpret_cast<const f32x4 *>(p.pairs.row_inv + col0 + 16 * ob + 4 * g) * p.pairs.ln_inv;
-    } else {
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int ob = 0; ob < OB; ++ob) acc[ob] = mfma(wf[kb][ob][e], x[kb][e], acc[ob]);
+        for (int ob = 0; ob < OB; ++ob) acc[ob] = __builtin_amdgcn_mfma_f32_16x16x32_f16(as_half8(wp[kb][ob][0]), xh, acc[ob], 0, 0, 0);
     }
+#pragma unroll
+    for (int ob = 0; ob < OB; ++ob)
+        acc[ob] = acc[ob] * *reinterpret_cast<const f32x4 *>(p.pairs.row_inv + col0 + 16 * ob + 4 * g) * p.pairs.ln_inv;
 #pragma unroll
     for (int ob = 0; ob < OB; ++ob)
         *reinterpret_cast<f32x4 *>(&part[w][m16][16 * ob + 4 * g]) = acc[ob];
     __syncthreads();
 
-    // Threads 0-255 finish row t / 16, columns 4 (t % 16) .. +3.
-    const int om = (tid >> 4) & (kRows - 1), oc = 4 * (tid & 15);
-    const bool finisher = tid < 16 * kRows;
-    const long long orow = row0 + om;
-    if (oc >= 16 * OB) return;  // OB = 2: only the GELU form, which has no barrier after this
-    f32x4 v = tree_sum<W>([&](int i) { return *reinterpret_cast<const f32x4 *>(&part[i][om][oc]); });
+    // Thread t finishes row t / 16, columns 4 (t % 16) .. +3.
+    const int om = tid >> 4, oc = 4 * (tid & 15);
+    f32x4 v = tree_sum([&](int i) { return *reinterpret_cast<const f32x4 *>(&part[i][om][oc]); });
     v += *reinterpret_cast<const f32x4 *>(p.b + col0 + oc);
-    if constexpr (EPI == kLnGelu) {
-        if (finisher && orow < p.m) {
+    // The head's query tile, then its MLP: wave w computes columns
+    // 16 w .. 16 w + 15 of each layer from the whole previous tile.
+    f32x4 mw[2][4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = gelu_erf(v[e]);
-            *reinterpret_cast<f32x4 *>(p.out + orow * p.ldo + col0 + oc) = v;
-        }
-    } else {
-        // The head's query tile, then its MLP: wave w < 4 computes columns
-        // 16 w .. 16 w + 15 of each layer from the whole previous tile (with
-        // eight waves, waves 4-7 only pass the barriers).
-        const bool mlp = w < 4;
-        const int wq = w & 3;
-        f32x4 mw[2][4];
+    for (int kb = 0; kb < 4; ++kb) {
+        mw[0][kb] = *reinterpret_cast<const f32x4 *>(p.qm0w + (16 * w + m16) * 64 + 16 * kb + 4 * g);
+        mw[1][kb] = *reinterpret_cast<const f32x4 *>(p.qm2w + (16 * w + m16) * 64 + 16 * kb + 4 * g);
+    }
+    *reinterpret_cast<f32x4 *>(&tile[0][om][oc]) = v;
+    __syncthreads();
+    auto layer = [&](const f32x4 *wt, const float *bias, int src) {
+        f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kb = 0; kb < 4; ++kb) {
-            mw[0][kb] = *reinterpret_cast<const f32x4 *>(p.qm0w + (16 * wq + m16) * 64 + 16 * kb + 4 * g);
-            mw[1][kb] = *reinterpret_cast<const f32x4 *>(p.qm2w + (16 * wq + m16) * 64 + 16 * kb + 4 * g);
+            const f32x4 xf = *reinterpret_cast<const f32x4 *>(&tile[src][m16][16 * kb + 4 * g]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a = mfma(wt[kb][e], xf[e], a);
         }
-        if (finisher) *reinterpret_cast<f32x4 *>(&tile[0][om][oc]) = v;
-        __syncthreads();
-        auto layer = [&](const f32x4 *wt, const float *bias, int src) {
-            f32x4 a = f32x4{0.f, 0.f, 0.f, 0.f};
+        return a + *reinterpret_cast<const f32x4 *>(bias + 16 * w + 4 * g);
+    };
+    f32x4 h = layer(mw[0], p.qm0b, 0);
 #pragma unroll
-            for (int kb = 0; kb < 4; ++kb) {
-                const f32x4 xf = *reinterpret_cast<const f32x4 *>(&tile[src][m16][16 * kb + 4 * g]);
+    for (int e = 0; e < 4; ++e) h[e] = gelu_erf(h[e]);
+    *reinterpret_cast<f32x4 *>(&tile[1][m16][16 * w + 4 * g]) = h;
+    __syncthreads();
+    if (row >= p.m) return;
+    const f32x4 gm = layer(mw[1], p.qm2b, 1);
+    const int head = blockIdx.y, col = 16 * w + 4 * g;
+    const f32x4 q = *reinterpret_cast<const f32x4 *>(&tile[0][m16][col]);
+    const f32x4 base = *reinterpret_cast<const f32x4 *>(p.base + head * 64 + col);
+    f32x4 o;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) a = mfma(wt[kb][e], xf[e], a);
-            }
-            return a + *reinterpret_cast<const f32x4 *>(bias + 16 * wq + 4 * g);
-        };
-        if (mlp) {
-            f32x4 h = layer(mw[0], p.qm0b, 0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = gelu_erf(h[e]);
-            *reinterpret_cast<f32x4 *>(&tile[1][m16][16 * wq + 4 * g]) = h;
-        }
-        __syncthreads();
-        if (mlp && row < p.m) {
-            const f32x4 gm = layer(mw[1], p.qm2b, 1);
-            const int head = blockIdx.y, col = 16 * wq + 4 * g;
-            const f32x4 q = *reinterpret_cast<const f32x4 *>(&tile[0][m16][col]);
-            const f32x4 base = *reinterpret_cast<const f32x4 *>(p.base + head * 64 + col);
-            f32x4 o;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = q[e] * base[e] * (1.0f + tanhf(gm[e]));
-            const long long b = row / p.rows, rr = row - b * p.rows;
-            *reinterpret_cast<f32x4 *>(p.out + (((b * kHeads + head) * p.rows + rr) * 64) + col) = o;
-        }
-    }
+    for (int e = 0; e < 4; ++e) o[e] = q[e] * base[e] * (1.0f + tanhf(gm[e]));
+    const long long b = row / p.rows, rr = row - b * p.rows;
+    *reinterpret_cast<f32x4 *>(p.out + (((b * kHeads + head) * p.rows + rr) * 64) + col) = o;
 }
 
-// Passes of at most eight rows (M = 1, 2, 4 or 8 after rounding up). The
-// 16-row MFMA tiles above would spend 128 serial MFMAs per wave on one or two
-// real rows; here every weight load is issued first, the rows' LayerNorms
+// Passes of at most kFewRows rows (M = 1, 2, 4 or 8 after rounding up): FP32 on
+// the VALU. Every weight load is issued first, the rows' LayerNorms
 // are taken under those loads (row r by wave r % waves, two-pass statistics
 // over a wave's 64 lanes) and staged in LDS, and each 16-lane group owns one
 // output column: lane i multiplies K floats 64 j + 4 i .. 64 j + 4 i + 3 and
@@ -447,24 +401,17 @@ void ln_linear512(const LnLinear &a, int epilogue, hipStream_t stream) {
     const double m = a.m, n = a.n;
     const double flops = 2.0 * m * n * 512 + (epilogue == kLnQass ? 2.0 * 2.0 * m * 8 * 64 * 64 : 0.0);
     KernelTimer timer(kFamGemm, stream, flops, 4.0 * (m * 512 + n * 512 + m * n));
-    const dim3 grid((unsigned)ceil_div((size_t)a.m, kRows), (unsigned)(a.n / 64));
-    if (a.m <= 8) {
+    if (a.m <= kFewRows) {
         if (epilogue == kLnQass)
             launch_rows<kLnQass>(a, stream);
         else
             launch_rows<kLnGelu>(a, stream);
-    } else if (epilogue == kLnQass && a.m <= 32) {
-        hipLaunchKernelGGL((ln_linear512_kernel<kLnQass, 4, 8>), grid, dim3(512), 0, stream, a);
-    } else if (epilogue == kLnQass) {
-        if (!a.pairs.pack || !a.pairs.row_inv ||
-            ((reinterpret_cast<uintptr_t>(a.pairs.pack) | reinterpret_cast<uintptr_t>(a.pairs.row_inv)) & 15))
-            fail(3, "ln_linear512: more than 32 rows need 16-byte aligned pairs");
-        hipLaunchKernelGGL((ln_linear512_kernel<kLnQass, 4, 4, true>), grid, dim3(256), 0, stream, a);
-    } else if (a.m <= 32) {
-        const dim3 narrow((unsigned)ceil_div((size_t)a.m, kRows), (unsigned)(a.n / 32));
-        hipLaunchKernelGGL((ln_linear512_kernel<kLnGelu, 2>), narrow, dim3(256), 0, stream, a);
     } else {
-        hipLaunchKernelGGL(ln_linear512_kernel<kLnGelu>, grid, dim3(256), 0, stream, a);
+        if (epilogue != kLnQass || !a.pairs.pack || !a.pairs.row_inv ||
+            ((reinterpret_cast<uintptr_t>(a.pairs.pack) | reinterpret_cast<uintptr_t>(a.pairs.row_inv)) & 15))
+            fail(3, "ln_linear512: larger products need the QASS epilogue and 16-byte aligned pairs");
+        const dim3 grid((unsigned)ceil_div((size_t)a.m, kRows), kHeads);
+        hipLaunchKernelGGL(ln_qass512_kernel, grid, dim3(256), 0, stream, a);
     }
     IRX_HIP(hipGetLastError());
 }

@@ -445,12 +445,6 @@ void set_device(const irx_device *d) { IRX_HIP(hipSetDevice(d->ordinal)); }
 // launch (prediction passes); larger ones (the build's N rows) take the
 // LayerNorm that the K/V projection shares and separate products.
 constexpr long long kLnLinearRows = 8192;
-// Rows above which the other 512-wide products run on FP16 pairs
-// (pair_linear): per 512-row pass the out-projection, FFN and decoder products
-// they replace took 12-21 us each on FP32 MFMAs; 1,024 rows against 10,000 x
-// 100 at auto went from 2.53 to 2.30 ms, the 10,000 x 100 fit from 41.2 to 39.8.
-// Smaller passes are bound by reading each weight once, not by products.
-constexpr long long kPairRows = 64;
 // States (columns x rows) from which a cached column block runs as one
 // kernel of 64-row tiles (column_block) rather than its small-pass form of
 // 16 rows per workgroup. Measured per block at 64 columns (the three
@@ -482,6 +476,19 @@ struct Stages {
         g.x = a, g.ldx = lda, g.lnw = lnw, g.lnb = lnb, g.w = wt, g.bias = b, g.residual = res, g.ldr = ldr, g.c = c;
         g.out = map, g.m = (int)m, g.n = n, g.k = k, g.epilogue = epi;
         pair_linear(g, s);
+    }
+
+    // gelu(LN(x) W^T + b) of 512-wide rows into out [m, n].
+    void ln_gelu512(const float *x, long long m, const float *lnw, const float *lnb, const Lin &l, int n,
+                    float *out) const {
+        if (m > kFewRows) {
+            linear_pairs(x, 512, m, 512, l.pairs, l.b, n, out, OutMap::row_major(n, n), kEpiGelu, nullptr, 0, lnw, lnb);
+            return;
+        }
+        LnLinear f{};
+        f.x = x, f.ldx = 512, f.lnw = lnw, f.lnb = lnb, f.w = l.w, f.b = l.b, f.out = out, f.ldo = n;
+        f.m = (int)m, f.n = n;
+        ln_linear512(f, kLnGelu, s);
     }
 
     // LayerNorm of 128-wide rows x [m, 128] and the product that reads it:
@@ -537,22 +544,19 @@ struct Stages {
         const bool packed = d == 128 && bw.tail_pack;
         const bool use_fused = fused < 0 ? packed : fused >= 1;
         const bool rows16 = fused < 0 ? m < 16384 : fused == 2;
-        if (d == 512 && m > kPairRows) {
-            const OutMap rows = OutMap::row_major(d, d);
-            linear_pairs(att, d, m, d, bw.out.pairs, bw.out.b, d, state, rows, kEpiResidual, state, d);
-            linear_pairs(state, d, m, d, bw.l1.pairs, bw.l1.b, 2 * d, hid, OutMap::row_major(2 * d, 2 * d), kEpiGelu,
-                         nullptr, 0, bw.n2w, bw.n2b);
-            linear_pairs(hid, 2 * d, m, 2 * d, bw.l2.pairs, bw.l2.b, d, state, rows, kEpiResidual, state, d);
-            return;
-        }
         if (d == 512) {
-            // Small 512-wide blocks: LN2 fused into the FFN's first product.
-            linear(att, d, m, d, bw.out.w, bw.out.b, d, state, d, kEpiResidual, state, d);
-            LnLinear f{};
-            f.x = state, f.ldx = d, f.lnw = bw.n2w, f.lnb = bw.n2b, f.w = bw.l1.w, f.b = bw.l1.b, f.out = hid;
-            f.ldo = 2 * d, f.m = (int)m, f.n = 2 * d;
-            ln_linear512(f, kLnGelu, s);
-            linear(hid, 2 * d, m, 2 * d, bw.l2.w, bw.l2.b, d, state, d, kEpiResidual, state, d);
+            // LN2 fused into the FFN's first product.
+            const OutMap rows = OutMap::row_major(d, d);
+            const bool few = m <= kFewRows;
+            if (few)
+                linear(att, d, m, d, bw.out.w, bw.out.b, d, state, d, kEpiResidual, state, d);
+            else
+                linear_pairs(att, d, m, d, bw.out.pairs, bw.out.b, d, state, rows, kEpiResidual, state, d);
+            ln_gelu512(state, m, bw.n2w, bw.n2b, bw.l1, 2 * d, hid);
+            if (few)
+                linear(hid, 2 * d, m, 2 * d, bw.l2.w, bw.l2.b, d, state, d, kEpiResidual, state, d);
+            else
+                linear_pairs(hid, 2 * d, m, 2 * d, bw.l2.pairs, bw.l2.b, d, state, rows, kEpiResidual, state, d);
             return;
         }
         if (use_fused) {
@@ -702,7 +706,7 @@ struct Stages {
     // K and V of an ICL block's n normalized rows, in two planes of head-major rows.
     void icl_kv_rows(const BlockW &bw, const float *norm, int n, float *out, long long plane) const {
         const OutMap map = OutMap::head_major(64, kHeads, n, plane);
-        if (n > kPairRows) {
+        if (n > kFewRows) {
             PairW kv = bw.in_pairs;
             kv.pack += (size_t)512 * 512, kv.row_inv += 512;  // past the query rows
             linear_pairs(norm, 512, n, 512, kv, bw.in_b + 512, 1024, out, map);
@@ -1410,15 +1414,7 @@ void issue_pass(irx_predictor *P, int slot, const PassBuffers &pb, const float *
         }
     }
     // Decoder (cached_icl_decoder, cpu.rs:2543-2580) into logits [B, Q, width].
-    if ((long long)B * R > kPairRows) {
-        st.linear_pairs(rows, 512, (long long)B * R, 512, W.dec0.pairs, W.dec0.b, 1024, ib.hid,
-                        OutMap::row_major(1024, 1024), kEpiGelu, nullptr, 0, W.ln_w, W.ln_b);
-    } else {
-        LnLinear f{};
-        f.x = rows, f.ldx = 512, f.lnw = W.ln_w, f.lnb = W.ln_b, f.w = W.dec0.w, f.b = W.dec0.b, f.out = ib.hid;
-        f.ldo = 1024, f.m = B * R, f.n = 1024;
-        ln_linear512(f, kLnGelu, s);
-    }
+    st.ln_gelu512(rows, (long long)B * R, W.ln_w, W.ln_b, W.dec0, 1024, ib.hid);
     OutMap lmap{width, 1, 0, 0, R, (long long)Q * width, width};
     st.linear_map(ib.hid, 1024, (long long)B * R, 1024, W.dec2.w, W.dec2.b, width, logits, lmap);
 }
@@ -2375,10 +2371,12 @@ int irx_test_ln_linear(irx_device *device, int epilogue, const float *x, size_t 
                               !tiled);
             IRX_HIP(hipDeviceSynchronize());
         } else {
-            LnLinear f{};
-            f.x = dx.f(), f.ldx = 512, f.lnw = dlw.f(), f.lnb = dlb.f(), f.w = dw.f(), f.b = db.f(), f.out = dout.f();
-            f.ldo = (long long)n, f.m = (int)m, f.n = (int)n;
-            ln_linear512(f, kLnGelu, nullptr);
+            DevBuf pack(pair_pack_floats((int)n, 512) * 4);
+            const Lin l{dw.f(), db.f(), pair_pack(dw.f(), (int)n, 512, lnw, lnb, pack.f(), nullptr)};
+            irx_weights none;
+            Stages{none, nullptr, device->compute_units}.ln_gelu512(dx.f(), (long long)m, dlw.f(), dlb.f(), l, (int)n,
+                                                                    dout.f());
+            IRX_HIP(hipDeviceSynchronize());
         }
         IRX_HIP(hipDeviceSynchronize());
         IRX_HIP(hipMemcpy(out, dout.p, m * n * 4, hipMemcpyDeviceToHost));

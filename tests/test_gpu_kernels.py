@@ -693,7 +693,8 @@ def ln64(x, w, b):
 @pytest.mark.parametrize("m,n", [(1, 512), (2, 1024), (3, 1024), (8, 512), (9, 1024), (16, 512), (17, 1024),
                                  (512, 1024), (1000, 512)])
 def test_ln_linear_gelu_matches_float64(device, m, n):
-    """LN2 + FFN up (and the decoder's LN + first layer) in one kernel."""
+    """LN2 + FFN up (and the decoder's LN + first layer) in one kernel (FP16 pairs
+    from nine rows)."""
     x = fast_values(m * 512, 1, 3.0) + 0.25
     lnw, lnb = fast_values(512, 2, 0.2) + 1.0, fast_values(512, 3, 0.1)
     w, b = fast_values(n * 512, 4, 0.05), fast_values(n, 5, 0.1)
@@ -770,7 +771,7 @@ def test_pair_linear_weights_of_any_size(device, m, k, norm, octaves):
                                                   (3, 1, 2049), (3, 3, 1001), (4, 1, 33), (4, 3, 17), (4, 2, 250)])
 def test_ln_linear_qass_matches_float64(device, form, estimators, rows):
     """LN1 + Q projection + QASSMax (query MLP and gate per head), head-major:
-    forms 2 and 4 the prediction's fused kernels (FP16 pairs from 33 rows), form
+    forms 2 and 4 the prediction's fused kernels (FP16 pairs from nine rows), form
     3 the build's (LayerNorm, projection on FP16 pairs, then the MLP and gate
     over the projected rows, whose waves each take a contiguous share of 16-row
     tasks; 3 x 1001 x 8 rows end mid-task)."""
@@ -793,10 +794,10 @@ def test_ln_linear_qass_matches_float64(device, form, estimators, rows):
     np.testing.assert_allclose(out.reshape(estimators, 8, rows, 64), want, rtol=1e-4, atol=2e-5)
 
 
-@pytest.mark.parametrize("rows", [1, 64, 65, 1000, 4097])
+@pytest.mark.parametrize("rows", [1, 8, 9, 64, 65, 1000, 4097])
 @pytest.mark.parametrize("estimators,estimator", [(1, 0), (3, 1)])
 def test_icl_kv_matches_float64(device, rows, estimators, estimator):
-    """The build's K and V projection (FP16 pairs above 64 rows): the weights'
+    """The build's K and V projection (FP16 pairs from nine rows): the weights'
     rows past the query's, into two planes of head-major rows of one estimator;
     the other estimators' parts stay as they were."""
     x = fast_values(rows * 512, 1, 2.0)
