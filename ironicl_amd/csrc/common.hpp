@@ -237,6 +237,7 @@ struct PairLinear {
     OutMap out;
     int m, n, k;
     int epilogue;
+    int compute_units;
 };
 void pair_linear(const PairLinear &a, hipStream_t stream);
 

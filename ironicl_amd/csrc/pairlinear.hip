@@ -258,9 +258,18 @@ void pair_linear(const PairLinear &a, hipStream_t stream) {
     // 16; at depth 1,024 the rows' pairs take the LDS of 16), and 256 columns
     // rather than 64 once that leaves two workgroups a CU: the prologue, several
     // times a 64-column product's time, is then paid by a fourth of them.
-    const int rg = a.k == 512 && (long long)ceil_div(a.m, 32) * (a.n / 64) >= 256 ? 2 : 1;
+    // Repeated launches alone, us, of 512 -> 1,024 with LayerNorm: 16 / 32 rows at
+    // 512 rows (256 workgroups) 9.2 / 11.0, at 1,000 13.5 / 13.7, at 8,192 62.8 /
+    // 49.9; 64 / 256 columns at 1,000 rows (128 workgroups of 256) 13.7 / 18.6, at
+    // 2,048 (256) 23.9 / 20.2, at 4,096 (512) 44.2 / 26.8. Lines one doubling
+    // higher for the rows and lower for the columns look better by these, but in
+    // place, beside another stream or on weights not yet in L2, they lose: 1,024 rows
+    // against 10,000 x 100 at auto 2,228 us here and 2,334 so, a 2,048-row build 3.52
+    // and 3.62 ms (3,000 rows 4.63 and 4.56).
+    const long long cus = std::max(1, a.compute_units);
+    const int rg = a.k == 512 && (long long)ceil_div(a.m, 32) * (a.n / 64) >= cus ? 2 : 1;
     const long long groups = ceil_div(a.m, 16 * rg);
-    const bool wide = a.n % 256 == 0 && groups * (a.n / 256) >= 512;
+    const bool wide = (rg == 2 || a.k == 1024) && a.n % 256 == 0 && groups * (a.n / 256) >= 2 * cus;
     const int cgs = a.n / (wide ? 256 : 64);
     const long long count = groups * cgs, per_xcd = (count + 7) / 8;
     if (per_xcd * 8 > 0x7fffffffLL) fail(3, "pair_linear: too many rows");
@@ -285,11 +294,11 @@ void pair_linear(const PairLinear &a, hipStream_t stream) {
     else if (ln && rg == 2)
         width.template operator()<512, 2, true>();
     else if (ln)
-        width.template operator()<512, 1, true>();
+        go.template operator()<512, 1, 1, true>();
     else if (rg == 2)
         width.template operator()<512, 2, false>();
     else
-        width.template operator()<512, 1, false>();
+        go.template operator()<512, 1, 1, false>();
 }
 
 }  // namespace irx

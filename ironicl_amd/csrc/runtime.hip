@@ -474,7 +474,7 @@ struct Stages {
                       const float *lnw = nullptr, const float *lnb = nullptr) const {
         PairLinear g{};
         g.x = a, g.ldx = lda, g.lnw = lnw, g.lnb = lnb, g.w = wt, g.bias = b, g.residual = res, g.ldr = ldr, g.c = c;
-        g.out = map, g.m = (int)m, g.n = n, g.k = k, g.epilogue = epi;
+        g.out = map, g.m = (int)m, g.n = n, g.k = k, g.epilogue = epi, g.compute_units = cus;
         pair_linear(g, s);
     }
 
@@ -2428,6 +2428,7 @@ int irx_test_pair_linear(irx_device *device, int epilogue, const float *x, size_
         g.w = pair_pack(dw.f(), (int)n, (int)k, lnw, lnb, pack.f(), nullptr);
         g.bias = db.f(), g.residual = dout.f(), g.ldr = (long long)n, g.c = dout.f();
         g.out = OutMap::row_major((int)n, (long long)n), g.m = (int)m, g.n = (int)n, g.k = (int)k, g.epilogue = epilogue;
+        g.compute_units = device->compute_units;
         pair_linear(g, nullptr);
         IRX_HIP(hipDeviceSynchronize());
         IRX_HIP(hipMemcpy(out, dout.p, m * n * 4, hipMemcpyDeviceToHost));

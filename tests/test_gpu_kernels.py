@@ -706,7 +706,7 @@ def test_ln_linear_gelu_matches_float64(device, m, n):
     np.testing.assert_allclose(out.reshape(m, n), want, rtol=1e-4, atol=2e-5)
 
 
-@pytest.mark.parametrize("m", [1, 65, 512, 1000, 9001])
+@pytest.mark.parametrize("m", [1, 65, 512, 1000, 2045, 4090, 9001])
 @pytest.mark.parametrize("epilogue,k,n,norm", [(0, 512, 64, False), (0, 512, 1024, False), (1, 512, 1024, True),
                                                (2, 512, 512, False), (2, 1024, 512, False), (1, 1024, 64, False)])
 def test_pair_linear_matches_float64(device, m, epilogue, k, n, norm):
