@@ -140,8 +140,8 @@ constexpr int kFlushTiles = 64;
 // Scales, all powers of two. Queries: per row, in registers. Keys and values:
 // per wave's share of a tile (8 keys x 64 dims), kept while the share's
 // largest scaled magnitude stays below 2^15 (keys' at 2^11 or more) and else
-// set to bring it into [2^13, 2^14): a pair holds an operand to 2^-24 of itself, or to 2^-25
-// absolute (scaled) below that. The key scale joins the softmax's multiply (four keys of
+// set to bring it into [2^13, 2^14): a pair holds an operand to 2^-23 of itself, or to 2^-25
+// absolute (scaled) below 1/4. The key scale joins the softmax's multiply (four keys of
 // it to a register group); the value scale joins the exponent, so that the
 // probability carries its inverse, and is taken out of the row sum. The
 // reference the exponent is taken against is raised, to 8 (base 2) below the
@@ -157,7 +157,7 @@ constexpr int kFlushTiles = 64;
 //   values that spread too far: a share's smallest key times its smallest dim
 //     (zeros aside, each by its largest value) over the largest, the size of a
 //     value that is small both ways, must be 1/2 or more scaled, so that every
-//     value is held to 2^-24 of the size its key and dim have. That each dim's
+//     value is held to 2^-23 of the size its key and dim have. That each dim's
 //     largest value reaches 2^7, and that some dim's smallest does, shows it in
 //     most tiles (2^7 2^7 / 2^15) and keeps the scale.
 struct IclPairTile {
@@ -502,15 +502,17 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
             k_high = limit(kPairHigh - ek), k_low = limit(kPairLow - ek);
             v_high = limit(kPairHigh - ev), v_even = limit(kPairEven - ev);
             if (vb && vb < 0x7f800000u && uneven()) {
-                // The smallest nonzero key and dim, each by its largest value.
-                float key = -INFINITY;
+                // The least that every nonzero key must reach somewhere, by
+                // the smallest nonzero dim's largest value. (Of a single key
+                // that is its smallest value, which says less of the dim.)
+                int nonzero = 0;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float m = wave_max_all(fabsf(vr[i]));
-                    key = fmaxf(key, m > 0.f ? -m : -INFINITY);
-                }
-                const float dim = wave_max_all(vm > 0.f ? -vm : -INFINITY), up = pow2(ev);
-                if (dim * up * (key * up) < 0.5f * (v_largest * up)) special = true;
+                for (int i = 0; i < 8; ++i) nonzero += __ballot(vr[i] != 0.f) != 0;
+                const float dim = -wave_max_all(vm > 0.f ? -vm : -INFINITY) * pow2(ev);
+                const float least = (nonzero > 1 ? 0x1p-1f : 0x1p-9f) * v_largest * __builtin_amdgcn_rcpf(dim);
+#pragma unroll
+                for (int i = 0; i < 8; ++i)
+                    if (__ballot(fabsf(vr[i]) >= least) == 0 && __ballot(vr[i] != 0.f) != 0) special = true;
             }
         }
     };
@@ -717,7 +719,7 @@ __global__ __launch_bounds__(kPairWaves * 64, 2) void icl_attention_kernel(IclAt
             }
             ++since;
         }
-        update_scales();
+        if (t + 1 < tiles) update_scales();
         convert_k(t + 1 + khalf), convert_v(t + 1, vb_next);
         load_k(tile_at(t + 2 + khalf)), load_v(tile_at(t + 2));
         softmax(t);

@@ -99,13 +99,15 @@ def attention64(q, k, v, scale):
 
 
 @pytest.mark.parametrize("query_rows,rows", [(33, 1), (65, 31), (64, 129), (257, 700), (300, 9001)])
-@pytest.mark.parametrize("kind", ["spread", "tiny", "large", "zeros", "outlier"])
+@pytest.mark.parametrize("kind", ["spread", "small", "tiny", "large", "zeros", "outlier"])
 def test_icl_attention_operand_ranges(device, query_rows, rows, kind):
     """The FP16-pair products scale their operands by the magnitudes they meet:
     per query row, and per eight keys. Keys and values spread over 2^-12 ..
     2^12 from row to row (with queries kept small, so that scores stay of
-    order one) and dims over 2^-6 .. 2^6; all of them tiny or large; rows of
-    zeros; one key of 1e4 times the others' size that no query attends to. An
+    order one) and dims over 2^-6 .. 2^6; all of them small (scales near their
+    ends), tiny (values below what the scales reach: FP32 products) or large;
+    rows of zeros; one key of 1e4 times the others' size that no query attends
+    to. "spread" and "outlier" are left to FP32 products too. An
     error is at most a few FP32 roundings of the row's sum of |p v| (2^-18 of
     it: scores of at most 16 carry 16 x 2^-23, exponentiated, and the sums'
     roundings)."""
@@ -117,6 +119,10 @@ def test_icl_attention_operand_ranges(device, query_rows, rows, kind):
         v *= np.exp2(rng.integers(-6, 7, (1, 1, 64))).astype(np.float32)
         size = np.exp2(rng.integers(-12, 1, (pairs, rows, 1))).astype(np.float32)
         k *= size
+    elif kind == "small":
+        k *= np.float32(1e-30)
+        q *= np.float32(1e30)
+        v *= np.float32(1e-13)
     elif kind == "tiny":
         k *= np.float32(1e-20)
         q *= np.float32(1e20)
@@ -216,7 +222,7 @@ def test_icl_attention_value_spread(device, query_rows, rows, kind, octaves):
     which scaled FP16 pairs no longer hold them: every 8th key 2^octaves
     larger, at a score that gives it no weight; every 5th dim 2^octaves
     smaller; both. Scores are below 1, so a term p v carries a few roundings
-    (the pair of p 2^-24, that of v 2^-24 of v or of the size its key and dim
+    (the pair of p 2^-23, that of v 2^-23 of v or of the size its key and dim
     have, the exponent's sum and exp2 2^-22, the accumulated sums' 2^-22 over
     700 keys): 2^-20 of the sum of p and those sizes."""
     pairs = 8
