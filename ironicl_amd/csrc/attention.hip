@@ -116,12 +116,12 @@ constexpr int kFlushTiles = 64;
 // use throughout. The halves' results are merged through LDS at the end (and,
 // FLUSH, every kFlushTiles tiles).
 //
-// 512 queries x 50,000 keys x 8 pairs takes 164 us: 956 TFLOP/s of FP16
+// 512 queries x 50,000 keys x 8 pairs takes 167 us: 943 TFLOP/s of FP16
 // products (a large FP16 matrix product reaches 1,100 here), MFMAs busy 47% of
 // the cycles at a clock of 2.0 GHz. Orders of the same work that take fewer
 // cycles (fragments read across the barrier, wave priorities, the conversions
 // stage by stage) take the same time. The FP32 MFMA kernel before it took 388
-// us, 135 of 157 TFLOP/s; 10,007 queries x 10,007 keys went from 1,553 to 595.
+// us, 135 of 157 TFLOP/s; 10,007 queries x 10,007 keys went from 1,553 to 600.
 //   S^T (key x query), A = K[key 32 (w / 4) + lane % 32][dims 16 m +
 //     8 (lane / 32) .. +7], B = the lane's query, same dims; register r is
 //     key 8 (r / 4) + 4 (lane / 32) + r % 4 of the half;
