@@ -153,7 +153,8 @@ constexpr int kFlushTiles = 64;
 //   infinite keys or values, and values all below 2^-47;
 //   keys so large that scores could pass 2^17 where their scale is set (as
 //     8 |q| |k| of the largest magnitudes). Below it the absolute parts of the
-//     64 products of q and k add up to at most 2^-21 of score;
+//     64 products of q and k add up to less than 2^-18 of score, were every one
+//     at its worst (random ones to 2^-23);
 //   values that spread too far: a share's smallest key times its smallest dim
 //     (zeros aside, each by its largest value) over the largest, the size of a
 //     value that is small both ways, must be 1/2 or more scaled, so that every
